@@ -74,6 +74,11 @@ struct og_jpend {
     bool  live;
 };
 
+// 64-bit integer add at a uniform base plus a 32-bit byte offset
+__device__ __forceinline__ void og_atomic_add_at(OG_GLOBAL(char) *base, unsigned off, unsigned long long v) {
+    __hip_atomic_fetch_add((OG_GLOBAL(unsigned long long) *)(base + off), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Fixed-point add of a lane's gradient (x, y, z) at grid slot a (the
 // j-gradient enters with a minus sign).  Zero contributions are skipped.
 __device__ __forceinline__ void og_add_fx3(OG_GLOBAL(long long) *FX, int cap, int a, double sx, double sy,
@@ -89,20 +94,30 @@ __device__ __forceinline__ void og_add_fx3(OG_GLOBAL(long long) *FX, int cap, in
 // next lane holds the pair's other slot (rows of one cell2 queue in atom
 // order) the lower lane adds both fields with one atomic.  The memory-side
 // atomics cost per element, so about 1.6 per row instead of three.  Called
-// by the whole wave.
-__device__ __forceinline__ void og_flush_j(OG_GLOBAL(long long) *FX, int cap, og_jpend &p) {
-    const int  lane = threadIdx.x & 63;
-    const int  f    = og_fx_slot(p.a);
-    const int  fz   = (int)__builtin_rintf(-p.z * 524288.0f);  // |z| < 4096: exact scaling, half-even rounding
-    const int  fn = __shfl_down(f, 1, 64), zn = __shfl_down(fz, 1, 64), ln = __shfl_down((int)p.live, 1, 64);
-    const int  fp = __shfl_up(f, 1, 64), lp = __shfl_up((int)p.live, 1, 64);
-    const bool lower = !(f & 1) && lane < 63 && ln && fn == (f ^ 1);  // this lane adds the pair's both fields
-    const bool upper = (f & 1) && lane > 0 && lp && fp == (f ^ 1);    // the lane below adds this field
+// by the whole wave.  The neighbours come by DPP wave shifts, the words are
+// built in 32-bit halves and addressed as a uniform base plus a 32-bit byte
+// offset: 40 VALU per pass instead of 75 with shuffles through LDS and 64-bit
+// index arithmetic.
+__device__ __forceinline__ void og_flush_j(OG_GLOBAL(char) *FXJ, OG_GLOBAL(char) *FXZ, og_jpend &p) {
+    // slot index with cell bits 0 and 1 swapped (og_fx_slot); idle lanes pair with nobody
+    const unsigned t   = (unsigned)(p.a ^ (p.a >> 1)) & 8u;
+    const int      f   = p.live ? (int)((unsigned)p.a ^ (t | (t << 1))) : -2;
+    const int      fx  = (int)__builtin_rintf(-p.x * 524288.0f);  // |x| < 4096: exact scaling, half-even rounding
+    const int      fy  = (int)__builtin_rintf(-p.y * 524288.0f);
+    const int      fz  = (int)__builtin_rintf(-p.z * 524288.0f);
+    const int      fn  = __builtin_amdgcn_update_dpp(-2, f, 0x130, 0xf, 0xf, false);  // the next lane's slot
+    const int      fp  = __builtin_amdgcn_update_dpp(-2, f, 0x138, 0xf, 0xf, false);  // the previous lane's slot
+    const int      zn  = __builtin_amdgcn_update_dpp(0, fz, 0x130, 0xf, 0xf, false);  // the next lane's z
+    const bool     odd = f & 1;
+    const bool     lower = !odd && (fn ^ f) == 1;  // this lane adds the pair's both fields
+    const bool     upper = odd && (fp ^ f) == 1;   // the lane below adds this field
+    // 64-bit sums of sign-extended fields: x + y * 2^32 and z_even + z_odd * 2^32
+    const unsigned xlo = (unsigned)fx, xhi = (unsigned)(fy + (fx >> 31));
+    const unsigned zlo = odd ? 0u : (unsigned)fz;
+    const unsigned zhi = odd ? (unsigned)fz : (unsigned)((fz >> 31) + (lower ? zn : 0));
     if (p.live) {
-        const unsigned long long xy = og_fxj_pack_f(-p.x, -p.y);
-        if (xy != 0) og_atomic_add_fx_g(FX + 3 * cap + f, (long long)xy);
-        const long long vz = lower ? (long long)fz + ((long long)zn << 32) : (long long)fz << (32 * (f & 1));
-        if (!upper && vz != 0) og_atomic_add_fx_g(FX + OG_FX_ZJ(cap) + (f >> 1), vz);
+        if (xlo | xhi) og_atomic_add_at(FXJ, (unsigned)f << 3, ((unsigned long long)xhi << 32) | xlo);
+        if (!upper && (zlo | zhi)) og_atomic_add_at(FXZ, ((unsigned)f << 2) & ~7u, ((unsigned long long)zhi << 32) | zlo);
     }
     p.live = false;
 }
@@ -245,7 +260,7 @@ template <int FORM, bool ENERGY, bool LJ_LDS>
 __device__ __forceinline__ void og_pass(const og_dev_sys &s, const og_cell1 &c, const og_f4 *qp, const int2 *qa,
                                         const int q0, const int cnt, const typename og_ljt<FORM>::type *ljl,
                                         const OG_GLOBAL(typename og_ljt<FORM>::type) *__restrict__ LJP,
-                                        OG_GLOBAL(long long) *FX,
+                                        OG_GLOBAL(char) *FXJ, OG_GLOBAL(char) *FXZ,
                                         float (&fi)[3 * OG_NAC], int &npair, float &vmax, float &vsum, double &ev,
                                         double &ee, double &vir, og_jpend &pend) {
     const int  lane = threadIdx.x & 63;
@@ -261,7 +276,7 @@ __device__ __forceinline__ void og_pass(const og_dev_sys &s, const og_cell1 &c, 
     // out, so nothing in the pass waits on the vector-memory counter
     // (s_waitcnt vmcnt(0); expcnt and lgkmcnt left at their maxima)
     __builtin_amdgcn_s_waitcnt(0x0F70);
-    og_flush_j(FX, s.cap_atom_array, pend);
+    og_flush_j(FXJ, FXZ, pend);
     og_rows<FORM, ENERGY, LJ_LDS>(s, c, pj, tj, m8, ax.x, live, ljl, LJP, fi, npair, vmax, vsum, ev, ee, vir, pend);
 }
 
@@ -295,6 +310,9 @@ __device__ __forceinline__ void og_pair_cell(const og_dev_sys &s, const int c1, 
     OG_GLOBAL(long long) *__restrict__ FX       = (OG_GLOBAL(long long) *)s.fx;
     const int   cap = s.cap_atom_array;
     const int   nt  = s.n_types;
+    // packed j-side words of the gradient: (x, y) per slot, z per slot pair
+    OG_GLOBAL(char) *FXJ = (OG_GLOBAL(char) *)(FX + 3 * (size_t)cap);
+    OG_GLOBAL(char) *FXZ = (OG_GLOBAL(char) *)(FX + OG_FX_ZJ(cap));
     // keep-test radius: the cutoff plus 10 ppm, so float rounding of the box
     // distance can never drop a row that holds an in-range pair
     const float rcb2 = s.cutoff2 * 1.00001f;
@@ -382,7 +400,7 @@ __device__ __forceinline__ void og_pair_cell(const og_dev_sys &s, const int c1, 
         }
         qn += __builtin_popcountll(ub);
         if (qn - qd >= 64) {
-            og_pass<FORM, ENERGY, LJ_LDS>(s, c, qp, qa, qd, 64, ljl, LJP, FX, fi, npair, vmax, vsum, ev, ee, vir, pend);
+            og_pass<FORM, ENERGY, LJ_LDS>(s, c, qp, qa, qd, 64, ljl, LJP, FXJ, FXZ, fi, npair, vmax, vsum, ev, ee, vir, pend);
             qd += 64;
         }
         cp    = cpn;
@@ -390,8 +408,8 @@ __device__ __forceinline__ void og_pair_cell(const og_dev_sys &s, const int c1, 
         valid = validn;
     }
     if (qn > qd)
-        og_pass<FORM, ENERGY, LJ_LDS>(s, c, qp, qa, qd, qn - qd, ljl, LJP, FX, fi, npair, vmax, vsum, ev, ee, vir, pend);
-    og_flush_j(FX, cap, pend);
+        og_pass<FORM, ENERGY, LJ_LDS>(s, c, qp, qa, qd, qn - qd, ljl, LJP, FXJ, FXZ, fi, npair, vmax, vsum, ev, ee, vir, pend);
+    og_flush_j(FXJ, FXZ, pend);
 
     // i-gradients: reduce-scatter the 24 partial sums over the wave.  After
     // the xor-32/16/8 steps lane L holds atom L>>3's (x, y, z) summed over 8
