@@ -1283,7 +1283,7 @@ og_status og_system_footprint(const og_system_desc *d, const og_params *p, uint6
     b += 2 * (n + 1) * 4 + std::max(2 * ex, 1.0) * 16 + std::max(2 * nb, 1.0) * 16;      // per-atom pair lists
     b += (ng + 1) * 4 + ng_atoms * 4 + (ng + 1) * 4 + 3 * (ng + 1) * 8;
     b += cols * (4 * 6 + 8) + 2 * (cols + 2) * g.n_uni_z * 4;
-    b += cap * (4 + 4 + 24 + 16 + 4 + 4 + 32);                            // tmp_ids, atomids, gcrd, gxyzq, gtype, gcomp, fx
+    b += cap * (4 + 4 + 24 + 16 + 4 + 4 + 36);                            // tmp_ids, atomids, gcrd, gxyzq, gtype, gcomp, fx
     b += cells * (6 * 4 + 4.0 * OG_ENUM_STAGE + 8) + (cells / 1024 + 1) * 8;
     b += pairs * 12;
     b += 8.0 * OG_EACC_SLOTS * OG_EACC_STRIDE + ke_parts * 8 + OG_E_NTERMS * 8 + log_rows * OG_E_NTERMS * 8;

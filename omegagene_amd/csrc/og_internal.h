@@ -23,17 +23,14 @@
 #define OG_FXJ_SCALE 524288.0
 #define OG_FXJ_INV (1.0 / 524288.0)
 #define OG_FXJ_ROW_LIMIT 2048.0f
-// Words of the fixed-point gradient per system (cap = cap_atom_array, a
-// multiple of 32): x, y, z of the i side and of excluded pairs at 2^32 units
-// (cap each); the j-side (x, y) words (cap); the j-side z of each slot pair
-// (2k, 2k + 1) as two 32-bit fields at 2^19 units in one word (cap / 2), so
-// neighbouring rows of one cell2 add both with one atomic; and the value of
-// that word each slot last took (cap).  The pair word is never cleared: a slot
-// takes the change since its last read, so the two slots of a pair may read it
-// in any order (a slot reads it once per evaluation).
-#define OG_FX_ZJ(cap) (4 * (size_t)(cap))
-#define OG_FX_ZLAST(cap) (OG_FX_ZJ(cap) + (size_t)(cap) / 2)
-#define OG_FX_WORDS(cap) (OG_FX_ZLAST(cap) + (size_t)(cap))
+// Words of the fixed-point gradient per system, each component padded to whole
+// groups of eight cells (og_fx_slot): x, y, z of the i side and of excluded
+// pairs at 2^32 units (one word per slot each); the j-side (x, y) words; the
+// j-side z at 2^19 units, 32 bits per slot.
+#define OG_FX_CAP(cap) (((size_t)(cap) + 63) / 64 * 64)
+#define OG_FX_XY(cap) (3 * OG_FX_CAP(cap))
+#define OG_FX_Z(cap) (4 * OG_FX_CAP(cap))
+#define OG_FX_WORDS(cap) (OG_FX_Z(cap) + OG_FX_CAP(cap) / 2)
 #define OG_NO_STEP_END 0x7fffffffffffffffLL  // og_dev_counters::step_end of a system with no segment limit
 #define OG_TH_SCALING 1  // og_params::thermostat value of the scaling thermostat (OG_THERMOSTAT_SCALING)
 // og_dev_sys::mc_mode values (the public OG_EXT_VMCMD / OG_EXT_VAUS) and coefficients per state (OG_MC_MAX_ORDER + 1)
@@ -226,7 +223,7 @@ struct og_dev_sys {
     uint64_t *cp_mask;      // [cap_cell_pairs] bit a2*8+a1 set = skip
     // ---- forces / energies ----
     long long *fx;          // [OG_FX_WORDS(cap_atom_array)] fixed-point gradient, slot g at og_fx_slot(g)
-                            // (2^32 units) | packed j-side (x, y) (og_fxj_pack)
+                            // (2^32 units) | packed j-side (x, y) | j-side z
     long long *e_acc;       // [OG_EACC_SLOTS][OG_EACC_STRIDE] energy accumulators, 2^32 fixed point (the pair
                             // count as an integer): vdw, ele, virial, pairs, excess, bond; a cell / block adds to
                             // slot (index % OG_EACC_SLOTS), so no cache line takes every add; zeroed by the reader
@@ -335,14 +332,14 @@ __device__ __forceinline__ float og_dpp_sum8(float x) {
 
 __device__ __forceinline__ long long og_to_fixed(double v) { return __double2ll_rn(v * OG_FX_SCALE); }
 
-// Index of grid slot g in each component of the fixed-point gradient: cell
-// index bits 0 and 1 swapped, so cells c and c + 2 -- the same-parity cells
-// one cell1 takes from a neighbour column -- share a 128-byte line and one
-// memory-side atomic request covers both.  A bijection on every group of
-// four cells (cap_atom_array is a multiple of 32 slots).
+// Index of grid slot g in each component of the fixed-point gradient: within
+// eight cells those of one parity come together (cell bits b2 b1 b0 -> b0 b2
+// b1).  A cell1 takes the cells of one parity from a neighbour column, so the
+// (x, y) words of its cells c and c + 2 share a 128-byte line, and the z words
+// of c, c + 2, c + 4 and c + 6, and one memory-side atomic request covers them.
+// A bijection on every group of eight cells.
 __device__ __forceinline__ int og_fx_slot(int g) {
-    const int c = g >> 3;
-    return ((((c & ~3) | ((c & 1) << 1) | ((c >> 1) & 1))) << 3) | (g & 7);
+    return (g & ~0x38) | ((g & 8) << 2) | ((g >> 1) & 0x18);
 }
 
 // Round-to-nearest fixed point without a conversion sequence: adding
@@ -355,20 +352,6 @@ __device__ __forceinline__ long long og_fx_fast(double v) {
     const double t = v * OG_FX_SCALE + OG_FX_MAGIC;
     return __double_as_longlong(t) - OG_FX_MAGIC_BITS;
 }
-// (x, y) rounded to 2^-19 and packed as x + y * 2^32 (|x|, |y| < 4096)
-__device__ __forceinline__ unsigned long long og_fxj_pack(double x, double y) {
-    const long long ix = __double_as_longlong(x * OG_FXJ_SCALE + OG_FX_MAGIC) - OG_FX_MAGIC_BITS;
-    const long long iy = __double_as_longlong(y * OG_FXJ_SCALE + OG_FX_MAGIC) - OG_FX_MAGIC_BITS;
-    return (unsigned long long)ix + ((unsigned long long)iy << 32);
-}
-// The same word from float inputs (|x|, |y| below 4096): x * 2^19 is exact in
-// float and rintf rounds half to even like the FP64 form, so the result is
-// bit-identical to og_fxj_pack((double)x, (double)y), in FP32 instructions.
-__device__ __forceinline__ unsigned long long og_fxj_pack_f(float x, float y) {
-    const long long ix = (long long)(int)__builtin_rintf(x * 524288.0f);
-    const long long iy = (long long)(int)__builtin_rintf(y * 524288.0f);
-    return (unsigned long long)ix + ((unsigned long long)iy << 32);
-}
 // the two fields of a packed sum (each within +-2^31 units)
 __device__ __forceinline__ void og_fxj_unpack(long long w, double &x, double &y) {
     const long long ix = (long long)(int)(unsigned)(unsigned long long)w;
@@ -378,19 +361,19 @@ __device__ __forceinline__ void og_fxj_unpack(long long w, double &x, double &y)
 }
 // the pair gradient of grid slot g (index f = og_fx_slot(g)) in kcal/mol/A
 __device__ __forceinline__ void og_fx_read(const long long *fx, int cap, int f, double *w) {
-    double jx, jy, zlo, zhi;
-    og_fxj_unpack(fx[3 * cap + f], jx, jy);
-    // the slot pair's z word changed by both slots' sums since this slot's last read
-    og_fxj_unpack(fx[OG_FX_ZJ(cap) + (f >> 1)] - fx[OG_FX_ZLAST(cap) + f], zlo, zhi);
+    const size_t stride = OG_FX_CAP(cap);
+    double       jx, jy;
+    og_fxj_unpack(fx[OG_FX_XY(cap) + f], jx, jy);
+    const int jz = ((const int *)(fx + OG_FX_Z(cap)))[f];
     w[0] = (double)fx[f] * OG_FX_INV + jx;
-    w[1] = (double)fx[cap + f] * OG_FX_INV + jy;
-    w[2] = (double)fx[2 * cap + f] * OG_FX_INV + ((f & 1) ? zhi : zlo);
+    w[1] = (double)fx[stride + f] * OG_FX_INV + jy;
+    w[2] = (double)fx[2 * stride + f] * OG_FX_INV + (double)jz * OG_FXJ_INV;
 }
-// after og_fx_read: clear the slot's own words and note the pair word it has taken
+// after og_fx_read: clear the slot's words
 __device__ __forceinline__ void og_fx_consume(long long *fx, int cap, int f) {
-    fx[OG_FX_ZLAST(cap) + f] = fx[OG_FX_ZJ(cap) + (f >> 1)];
-    fx[3 * cap + f]          = 0;
-    for (int k = 0; k < 3; k++) fx[k * cap + f] = 0;
+    const size_t stride = OG_FX_CAP(cap);
+    for (int k = 0; k < 4; k++) fx[k * stride + f] = 0;
+    ((int *)(fx + OG_FX_Z(cap)))[f] = 0;
 }
 
 #define OG_GLOBAL(T) __attribute__((address_space(1))) T

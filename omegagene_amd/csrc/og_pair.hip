@@ -24,7 +24,7 @@
 
 #define OG_CHARGE_COEFF 332.06378f   // CelesteObject.cpp:36
 #define OG_QCAP 128                  // per-wave row queue (two passes of 64)
-#define OG_LJ_LDS_ENTRIES 512        // LJ table entries (whole leading rows) held in LDS per block
+#define OG_LJ_LDS_ENTRIES(FORM) ((FORM) == 2 ? 256 : 512)  // LJ table entries (whole leading rows, 4 KB) in LDS
 
 typedef float og_f4 __attribute__((ext_vector_type(4)));
 typedef float og_f2 __attribute__((ext_vector_type(2)));
@@ -54,9 +54,22 @@ __device__ __forceinline__ float og_rlane(float v, int k) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k));
 }
 
-// Cell1 data held by the wave: atom coordinates, charge * 332.06378, LJ row
-// offsets (type * n_types, the same in the global table and in the block's
-// LDS copy of its leading rows) and the bounding box.
+// a uniform value kept in a vector register: an FP32 add, multiply or fma
+// with a scalar-register operand issues at half the rate of one without
+// (4.2-4.5 cycles per wave against 2.2 measured on gfx950)
+__device__ __forceinline__ float og_vgpr(float v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+template <int CTRL> __device__ __forceinline__ float og_dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+
+// Cell1 data held by the wave, the same in every lane: atom coordinates and
+// charge * 332.06378 (vector registers, see og_vgpr), LJ row offsets (type *
+// n_types, the same in the global table and in the block's LDS copy of its
+// leading rows; scalar) and the bounding box.
 struct og_cell1 {
     float    x[OG_NAC], y[OG_NAC], z[OG_NAC], q[OG_NAC];
     unsigned row[OG_NAC];
@@ -74,50 +87,37 @@ struct og_jpend {
     bool  live;
 };
 
-// 64-bit integer add at a uniform base plus a 32-bit byte offset
-__device__ __forceinline__ void og_atomic_add_at(OG_GLOBAL(char) *base, unsigned off, unsigned long long v) {
-    __hip_atomic_fetch_add((OG_GLOBAL(unsigned long long) *)(base + off), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // Fixed-point add of a lane's gradient (x, y, z) at grid slot a (the
 // j-gradient enters with a minus sign).  Zero contributions are skipped.
 __device__ __forceinline__ void og_add_fx3(OG_GLOBAL(long long) *FX, int cap, int a, double sx, double sy,
                                            double sz) {
+    const size_t    stride = OG_FX_CAP(cap);
     const long long vx = og_fx_fast(sx), vy = og_fx_fast(sy), vz = og_fx_fast(sz);
     if (vx != 0) og_atomic_add_fx_g(FX + a, vx);
-    if (vy != 0) og_atomic_add_fx_g(FX + cap + a, vy);
-    if (vz != 0) og_atomic_add_fx_g(FX + 2 * cap + a, vz);
+    if (vy != 0) og_atomic_add_fx_g(FX + stride + a, vy);
+    if (vz != 0) og_atomic_add_fx_g(FX + 2 * stride + a, vz);
 }
 
-// j-gradient of a row: (x, y) packed into one 64-bit atomic; z at 2^19 units
-// into the 32-bit field of its slot in the slot pair's word, and when the
-// next lane holds the pair's other slot (rows of one cell2 queue in atom
-// order) the lower lane adds both fields with one atomic.  The memory-side
-// atomics cost per element, so about 1.6 per row instead of three.  Called
-// by the whole wave.  The neighbours come by DPP wave shifts, the words are
-// built in 32-bit halves and addressed as a uniform base plus a 32-bit byte
-// offset: 40 VALU per pass instead of 75 with shuffles through LDS and 64-bit
-// index arithmetic.
+// j-gradient of a row at 2^19 units: (x, y) packed into one 64-bit atomic, z
+// into one 32-bit atomic.  The memory-side atomics cost per request and per
+// byte, so two per row instead of three (z of a slot pair in one 64-bit word,
+// added for two neighbouring rows at once, took 133 us at 99,200 atoms against
+// 127 for this; x, y and z as three 32-bit words 145).  The (x, y) word is
+// built in 32-bit halves and the words are addressed as a uniform base plus a
+// 32-bit byte offset (no 64-bit index arithmetic).  Called by the whole wave.
 __device__ __forceinline__ void og_flush_j(OG_GLOBAL(char) *FXJ, OG_GLOBAL(char) *FXZ, og_jpend &p) {
-    // slot index with cell bits 0 and 1 swapped (og_fx_slot); idle lanes pair with nobody
-    const unsigned t   = (unsigned)(p.a ^ (p.a >> 1)) & 8u;
-    const int      f   = p.live ? (int)((unsigned)p.a ^ (t | (t << 1))) : -2;
-    const int      fx  = (int)__builtin_rintf(-p.x * 524288.0f);  // |x| < 4096: exact scaling, half-even rounding
-    const int      fy  = (int)__builtin_rintf(-p.y * 524288.0f);
-    const int      fz  = (int)__builtin_rintf(-p.z * 524288.0f);
-    const int      fn  = __builtin_amdgcn_update_dpp(-2, f, 0x130, 0xf, 0xf, false);  // the next lane's slot
-    const int      fp  = __builtin_amdgcn_update_dpp(-2, f, 0x138, 0xf, 0xf, false);  // the previous lane's slot
-    const int      zn  = __builtin_amdgcn_update_dpp(0, fz, 0x130, 0xf, 0xf, false);  // the next lane's z
-    const bool     odd = f & 1;
-    const bool     lower = !odd && (fn ^ f) == 1;  // this lane adds the pair's both fields
-    const bool     upper = odd && (fp ^ f) == 1;   // the lane below adds this field
-    // 64-bit sums of sign-extended fields: x + y * 2^32 and z_even + z_odd * 2^32
-    const unsigned xlo = (unsigned)fx, xhi = (unsigned)(fy + (fx >> 31));
-    const unsigned zlo = odd ? 0u : (unsigned)fz;
-    const unsigned zhi = odd ? (unsigned)fz : (unsigned)((fz >> 31) + (lower ? zn : 0));
     if (p.live) {
-        if (xlo | xhi) og_atomic_add_at(FXJ, (unsigned)f << 3, ((unsigned long long)xhi << 32) | xlo);
-        if (!upper && (zlo | zhi)) og_atomic_add_at(FXZ, ((unsigned)f << 2) & ~7u, ((unsigned long long)zhi << 32) | zlo);
+        const unsigned f  = (unsigned)og_fx_slot(p.a);
+        const int      fx = (int)__builtin_rintf(-p.x * 524288.0f);  // |x| < 4096: exact scaling, half-even rounding
+        const int      fy = (int)__builtin_rintf(-p.y * 524288.0f);
+        const int      fz = (int)__builtin_rintf(-p.z * 524288.0f);
+        // the 64-bit sum x + y * 2^32 of sign-extended fields
+        const unsigned xlo = (unsigned)fx, xhi = (unsigned)(fy + (fx >> 31));
+        if (xlo | xhi)
+            __hip_atomic_fetch_add((OG_GLOBAL(unsigned long long) *)(FXJ + (f << 3)), ((unsigned long long)xhi << 32) | xlo,
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (fz)
+            __hip_atomic_fetch_add((OG_GLOBAL(int) *)(FXZ + (f << 2)), fz, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     p.live = false;
 }
@@ -133,7 +133,7 @@ __device__ __forceinline__ void og_rows(const og_dev_sys &s, const og_cell1 &c, 
                                         float (&fi)[3 * OG_NAC], int &npair, float &vmax, float &vsum, double &ev,
                                         double &ee, double &vir, og_jpend &pend) {
     const float rc2 = s.cutoff2;
-    const float zcore = s.zcore, bcoeff = s.bcoeff, fcoeff = s.fcoeff;
+    const float zcore = og_vgpr(s.zcore), bcoeff = og_vgpr(s.bcoeff), fcoeff = og_vgpr(s.fcoeff);
     const float alpha = s.alpha, piewald = s.piewald;
     const float hps_eps = s.hps_eps, kappa = s.dh_kappa;
     const float zmc = s.zm_core, ze0 = s.zm_c[0], ze1 = s.zm_c[1], ze2 = s.zm_c[2], ze3 = s.zm_c[3];
@@ -254,24 +254,27 @@ __device__ __forceinline__ void og_rows(const og_dev_sys &s, const og_cell1 &c, 
     }
 }
 
-// Pass over queue entries [q0, q0 + cnt): reads the rows, adds the previous
-// pass's j-gradient, then evaluates the rows.
+// Pass over queue entries [q0, q0 + cnt) (q0 a multiple of 64): reads the
+// rows, adds the previous pass's j-gradient, then evaluates the rows.
 template <int FORM, bool ENERGY, bool LJ_LDS>
 __device__ __forceinline__ void og_pass(const og_dev_sys &s, const og_cell1 &c, const og_f4 *qp, const int2 *qa,
                                         const int q0, const int cnt, const typename og_ljt<FORM>::type *ljl,
                                         const OG_GLOBAL(typename og_ljt<FORM>::type) *__restrict__ LJP,
-                                        OG_GLOBAL(char) *FXJ, OG_GLOBAL(char) *FXZ,
-                                        float (&fi)[3 * OG_NAC], int &npair, float &vmax, float &vsum, double &ev,
-                                        double &ee, double &vir, og_jpend &pend) {
+                                        OG_GLOBAL(char) *FXJ, OG_GLOBAL(char) *FXZ, float (&fi)[3 * OG_NAC],
+                                        int &npair, float &vmax, float &vsum, double &ev, double &ee, double &vir,
+                                        og_jpend &pend) {
     const int  lane = threadIdx.x & 63;
-    const int  slot = (q0 + lane) & (OG_QCAP - 1);
+    const int  slot = (q0 & (OG_QCAP - 1)) + lane;
     const bool live = lane < cnt;
     og_f4      pj   = qp[slot];
     const int2 ax   = qa[slot];
+    unsigned   m8 = (unsigned)ax.y >> 24, tj = (unsigned)ax.y & 0xffffffu;
     // idle lanes (stale queue slots): finite coordinates, LJ column 0, every pair masked
-    if (!live) pj = og_f4{0.0f, 0.0f, 0.0f, 0.0f};
-    const unsigned m8  = live ? ((unsigned)ax.y >> 24) : 0xffu;
-    const unsigned tj  = live ? ((unsigned)ax.y & 0xffffffu) : 0u;
+    if (cnt < 64) {
+        if (!live) pj = og_f4{0.0f, 0.0f, 0.0f, 0.0f};
+        m8 = live ? m8 : 0xffu;
+        tj = live ? tj : 0u;
+    }
     // every outstanding load of the filter is complete before the atomics go
     // out, so nothing in the pass waits on the vector-memory counter
     // (s_waitcnt vmcnt(0); expcnt and lgkmcnt left at their maxima)
@@ -280,12 +283,37 @@ __device__ __forceinline__ void og_pass(const og_dev_sys &s, const og_cell1 &c, 
     og_rows<FORM, ENERGY, LJ_LDS>(s, c, pj, tj, m8, ax.x, live, ljl, LJP, fi, npair, vmax, vsum, ev, ee, vir, pend);
 }
 
-// a <- the kept half of (a, b) summed with the partner lane's other half
-// (partner = lane ^ off, off = 32 or 16); "upper" lanes keep b.
-__device__ __forceinline__ float og_keep_add(float a, float b, bool upper, int off) {
-    const float keep = upper ? b : a;
-    const float send = upper ? a : b;
-    return keep + __shfl_xor(send, off, 64);
+// Halves of two registers exchanged and added: lanes of the lower half (of
+// 64, or of each 32) get a summed over both halves, lanes of the upper half b.
+__device__ __forceinline__ float og_fold32(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float og_fold16(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// the same over the halves of each 16 lanes (upper: the lane's bit 3)
+__device__ __forceinline__ float og_fold8(float a, float b, bool upper) {
+    const float keep = upper ? b : a, send = upper ? a : b;
+    return keep + og_dpp<0x128>(send);
+}
+// Sum over the wave, in the order of a butterfly over 1, 2, 4, 8, 16, 32.
+template <int CTRL> __device__ __forceinline__ double og_dpp_add64(double v) {
+    return v + __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true),
+                                __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double og_wave_sum64(double v) {
+    v = og_dpp_add64<0xB1>(v);
+    v = og_dpp_add64<0x4E>(v);
+    v = og_dpp_add64<0x141>(v);  // the quads of a half row hold equal sums: mirroring is the exchange over 4
+    v = og_dpp_add64<0x128>(v);
+    double r[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        r[k] = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 16 * k),
+                                __builtin_amdgcn_readlane(__double2loint(v), 16 * k));
+    return (r[0] + r[1]) + (r[2] + r[3]);
 }
 
 // One cell1 (one wave), its cell-pair records [p0, p1) (all of them, or
@@ -300,40 +328,62 @@ __device__ __forceinline__ void og_pair_cell(const og_dev_sys &s, const int c1, 
     const int lane = threadIdx.x & 63;
     const int jl   = lane & 7;
 
-    const OG_GLOBAL(og_f4) *__restrict__ X      = (const OG_GLOBAL(og_f4) *)s.gxyzq;
-    const OG_GLOBAL(int) *__restrict__ TY       = (const OG_GLOBAL(int) *)s.gtype;
     typedef typename og_ljt<FORM>::type ljt;
+    const OG_GLOBAL(char) *__restrict__ X = (const OG_GLOBAL(char) *)s.gxyzq;
+    const OG_GLOBAL(char) *__restrict__ TY = (const OG_GLOBAL(char) *)s.gtype;
     const OG_GLOBAL(ljt) *__restrict__ LJP =
         (const OG_GLOBAL(ljt) *)(FORM == 2 ? (const void *)s.lj_hps : (const void *)s.lj_pair);
-    const OG_GLOBAL(unsigned) *__restrict__ CP  = (const OG_GLOBAL(unsigned) *)s.cp_c2;
-    const OG_GLOBAL(uint64_t) *__restrict__ CM  = (const OG_GLOBAL(uint64_t) *)s.cp_mask;
-    OG_GLOBAL(long long) *__restrict__ FX       = (OG_GLOBAL(long long) *)s.fx;
-    const int   cap = s.cap_atom_array;
-    const int   nt  = s.n_types;
-    // packed j-side words of the gradient: (x, y) per slot, z per slot pair
-    OG_GLOBAL(char) *FXJ = (OG_GLOBAL(char) *)(FX + 3 * (size_t)cap);
-    OG_GLOBAL(char) *FXZ = (OG_GLOBAL(char) *)(FX + OG_FX_ZJ(cap));
+    const OG_GLOBAL(unsigned) *__restrict__ CP = (const OG_GLOBAL(unsigned) *)s.cp_c2;
+    const OG_GLOBAL(uint64_t) *__restrict__ CM = (const OG_GLOBAL(uint64_t) *)s.cp_mask;
+    OG_GLOBAL(long long) *__restrict__ FX      = (OG_GLOBAL(long long) *)s.fx;
+    const int cap = s.cap_atom_array;
+    const int nt  = s.n_types;
+    // j-side words of the gradient: packed (x, y) and z, per slot
+    OG_GLOBAL(char) *FXJ = (OG_GLOBAL(char) *)(FX + OG_FX_XY(cap));
+    OG_GLOBAL(char) *FXZ = (OG_GLOBAL(char) *)(FX + OG_FX_Z(cap));
     // keep-test radius: the cutoff plus 10 ppm, so float rounding of the box
     // distance can never drop a row that holds an in-range pair
     const float rcb2 = s.cutoff2 * 1.00001f;
 
-    // the first group's cell-pair records load with the cell1 atoms
-    // (lane = 8 * (cell pair in the group) + j atom)
-    unsigned cp = 0u;
-    uint64_t mk = ~0ull;
-    bool     valid = false;
+    // Cell-pair records of the group of eight at base (lane = 8 * record + j
+    // atom): cell2 | image << 24 and the j atom's mask byte.  Uniform base plus
+    // a lane offset that is constant but for the last group, where lanes past
+    // the end read its last record.
+    struct rec_t {
+        unsigned cp, m8;
+    };
+    auto load_rec = [&](const int base) {
+        const int b = min(base, p1 - 1), r = p1 - b;
+        unsigned  k = (unsigned)lane >> 3;
+        if (r < OG_NAC) k = min(k, (unsigned)(r - 1));
+        rec_t t;
+        t.cp = *(const OG_GLOBAL(unsigned) *)((const OG_GLOBAL(char) *)(CP + b) + 4u * k);
+        t.m8 = *((const OG_GLOBAL(unsigned char) *)(CM + b) + (8u * k + (unsigned)jl));
+        return t;
+    };
+    struct atom_t {
+        og_f4    p;
+        unsigned ty;
+    };
+    auto load_atom = [&](const unsigned cp) {
+        const unsigned off = ((cp << 7) & 0x7fffffffu) | ((unsigned)jl << 4);  // 16 bytes per slot
+        atom_t t;
+        t.p  = *(const OG_GLOBAL(og_f4) *)(X + off);
+        t.ty = *(const OG_GLOBAL(unsigned) *)(TY + (off >> 2));
+        return t;
+    };
+
+    // the first groups' records load with the cell1 atoms
+    rec_t rec{0u, 0xffu}, rec1{0u, 0xffu};
     if (p0 < p1) {
-        const int t = p0 + (lane >> 3);
-        valid       = t < p1;
-        const int tc = valid ? t : p1 - 1;
-        cp = CP[tc];
-        mk = CM[tc];
+        rec  = load_rec(p0);
+        rec1 = load_rec(p0 + OG_NAC);
     }
 
     og_cell1 c;
     {
-        const og_f4 p  = X[c1 * OG_NAC + jl];
-        const int   ty = TY[c1 * OG_NAC + jl];
+        const og_f4 p  = *(const OG_GLOBAL(og_f4) *)(X + (16u * (unsigned)(c1 * OG_NAC + jl)));
+        const int   ty = *(const OG_GLOBAL(int) *)(TY + (4u * (unsigned)(c1 * OG_NAC + jl)));
         // charge x 332.06378 (x 1/eps_r under Debye-Hueckel)
         const float qc = FORM == 2 ? p.w * OG_CHARGE_COEFF * s.dh_diel_inv : p.w * OG_CHARGE_COEFF;
 #pragma unroll
@@ -342,22 +392,18 @@ __device__ __forceinline__ void og_pair_cell(const og_dev_sys &s, const int c1, 
             c.y[i]   = og_rlane(p.y, i);
             c.z[i]   = og_rlane(p.z, i);
             c.q[i]   = og_rlane(qc, i);
-            const unsigned t = (unsigned)__builtin_amdgcn_readlane(ty, i) * (unsigned)nt;
-            c.row[i] = t;
+            c.row[i] = (unsigned)__builtin_amdgcn_readlane(ty, i) * (unsigned)nt;
         }
-        c.lo[0] = c.hi[0] = c.x[0];
-        c.lo[1] = c.hi[1] = c.y[0];
-        c.lo[2] = c.hi[2] = c.z[0];
+        // bounding box: minima and maxima over the eight lanes
+        float lo[3] = {p.x, p.y, p.z}, hi[3] = {p.x, p.y, p.z};
 #pragma unroll
-        for (int i = 1; i < OG_NAC; i++) {
-            c.lo[0] = fminf(c.lo[0], c.x[i]), c.hi[0] = fmaxf(c.hi[0], c.x[i]);
-            c.lo[1] = fminf(c.lo[1], c.y[i]), c.hi[1] = fmaxf(c.hi[1], c.y[i]);
-            c.lo[2] = fminf(c.lo[2], c.z[i]), c.hi[2] = fmaxf(c.hi[2], c.z[i]);
-        }
-#pragma unroll
-        for (int k = 0; k < 3; k++) {  // wave-uniform: keep in scalar registers
-            c.lo[k] = og_rlane(c.lo[k], 0);
-            c.hi[k] = og_rlane(c.hi[k], 0);
+        for (int k = 0; k < 3; k++) {
+            lo[k]   = fminf(lo[k], og_dpp<0xB1>(lo[k]));
+            hi[k]   = fmaxf(hi[k], og_dpp<0xB1>(hi[k]));
+            lo[k]   = fminf(lo[k], og_dpp<0x4E>(lo[k]));
+            hi[k]   = fmaxf(hi[k], og_dpp<0x4E>(hi[k]));
+            c.lo[k] = fminf(lo[k], og_dpp<0x141>(lo[k]));
+            c.hi[k] = og_rlane(fmaxf(hi[k], og_dpp<0x141>(hi[k])), 0);  // one scalar operand per instruction
         }
     }
 
@@ -370,58 +416,58 @@ __device__ __forceinline__ void og_pair_cell(const og_dev_sys &s, const int c1, 
     int    qn = 0, qd = 0;               // rows queued / rows evaluated (wave-uniform)
     og_jpend pend{0.0f, 0.0f, 0.0f, 0, false};
 
+    // Two groups in flight: the next group's atoms and the records after them
+    // load while this group is filtered (and its full pass evaluated).
+    atom_t at{og_f4{0.0f, 0.0f, 0.0f, 0.0f}, 0u};
+    if (p0 < p1) at = load_atom(rec.cp);
     for (int base = p0; base < p1; base += OG_NAC) {
-        const int   a2 = (int)(cp & 0xffffffu) * OG_NAC + jl;
-        const og_f4 pj = X[a2];
-        const int   ty = TY[a2];
-        // the next group's records load while this group's atoms are in flight
-        // (past the end: a valid record that the validity flag masks)
-        const int      tn     = base + OG_NAC + (lane >> 3);
-        const bool     validn = tn < p1;
-        const int      tcn    = validn ? tn : p1 - 1;
-        const unsigned cpn    = CP[tcn];
-        const uint64_t mkn    = CM[tcn];
-        // wait for this group's atoms (and types) here, with the next records still in flight
-        asm volatile("" ::"v"(pj.x), "v"(ty));
-        const og_f4    sh = shift[(cp >> 24) & 63u];  // periodic image of the cell pair
-        const float    px = pj.x + sh.x, py = pj.y + sh.y, pz = pj.z + sh.z;
-        const float    gx = fmaxf(fmaxf(c.lo[0] - px, px - c.hi[0]), 0.0f);
-        const float    gy = fmaxf(fmaxf(c.lo[1] - py, py - c.hi[1]), 0.0f);
-        const float    gz = fmaxf(fmaxf(c.lo[2] - pz, pz - c.hi[2]), 0.0f);
-        const unsigned m8 = valid ? (unsigned)(mk >> (8 * jl)) & 0xffu : 0xffu;
-        const bool     use = (gx * gx + gy * gy + gz * gz < rcb2) && m8 != 0xffu;
-        const uint64_t ub  = __ballot(use);
-        const int2     ent = make_int2(a2, (int)((unsigned)ty | (m8 << 24)));
-        if (use) {
+        const atom_t at1  = load_atom(rec1.cp);
+        const rec_t  rec2 = load_rec(base + 2 * OG_NAC);
+        unsigned     m8   = rec.m8;
+        if (p1 - base < OG_NAC) m8 = (lane >> 3) < p1 - base ? m8 : 0xffu;  // lanes past the last record
+        float px = at.p.x, py = at.p.y, pz = at.p.z;
+        if (__builtin_amdgcn_ballot_w64(rec.cp > 0xffffffu)) {  // a periodic image among the group's pairs
+            const og_f4 sh = shift[(rec.cp >> 24) & 63u];
+            px += sh.x;
+            py += sh.y;
+            pz += sh.z;
+        }
+        // distance to the cell1 box
+        const float    gx = px - __builtin_amdgcn_fmed3f(px, c.lo[0], c.hi[0]);
+        const float    gy = py - __builtin_amdgcn_fmed3f(py, c.lo[1], c.hi[1]);
+        const float    gz = pz - __builtin_amdgcn_fmed3f(pz, c.lo[2], c.hi[2]);
+        const uint64_t ub = __builtin_amdgcn_ballot_w64(fmaf(gz, gz, fmaf(gx, gx, gy * gy)) < rcb2) &
+                            __builtin_amdgcn_ballot_w64(m8 != 0xffu);
+        if (__builtin_amdgcn_inverse_ballot_w64(ub)) {
             const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(ub >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)ub, 0u));
             const int slot = (qn + rank) & (OG_QCAP - 1);
-            qp[slot] = og_f4{px, py, pz, pj.w};
-            qa[slot] = ent;
+            const int a2   = (int)(rec.cp & 0xffffffu) * OG_NAC + jl;
+            qp[slot]       = og_f4{px, py, pz, at.p.w};
+            qa[slot]       = make_int2(a2, (int)(at.ty | (m8 << 24)));
         }
         qn += __builtin_popcountll(ub);
         if (qn - qd >= 64) {
             og_pass<FORM, ENERGY, LJ_LDS>(s, c, qp, qa, qd, 64, ljl, LJP, FXJ, FXZ, fi, npair, vmax, vsum, ev, ee, vir, pend);
             qd += 64;
         }
-        cp    = cpn;
-        mk    = mkn;
-        valid = validn;
+        rec  = rec1;
+        rec1 = rec2;
+        at   = at1;
     }
     if (qn > qd)
         og_pass<FORM, ENERGY, LJ_LDS>(s, c, qp, qa, qd, qn - qd, ljl, LJP, FXJ, FXZ, fi, npair, vmax, vsum, ev, ee, vir, pend);
     og_flush_j(FXJ, FXZ, pend);
 
     // i-gradients: reduce-scatter the 24 partial sums over the wave.  After
-    // the xor-32/16/8 steps lane L holds atom L>>3's (x, y, z) summed over 8
+    // the folds over 32, 16 and 8 lane L holds atom L>>3's (x, y, z) summed over 8
     // lanes; an 8-lane butterfly completes the sum.
-    const bool b5 = lane & 32, b4 = lane & 16, b3 = lane & 8;
-    float      h12[12], h6[6], h3[3];
+    float h12[12], h6[6], h3[3];
 #pragma unroll
-    for (int k = 0; k < 12; k++) h12[k] = og_keep_add(fi[k], fi[12 + k], b5, 32);
+    for (int k = 0; k < 12; k++) h12[k] = og_fold32(fi[k], fi[12 + k]);
 #pragma unroll
-    for (int k = 0; k < 6; k++) h6[k] = og_keep_add(h12[k], h12[6 + k], b4, 16);
+    for (int k = 0; k < 6; k++) h6[k] = og_fold16(h12[k], h12[6 + k]);
 #pragma unroll
-    for (int k = 0; k < 3; k++) h3[k] = og_dpp_sum8(og_keep_add(h6[k], h6[3 + k], b3, 8));
+    for (int k = 0; k < 3; k++) h3[k] = og_dpp_sum8(og_fold8(h6[k], h6[3 + k], lane & 8));
     if (!(vmax <= OG_FXJ_ROW_LIMIT) || !(fabsf(vsum) < INFINITY)) atomicOr(&s.cnt->flags, OG_F_NAN);
     if (jl == 0) {
         const int a1 = c1 * OG_NAC + (lane >> 3);
@@ -429,11 +475,9 @@ __device__ __forceinline__ void og_pair_cell(const og_dev_sys &s, const int c1, 
         og_add_fx3(FX, cap, og_fx_slot(a1), (double)h3[0], (double)h3[1], (double)h3[2]);
     }
     if (!ENERGY) return;
-    for (int off = 1; off < 64; off <<= 1) {
-        ev += __shfl_xor(ev, off, 64);
-        ee += __shfl_xor(ee, off, 64);
-        vir += __shfl_xor(vir, off, 64);
-    }
+    ev  = og_wave_sum64(ev);
+    ee  = og_wave_sum64(ee);
+    vir = og_wave_sum64(vir);
     if (lane == 0) {
         OG_GLOBAL(long long) *A = (OG_GLOBAL(long long) *)s.e_acc + (c1 % OG_EACC_SLOTS) * OG_EACC_STRIDE;
         og_atomic_add_fx_g(A + OG_EACC_VDW, og_to_fixed(FORM == 2 ? ev : ev * (-1.0 / 12.0)));
@@ -443,26 +487,15 @@ __device__ __forceinline__ void og_pair_cell(const og_dev_sys &s, const int c1, 
     }
 }
 
-// WAVES waves (one work unit each: a cell, or half of one of the last
-// cells) per block sharing the image table and an LDS
-// copy of the leading rows of the LJ table (as many whole rows as fit in
-// OG_LJ_LDS_ENTRIES; the engine numbers types by frequency, so for water the
-// oxygen and hydrogen rows against every type).  A cell1 whose types are all
-// in it reads LJ pairs from LDS, otherwise from the global table.  The block
-// size is a launch shape the autotuner chooses (results do not depend on it).
-template <int FORM, int WAVES>
-__global__ void __launch_bounds__(64 * WAVES) k_pair(const og_dev_sys *__restrict__ S, const int2 *__restrict__ map) {
+// The block's table of image shifts and its LDS copy of the leading rows of
+// the LJ table (as many whole rows as fit in OG_LJ_LDS_ENTRIES; the engine
+// numbers types by frequency, so for water the oxygen and hydrogen rows
+// against every type); returns the rows held.  Every thread of the block.
+template <int FORM, int THREADS>
+__device__ __forceinline__ int og_pair_tables(const og_dev_sys &s, og_f4 *shift, typename og_ljt<FORM>::type *ljl) {
     typedef typename og_ljt<FORM>::type ljt;
-    __shared__ og_f4 shift[64];              // image code -> shift of cell2
-    __shared__ ljt   ljl[OG_LJ_LDS_ENTRIES];
-    __shared__ og_f4 qpos[WAVES][OG_QCAP];  // row queue: shifted x, y, z, charge
-    __shared__ int2  qaux[WAVES][OG_QCAP];  // grid slot, LJ column | mask byte << 24
-    const int2        bm = map[blockIdx.x];
-    const og_dev_sys &s  = S[bm.x];
-    // block-uniform exits (one system per block; this kernel never sets the overflow flag)
-    if (og_frozen(s) || (s.cnt->flags & OG_F_CP_OVERFLOW)) return;
     const int nt   = s.n_types;
-    const int rows = min(nt, OG_LJ_LDS_ENTRIES / nt);  // table rows held in LDS
+    const int rows = min(nt, OG_LJ_LDS_ENTRIES(FORM) / nt);
     if (threadIdx.x < 64) {
         // image bits of MiniCell::add_cell_pair (MiniCell.cpp:1174-1187): neg bit -> -L, pos bit -> +L
         const unsigned img = threadIdx.x;
@@ -471,7 +504,52 @@ __global__ void __launch_bounds__(64 * WAVES) k_pair(const og_dev_sys *__restric
                            (img & 16u) ? -L2 : ((img & 32u) ? L2 : 0.0f), 0.0f};
     }
     const ljt *tab = (const ljt *)(FORM == 2 ? (const void *)s.lj_hps : (const void *)s.lj_pair);
-    for (int k = threadIdx.x; k < rows * nt; k += 64 * WAVES) ljl[k] = tab[k];
+    for (int k = threadIdx.x; k < rows * nt; k += THREADS) ljl[k] = tab[k];
+    return rows;
+}
+
+// One work unit: cell c1, half -1 (whole), 0 or 1 (first or second half of
+// its records).  A cell1 whose types are all in the block's LDS rows reads LJ
+// pairs from LDS, otherwise from the global table.
+template <int FORM>
+__device__ __forceinline__ void og_pair_unit(const og_dev_sys &s, const int c1, const int half, const int rows,
+                                             const og_f4 *shift, const typename og_ljt<FORM>::type *ljl, og_f4 *qp,
+                                             int2 *qa) {
+    int p0 = __builtin_amdgcn_readfirstlane(s.cp_head[c1]);
+    int p1 = __builtin_amdgcn_readfirstlane(s.cp_head[c1 + 1]);
+    if (half >= 0) {
+        const int pm = p0 + ((p1 - p0 + 1) >> 1);
+        if (half == 0) p1 = pm;
+        else p0 = pm;
+    }
+    // scalar bounds: the record loop counts and addresses on the scalar unit
+    p0 = __builtin_amdgcn_readfirstlane(p0);
+    p1 = __builtin_amdgcn_readfirstlane(p1);
+    const bool lds = __builtin_amdgcn_readfirstlane(__all(s.gtype[c1 * OG_NAC + (threadIdx.x & 7)] < rows)) != 0;
+    if (og_energy_step(s)) {
+        if (lds) og_pair_cell<FORM, true, true>(s, c1, p0, p1, shift, ljl, qp, qa);
+        else og_pair_cell<FORM, true, false>(s, c1, p0, p1, shift, ljl, qp, qa);
+    } else {
+        if (lds) og_pair_cell<FORM, false, true>(s, c1, p0, p1, shift, ljl, qp, qa);
+        else og_pair_cell<FORM, false, false>(s, c1, p0, p1, shift, ljl, qp, qa);
+    }
+}
+
+// WAVES waves (one work unit each: a cell, or half of one of the last
+// cells) per block.  The block size is a launch shape the autotuner chooses
+// (results do not depend on it).
+template <int FORM, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES) k_pair(const og_dev_sys *__restrict__ S, const int2 *__restrict__ map) {
+    typedef typename og_ljt<FORM>::type ljt;
+    __shared__ og_f4 shift[64];              // image code -> shift of cell2
+    __shared__ ljt   ljl[OG_LJ_LDS_ENTRIES(FORM)];
+    __shared__ og_f4 qpos[WAVES][OG_QCAP];  // row queue: shifted x, y, z, charge
+    __shared__ int2  qaux[WAVES][OG_QCAP];  // grid slot, LJ column | mask byte << 24
+    const int2        bm = map[blockIdx.x];
+    const og_dev_sys &s  = S[bm.x];
+    // block-uniform exits (one system per block; this kernel never sets the overflow flag)
+    if (og_frozen(s) || (s.cnt->flags & OG_F_CP_OVERFLOW)) return;
+    const int rows = og_pair_tables<FORM, 64 * WAVES>(s, shift, ljl);
     __syncthreads();
     // work unit u of the system: cells 0 .. n-m-1 whole, then the last m
     // cells as two units each (first and second half of their records)
@@ -485,21 +563,7 @@ __global__ void __launch_bounds__(64 * WAVES) k_pair(const og_dev_sys *__restric
         c1   = n - m + ((u - (n - m)) >> 1);
         half = (u - (n - m)) & 1;
     }
-    int p0 = __builtin_amdgcn_readfirstlane(s.cp_head[c1]);
-    int p1 = __builtin_amdgcn_readfirstlane(s.cp_head[c1 + 1]);
-    if (half >= 0) {
-        const int pm = p0 + ((p1 - p0 + 1) >> 1);
-        if (half == 0) p1 = pm;
-        else p0 = pm;
-    }
-    const bool lds = __builtin_amdgcn_readfirstlane(__all(s.gtype[c1 * OG_NAC + (threadIdx.x & 7)] < rows)) != 0;
-    if (og_energy_step(s)) {
-        if (lds) og_pair_cell<FORM, true, true>(s, c1, p0, p1, shift, ljl, qpos[w], qaux[w]);
-        else og_pair_cell<FORM, true, false>(s, c1, p0, p1, shift, ljl, qpos[w], qaux[w]);
-    } else {
-        if (lds) og_pair_cell<FORM, false, true>(s, c1, p0, p1, shift, ljl, qpos[w], qaux[w]);
-        else og_pair_cell<FORM, false, false>(s, c1, p0, p1, shift, ljl, qpos[w], qaux[w]);
-    }
+    og_pair_unit<FORM>(s, c1, half, rows, shift, ljl, qpos[w], qaux[w]);
 }
 
 // Per atom: fixed-point pair gradient -> FP64 "work" with the atom's
@@ -529,26 +593,23 @@ __global__ void __launch_bounds__(64) k_energy_reduce(const og_dev_sys *__restri
 }
 
 // ------------------------------------------------------------- launchers --
-template <int WAVES>
-static void og_launch_pair_w(const og_launch &a, int form) {
-    if (form == OG_FORM_HPS_DH)
-        hipLaunchKernelGGL((k_pair<2, WAVES>), dim3(a.n_blocks), dim3(64 * WAVES), 0, a.stream, a.sys, a.map);
-    else if (form == OG_FORM_ZM)
-        hipLaunchKernelGGL((k_pair<3, WAVES>), dim3(a.n_blocks), dim3(64 * WAVES), 0, a.stream, a.sys, a.map);
-    else if (form == OG_FORM_ZM_ALPHA)
-        hipLaunchKernelGGL((k_pair<4, WAVES>), dim3(a.n_blocks), dim3(64 * WAVES), 0, a.stream, a.sys, a.map);
-    else if (form == OG_FORM_ZD_ALPHA)
-        hipLaunchKernelGGL((k_pair<1, WAVES>), dim3(a.n_blocks), dim3(64 * WAVES), 0, a.stream, a.sys, a.map);
-    else
-        hipLaunchKernelGGL((k_pair<0, WAVES>), dim3(a.n_blocks), dim3(64 * WAVES), 0, a.stream, a.sys, a.map);
+template <int FORM>
+static void og_launch_pair_form(const og_launch &a, int waves) {
+    switch (waves) {
+    case 1: hipLaunchKernelGGL((k_pair<FORM, 1>), dim3(a.n_blocks), dim3(64), 0, a.stream, a.sys, a.map); break;
+    case 2: hipLaunchKernelGGL((k_pair<FORM, 2>), dim3(a.n_blocks), dim3(128), 0, a.stream, a.sys, a.map); break;
+    case 8: hipLaunchKernelGGL((k_pair<FORM, 8>), dim3(a.n_blocks), dim3(512), 0, a.stream, a.sys, a.map); break;
+    default: hipLaunchKernelGGL((k_pair<FORM, 4>), dim3(a.n_blocks), dim3(256), 0, a.stream, a.sys, a.map); break;
+    }
 }
 
 void og_launch_pair(const og_launch &a, int form, int waves) {
-    switch (waves) {
-    case 1: og_launch_pair_w<1>(a, form); break;
-    case 2: og_launch_pair_w<2>(a, form); break;
-    case 8: og_launch_pair_w<8>(a, form); break;
-    default: og_launch_pair_w<4>(a, form); break;
+    switch (form) {
+    case OG_FORM_HPS_DH: og_launch_pair_form<2>(a, waves); break;
+    case OG_FORM_ZM: og_launch_pair_form<3>(a, waves); break;
+    case OG_FORM_ZM_ALPHA: og_launch_pair_form<4>(a, waves); break;
+    case OG_FORM_ZD_ALPHA: og_launch_pair_form<1>(a, waves); break;
+    default: og_launch_pair_form<0>(a, waves); break;
     }
 }
 void og_launch_forces_to_work(const og_launch &a) {
