@@ -152,6 +152,11 @@ og_status cs_maps() {
 
 og_launch cs_launch(int2 *map, int nb) { return og_launch{g_cs.d_sys, map, nb, g_cs.stream}; }
 
+void cs_launch_pair(int form) {
+    if (g_cs.n_cells <= OG_TEAM_CELLS) og_launch_pair_team(cs_launch(nullptr, g_cs.n_cells), form);
+    else og_launch_pair(cs_launch(g_cs.map_cellw, g_cs.nb_cellw), form, 4);
+}
+
 // exclusion-connectivity components (union-find), as og_system_create does
 std::vector<int> cs_components(int n, const int *tab) {
     std::vector<int> p(n);
@@ -234,10 +239,11 @@ int og_alloc_atom_info(int max_n_atoms_exbox, int max_n_cells, int max_n_cell_pa
     g_cs.max_n_cells       = max_n_cells;
     g_cs.max_n_cell_pairs  = max_n_cell_pairs;
     g_cs.n_columns_alloc   = n_columns;
-    // whole groups of four cells: the fixed-point gradient layout (og_fx_slot) permutes within them
+    // the fixed-point gradient rounds up further (OG_FX_CAP)
     const int cap          = (std::max(g_cs.max_n_atom_array, max_n_cells * OG_NAC) + 31) / 32 * 32;
     h.cap_atom_array       = cap;
     h.cap_cells            = cap / OG_NAC;
+    h.head_cells           = h.cap_cells;
     h.cap_cell_pairs       = max_n_cell_pairs;
     h.n_atoms              = max_n_atoms_exbox;
     h.gap_bug              = 1;
@@ -612,7 +618,7 @@ int og_pairwise_ljzd(bool flg_mod_15mask) {
     og_dev_sys &h = g_cs.h;
     CS_TRY(cs_push_sys());
     CS_HIP(hipMemsetAsync(h.fx, 0, sizeof(long long) * OG_FX_WORDS(h.cap_atom_array), g_cs.stream));
-    og_launch_pair(cs_launch(g_cs.map_cellw, g_cs.nb_cellw), OG_FORM_ZD, 4);
+    cs_launch_pair(OG_FORM_ZD);
     og_launch_energy_reduce(cs_launch(g_cs.map_sys, 1));
     CS_HIP(hipGetLastError());
     return OG_OK;
@@ -628,7 +634,7 @@ int og_pairwise_hps_dh(bool flg_mod_15mask) {
     og_dev_sys &h = g_cs.h;
     CS_TRY(cs_push_sys());
     CS_HIP(hipMemsetAsync(h.fx, 0, sizeof(long long) * OG_FX_WORDS(h.cap_atom_array), g_cs.stream));
-    og_launch_pair(cs_launch(g_cs.map_cellw, g_cs.nb_cellw), OG_FORM_HPS_DH, 4);
+    cs_launch_pair(OG_FORM_HPS_DH);
     og_launch_energy_reduce(cs_launch(g_cs.map_sys, 1));
     CS_HIP(hipGetLastError());
     return OG_OK;

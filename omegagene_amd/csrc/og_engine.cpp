@@ -271,6 +271,7 @@ struct og_exec {
     bool                     any_bonded = false, any_quad = false;
     bool                     fused = false;       // every member takes the fused Langevin step
     int                      pair_shape = OG_PAIR_DEFAULT;  // pair-kernel launch shape (KIND_PAIR + pair_shape)
+    long long                cells = 0;           // cells of all members, at most a few per cent short
     int                      intvl = 1;
     int                      graph_steps = 0;     // steps per captured graph (0: automatic)
 };
@@ -316,6 +317,7 @@ og_status exec_prepare(og_exec &x) {
     x.any_langevin = x.any_leapfrog = x.any_com = x.any_constraint = x.any_vcmd = x.any_thermo = false;
     x.any_bonded = x.any_quad = x.any_vmcmd = false;
     x.fused        = true;
+    x.cells        = 0;
     x.intvl        = x.members[0]->prm.nsgrid_update_intvl;
     for (int si = 0; si < ns; si++) {
         og_system *s = x.members[si];
@@ -340,6 +342,7 @@ og_status exec_prepare(og_exec &x) {
         x.any_bonded |= d.n_bterms > 0;
         x.any_quad |= d.constraint != 0 && d.n_quads > 0;
         x.fused &= d.integrator == 1 && d.n_water_blocks > 0;
+        x.cells += cdiv(d.n_atoms, OG_NAC);
         const int n_bins = (d.n_columns + 1) * d.n_uni_z;
         int       cnt[KIND_N];
         cnt[KIND_ATOM]  = cdiv(d.n_atoms, OG_THREADS);
@@ -442,11 +445,19 @@ void enqueue_rebuild(og_exec &x) {
     og_launch_masks(L(x, KIND_CELLW));
 }
 
+void launch_pair(const og_exec &x, int shape) {
+    const bool t = (shape & 3) == 2 && x.cells <= OG_TEAM_CELLS;
+    og_launch  a = L(x, KIND_PAIR + (t ? shape & ~3 : shape));  // a team: the map of one unit per block
+    if (x.members.size() == 1 && shape < 4) a.map = nullptr;  // blocks in order: the map is the identity
+    if (t) og_launch_pair_team(a, x.pair_form);
+    else og_launch_pair(a, x.pair_form, 1 << (shape & 3));
+}
+
 // reduce: reduce the energies now (a single-point call); an MD step reduces
 // them in its closing kernel instead
 void enqueue_forces(og_exec &x, hipEvent_t e0, hipEvent_t e1, bool reduce = false) {
     if (e0) hipEventRecord(e0, x.stream);
-    og_launch_pair(L(x, KIND_PAIR + x.pair_shape), x.pair_form, 1 << (x.pair_shape & 3));
+    launch_pair(x, x.pair_shape);
     if (e1) hipEventRecord(e1, x.stream);
     // angles, torsions, impropers, 1-4 pairs: each atom's shares, summed with its pair gradient below (or in
     // the fused step kernel)
@@ -673,8 +684,9 @@ og_status sys_alloc(og_system *s, const og_system_desc *d, const og_params *p) {
     const GridGeom &g = s->geom;
     h.n_columns = g.n_columns;
     h.nx = g.nx, h.ny = g.ny, h.nnx = g.nnx, h.nny = g.nny, h.n_uni_z = g.n_uni_z;
-    h.cap_atom_array = (n + g.n_columns * OG_NAC + 31) / 32 * 32;  // whole groups of four cells (og_fx_slot)
+    h.cap_atom_array = (n + g.n_columns * OG_NAC + 31) / 32 * 32;  // OG_FX_CAP rounds up further
     h.cap_cells      = h.cap_atom_array / OG_NAC;
+    h.head_cells     = h.cap_cells;
     h.pair_split     = OG_PAIR_SPLIT;
     h.cap_cell_pairs   = pair_capacity(g, n, h.cap_cells, p->capacity_factor);
     h.n_types          = d->n_lj_types;
@@ -1127,11 +1139,9 @@ og_status exec_autotune(og_exec &x, int trials, int *shape_out, double *ms_out) 
     // shapes: waves per block in each block order (for one system only orders 0 and 3 differ)
     for (int shp = 0; shp < 16; shp++) {
         if (x.members.size() == 1 && shp >= 4 && shp < 12) continue;
-        const og_launch a = L(x, KIND_PAIR + shp);
-        const int       w = 1 << (shp & 3);
-        og_launch_pair(a, x.pair_form, w);
+        launch_pair(x, shp);
         OG_HIP(hipEventRecord(e0, x.stream));
-        for (int t = 0; t < trials; t++) og_launch_pair(a, x.pair_form, w);
+        for (int t = 0; t < trials; t++) launch_pair(x, shp);
         OG_HIP(hipEventRecord(e1, x.stream));
         OG_HIP(hipEventSynchronize(e1));
         float ms = 0.0f;

@@ -89,6 +89,8 @@ struct og_dev_sys {
     int n_atoms;
     int n_columns, nx, ny, nnx, nny, n_uni_z;
     int cap_atom_array, cap_cells, cap_cell_pairs;
+    int head_cells;        // cells for which cp_head[c + 1] and the grid slots exist (the pair kernel reads them
+                           // before it knows the cell count)
     int n_types;
     int n_excess, n_bonds, n_trios, n_pairs_c, n_settle;
     int n_angles, n_torsions, n_impros, n_nb14;  // bonded terms beyond bonds (og_bonded.hip)
@@ -454,7 +456,6 @@ __device__ __forceinline__ void og_take_pair_energies(const og_dev_sys &s, long 
 }
 
 
-
 __device__ __forceinline__ void og_atomic_add_fx(long long *p, long long v) {
     if (v != 0) atomicAdd((unsigned long long *)p, (unsigned long long)v);
 }
@@ -477,7 +478,7 @@ __device__ __forceinline__ float og_key_float(uint32_t k) {
 // kernel launch declarations (defined in og_grid.hip, og_pair.hip, og_integrate.hip)
 struct og_launch {
     const og_dev_sys *sys;   // device array
-    const int2       *map;   // device block map
+    const int2       *map;   // device block map (pair kernel, null: one system, blocks in order)
     int               n_blocks;
     hipStream_t       stream;
 };
@@ -498,6 +499,14 @@ void og_launch_masks(const og_launch &cp);
 // pair forms of og_launch_pair
 enum { OG_FORM_ZD = 0, OG_FORM_ZD_ALPHA = 1, OG_FORM_HPS_DH = 2, OG_FORM_ZM = 3, OG_FORM_ZM_ALPHA = 4 };
 void og_launch_pair(const og_launch &cells, int form, int waves);  // waves per block: 1, 2, 4 or 8
+// The same units and bits, a block of four waves on each unit: for launches of
+// at most OG_TEAM_CELLS cells.  A team's block takes 30 KB LDS and four to five
+// fit a CU, so up to about 1,000 units run at once, each on four SIMDs;
+// beyond, the last blocks wait for a whole unit's time.  Measured against a
+// wave per unit (us): 3,000 atoms 18.2 / 23.7, 4,230 19.9 / 24.3, 6,000
+// 21.9 / 25.0, 8,000 (1,000 cells and the columns' padding) 28.1 / 25.6.
+constexpr long long OG_TEAM_CELLS = 900;
+void og_launch_pair_team(const og_launch &units, int form);
 void og_launch_forces_to_work(const og_launch &atoms);
 void og_launch_energy_reduce(const og_launch &sys);
 // integration

@@ -3,14 +3,14 @@
 //
 // The caller owns every input and output buffer on the device.  What the
 // kernels need beyond them -- the system record the pair kernel reads, its
-// counters, the block map, the fixed-point gradient accumulators and the
-// energy accumulators -- lives in one file-scope device array, `scratch`,
+// counters, the fixed-point gradient accumulators and the energy
+// accumulators -- lives in one file-scope device array, `scratch`,
 // sized for OG_NOALLOC_MAX_ATOM_ARRAY grid slots.  Each GPU holds its own
 // copy for the life of the process; its device address is taken once per
 // device with hipGetSymbolAddress and only that address is used from the
-// host.  The call is four kernel launches on the caller's stream: set-up
-// (record, counters, block map, zeroed accumulators), the pair kernel of
-// og_pair.hip, the energy reduction, and the conversion to FP64 work.  It
+// host.  The call is three kernel launches on the caller's stream: set-up
+// (record, counters, zeroed accumulators), the pair kernel of og_pair.hip,
+// and the conversion to FP64 work with the energy reduction.  It
 // calls no allocator, no memset and no copy, so it can be captured into a
 // HIP graph.  Calls that overlap on one GPU share the array and race.
 #include "og_internal.h"
@@ -31,20 +31,19 @@ constexpr size_t kOffSys    = 0;
 constexpr size_t kOffCnt    = kOffSys + na_round(sizeof(og_dev_sys));
 constexpr size_t kOffEacc   = kOffCnt + na_round(sizeof(og_dev_counters));
 constexpr size_t kOffEnergy = kOffEacc + na_round(sizeof(long long) * OG_EACC_SLOTS * OG_EACC_STRIDE);
-constexpr size_t kOffMap    = kOffEnergy + na_round(sizeof(double) * OG_E_NTERMS);
-constexpr size_t kOffFx     = kOffMap + na_round(sizeof(int2) * kMaxCells);
+constexpr size_t kOffFx     = kOffEnergy + na_round(sizeof(double) * OG_E_NTERMS);
 constexpr size_t kBytes     = kOffFx + sizeof(long long) * OG_FX_WORDS(kMaxSlots);
 constexpr int    kWaves     = 4;  // waves (cells) per pair-kernel block
-static_assert(kMaxSlots % 32 == 0, "the fixed-point layout permutes slots within groups of 32");
+static_assert(kMaxSlots % 64 == 0, "the fixed-point layout permutes slots within groups of 64");
 
 }  // namespace
 
-// about 11.3 MiB per GPU at 262,144 slots
+// about 9.1 MiB per GPU at 262,144 slots
 static __device__ __align__(256) unsigned char scratch[kBytes];
 
 namespace {
 
-// Record, counters and block map into the scratch array; accumulators zeroed.
+// Record and counters into the scratch array; accumulators zeroed.
 __global__ void __launch_bounds__(OG_THREADS) k_na_setup(unsigned char *base, og_dev_sys sys, int n_cells) {
     const int g      = blockIdx.x * OG_THREADS + threadIdx.x;
     const int stride = gridDim.x * OG_THREADS;
@@ -52,8 +51,6 @@ __global__ void __launch_bounds__(OG_THREADS) k_na_setup(unsigned char *base, og
     for (size_t k = g; k < OG_FX_WORDS(sys.cap_atom_array); k += stride) fx[k] = 0;
     long long *eacc = (long long *)(base + kOffEacc);
     for (int k = g; k < OG_EACC_SLOTS * OG_EACC_STRIDE; k += stride) eacc[k] = 0;
-    int2 *map = (int2 *)(base + kOffMap);
-    for (int k = g; k < (n_cells + kWaves - 1) / kWaves; k += stride) map[k] = make_int2(0, k);
     if (g == 0) {
         *(og_dev_sys *)(base + kOffSys) = sys;
         og_dev_counters c{};
@@ -67,13 +64,19 @@ __global__ void __launch_bounds__(OG_THREADS) k_na_setup(unsigned char *base, og
 }
 
 // Grid-order FP64 work, the energies {vdw, ele} and the status flags out to
-// the caller (the layout of og_memcpy_dtoh_work).
+// the caller (the layout of og_memcpy_dtoh_work).  The energy accumulators
+// are reduced by the first block (a launch of its own took 4.6 us of 40).
 __global__ void __launch_bounds__(OG_THREADS) k_na_out(const og_dev_sys *__restrict__ S, double *__restrict__ work,
                                                        double *__restrict__ energy, int *__restrict__ flags,
                                                        int n_atom_array) {
     const og_dev_sys &s = S[0];
     const int         g = blockIdx.x * OG_THREADS + threadIdx.x;
     if (g < n_atom_array) og_fx_read(s.fx, s.cap_atom_array, og_fx_slot(g), work + 3 * (size_t)g);
+    if (blockIdx.x != 0) return;
+    if (!og_frozen(s)) {
+        __shared__ long long sh[16 * OG_EACC_STRIDE];
+        og_take_pair_energies<OG_THREADS>(s, sh);
+    }
     if (g == 0) {
         energy[0] = s.energy[OG_E_VDW];
         energy[1] = s.energy[OG_E_ELE];
@@ -133,6 +136,7 @@ extern "C" int og_pairwise_ljzd_noalloc(const float *d_xyzq, const int *d_atom_t
     h.n_atoms        = n_atom_array;
     h.cap_atom_array = (n_atom_array + 31) / 32 * 32;
     h.cap_cells      = h.cap_atom_array / OG_NAC;
+    h.head_cells     = n_cells;  // the caller's arrays end there
     h.n_types        = n_lj_types;
     h.gap_bug        = 1;
     h.log_stride     = 1;  // energies on every evaluation, as og_pairwise_ljzd
@@ -156,13 +160,12 @@ extern "C" int og_pairwise_ljzd_noalloc(const float *d_xyzq, const int *d_atom_t
     h.energy   = (double *)(base + kOffEnergy);
     h.cnt      = (og_dev_counters *)(base + kOffCnt);
     const og_dev_sys *d_sys = (const og_dev_sys *)(base + kOffSys);
-    const int2       *d_map = (const int2 *)(base + kOffMap);
     hipStream_t       st    = (hipStream_t)stream;
 
     const int nb_setup = (4 * h.cap_atom_array + OG_THREADS - 1) / OG_THREADS;
     hipLaunchKernelGGL(k_na_setup, dim3(nb_setup), dim3(OG_THREADS), 0, st, base, h, n_cells);
-    og_launch_pair(og_launch{d_sys, d_map, (n_cells + kWaves - 1) / kWaves, st}, 0, kWaves);
-    og_launch_energy_reduce(og_launch{d_sys, d_map, 1, st});
+    if (n_cells <= OG_TEAM_CELLS) og_launch_pair_team(og_launch{d_sys, nullptr, n_cells, st}, OG_FORM_ZD);
+    else og_launch_pair(og_launch{d_sys, nullptr, (n_cells + kWaves - 1) / kWaves, st}, OG_FORM_ZD, kWaves);
     hipLaunchKernelGGL(k_na_out, dim3((n_atom_array + OG_THREADS - 1) / OG_THREADS), dim3(OG_THREADS), 0, st, d_sys,
                        d_work, d_energy, d_flags, n_atom_array);
     const hipError_t e = hipGetLastError();

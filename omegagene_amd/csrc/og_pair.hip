@@ -76,6 +76,12 @@ struct og_cell1 {
     float    lo[3], hi[3];
 };
 
+// Sums of a row over the cell1 atoms, in atom order: j-gradient (before its
+// sign), LJ and electrostatic energy, virial.
+struct og_chain {
+    float x, y, z, e, q, v;
+};
+
 // j-gradient of the last pass, not yet added: its fixed-point atomics are
 // issued after the next pass has read its rows, so they complete while that
 // pass computes.  (A vector-memory wait counts stores and atomics too, so an
@@ -124,14 +130,14 @@ __device__ __forceinline__ void og_flush_j(OG_GLOBAL(char) *FXJ, OG_GLOBAL(char)
 
 // One pass over up to 64 queued rows (lane = row; lanes >= cnt idle).
 // m8: the row's excluded pairs (bit i set = skip atom i).  LJ_LDS: the
-// cell1's types are rows of the block's LDS copy of the LJ table.
-template <int FORM, bool ENERGY, bool LJ_LDS>
+// cell1's types are rows of the block's LDS copy of the LJ table.  The
+// i-gradients are added to fi, or (COEF, a team wave) each pair's gradient
+// coefficient is left in fi[i] for the wave that sums atom i.
+template <int FORM, bool ENERGY, bool LJ_LDS, bool COEF>
 __device__ __forceinline__ void og_rows(const og_dev_sys &s, const og_cell1 &c, const og_f4 pj, const unsigned tj,
-                                        const unsigned m8, const int a2, const bool live,
-                                        const typename og_ljt<FORM>::type *__restrict__ ljl,
+                                        const unsigned m8, const typename og_ljt<FORM>::type *__restrict__ ljl,
                                         const OG_GLOBAL(typename og_ljt<FORM>::type) *__restrict__ LJP,
-                                        float (&fi)[3 * OG_NAC], int &npair, float &vmax, float &vsum, double &ev,
-                                        double &ee, double &vir, og_jpend &pend) {
+                                        float (&fi)[COEF ? OG_NAC : 3 * OG_NAC], int &npair, og_chain &ch) {
     const float rc2 = s.cutoff2;
     const float zcore = og_vgpr(s.zcore), bcoeff = og_vgpr(s.bcoeff), fcoeff = og_vgpr(s.fcoeff);
     const float alpha = s.alpha, piewald = s.piewald;
@@ -141,7 +147,7 @@ __device__ __forceinline__ void og_rows(const og_dev_sys &s, const og_cell1 &c, 
     const bool  dh_fix_on = s.dh_grad_fix != 0;
     float fjx = 0.0f, fjy = 0.0f, fjz = 0.0f, fe = 0.0f, fq = 0.0f, fv = 0.0f;
     float px = pj.x, py = pj.y, pz = pj.z, pw = pj.w;
-    // the row's eight LJ pairs {A6, A12} load together, ahead of their use
+    // the row's LJ pairs {A6, A12} load together, ahead of their use
     typename og_ljt<FORM>::type ljv[OG_NAC];
 #pragma unroll
     for (int i = 0; i < OG_NAC; i++) ljv[i] = LJ_LDS ? ljl[c.row[i] + tj] : LJP[c.row[i] + tj];
@@ -225,9 +231,13 @@ __device__ __forceinline__ void og_rows(const og_dev_sys &s, const og_cell1 &c, 
         fjx               = fmaf(g, dx, fjx);
         fjy               = fmaf(g, dy, fjy);
         fjz               = fmaf(g, dz, fjz);
-        fi[3 * i]         = fmaf(g, dx, fi[3 * i]);
-        fi[3 * i + 1]     = fmaf(g, dy, fi[3 * i + 1]);
-        fi[3 * i + 2]     = fmaf(g, dz, fi[3 * i + 2]);
+        if constexpr (COEF) {
+            fi[i] = g;
+        } else {
+            fi[3 * i]     = fmaf(g, dx, fi[3 * i]);
+            fi[3 * i + 1] = fmaf(g, dy, fi[3 * i + 1]);
+            fi[3 * i + 2] = fmaf(g, dz, fi[3 * i + 2]);
+        }
         if (ENERGY) {
             fe += ZSEL || ok ? elj : 0.0f;
             fq += ZSEL || ok ? eel : 0.0f;
@@ -235,23 +245,20 @@ __device__ __forceinline__ void og_rows(const og_dev_sys &s, const og_cell1 &c, 
         }
         // finish atom i here: without this the compiler defers the
         // accumulations and keeps all 8 atoms' distances live
-        asm volatile("" : "+v"(fjx), "+v"(fjy), "+v"(fjz), "+v"(fi[3 * i]), "+v"(fi[3 * i + 1]), "+v"(fi[3 * i + 2]),
-                     "+v"(px), "+v"(py), "+v"(pz), "+v"(pw));
+        if constexpr (COEF)
+            asm volatile("" : "+v"(fjx), "+v"(fjy), "+v"(fjz), "+v"(fi[i]), "+v"(px), "+v"(py), "+v"(pz), "+v"(pw));
+        else
+            asm volatile("" : "+v"(fjx), "+v"(fjy), "+v"(fjz), "+v"(fi[3 * i]), "+v"(fi[3 * i + 1]),
+                         "+v"(fi[3 * i + 2]), "+v"(px), "+v"(py), "+v"(pz), "+v"(pw));
         if constexpr (ENERGY) asm volatile("" : "+v"(fe), "+v"(fq), "+v"(fv));
     }
-    pend.x    = fjx;
-    pend.y    = fjy;
-    pend.z    = fjz;
-    pend.a    = a2;
-    pend.live = live;
-    // range check of the converted values; fmaxf drops NaN, the sum keeps it
-    vmax = fmaxf(vmax, fmaxf(fabsf(fjx), fmaxf(fabsf(fjy), fabsf(fjz))));
-    vsum += fjx + fjy + fjz;
-    if (ENERGY) {
-        ev += (double)fe;
-        ee += (double)fq;
-        vir += (double)fv;
-    }
+    ch = og_chain{fjx, fjy, fjz, fe, fq, fv};
+}
+
+// range check of a pass's j-gradients; fmaxf drops NaN, the sum keeps it
+__device__ __forceinline__ void og_range(const og_chain &ch, float &vmax, float &vsum) {
+    vmax = fmaxf(vmax, fmaxf(fabsf(ch.x), fmaxf(fabsf(ch.y), fabsf(ch.z))));
+    vsum += ch.x + ch.y + ch.z;
 }
 
 // Pass over queue entries [q0, q0 + cnt) (q0 a multiple of 64): reads the
@@ -280,7 +287,137 @@ __device__ __forceinline__ void og_pass(const og_dev_sys &s, const og_cell1 &c, 
     // (s_waitcnt vmcnt(0); expcnt and lgkmcnt left at their maxima)
     __builtin_amdgcn_s_waitcnt(0x0F70);
     og_flush_j(FXJ, FXZ, pend);
-    og_rows<FORM, ENERGY, LJ_LDS>(s, c, pj, tj, m8, ax.x, live, ljl, LJP, fi, npair, vmax, vsum, ev, ee, vir, pend);
+    og_chain ch;
+    og_rows<FORM, ENERGY, LJ_LDS, false>(s, c, pj, tj, m8, ljl, LJP, fi, npair, ch);
+    og_range(ch, vmax, vsum);
+    pend = og_jpend{ch.x, ch.y, ch.z, ax.x, live};
+    if (ENERGY) {
+        ev += (double)ch.e;
+        ee += (double)ch.q;
+        vir += (double)ch.v;
+    }
+}
+
+// What the filter reads: grid-order atoms and types, cell-pair records.
+struct og_list {
+    const OG_GLOBAL(char) *X, *TY, *CP, *CM;
+};
+// Cell-pair record of a lane (lane = 8 * record + j atom): cell2 | image << 24
+// and the j atom's mask byte.
+struct og_rec {
+    unsigned cp, m8;
+};
+// The group of eight records at base.  Uniform base plus a lane offset that is
+// constant but for the last group, where lanes past the end read its last record.
+__device__ __forceinline__ og_rec og_load_rec(const og_list &L, const int base, const int p1) {
+    const int lane = threadIdx.x & 63;
+    const int b = min(base, p1 - 1), r = p1 - b;
+    unsigned  k = (unsigned)lane >> 3;
+    if (r < OG_NAC) k = min(k, (unsigned)(r - 1));
+    og_rec t;
+    t.cp = *(const OG_GLOBAL(unsigned) *)(L.CP + 4 * (size_t)b + 4u * k);
+    t.m8 = *((const OG_GLOBAL(unsigned char) *)(L.CM + 8 * (size_t)b) + (8u * k + (unsigned)(lane & 7)));
+    return t;
+}
+struct og_jatom {
+    og_f4    p;
+    unsigned ty;
+};
+__device__ __forceinline__ og_jatom og_load_atom(const og_list &L, const unsigned cp) {
+    const unsigned off = ((cp << 7) & 0x7fffffffu) | ((threadIdx.x & 7u) << 4);  // 16 bytes per slot
+    og_jatom       t;
+    t.p  = *(const OG_GLOBAL(og_f4) *)(L.X + off);
+    t.ty = *(const OG_GLOBAL(unsigned) *)(L.TY + (off >> 2));
+    return t;
+}
+// Filter of one group: shifts the lanes' atoms to their pairs' periodic images
+// and returns the mask of the lanes to keep (within the cutoff of the cell1
+// box and not masked against all its atoms).
+__device__ __forceinline__ uint64_t og_keep(const float (&lo)[3], const float (&hi)[3], const float rcb2,
+                                            const og_f4 *__restrict__ shift, const unsigned cp, const unsigned m8,
+                                            og_f4 &p) {
+    if (__builtin_amdgcn_ballot_w64(cp > 0xffffffu)) {  // a periodic image among the group's pairs
+        const og_f4 sh = shift[(cp >> 24) & 63u];
+        p.x += sh.x;
+        p.y += sh.y;
+        p.z += sh.z;
+    }
+    const float gx = p.x - __builtin_amdgcn_fmed3f(p.x, lo[0], hi[0]);
+    const float gy = p.y - __builtin_amdgcn_fmed3f(p.y, lo[1], hi[1]);
+    const float gz = p.z - __builtin_amdgcn_fmed3f(p.z, lo[2], hi[2]);
+    return __builtin_amdgcn_ballot_w64(fmaf(gz, gz, fmaf(gx, gx, gy * gy)) < rcb2) &
+           __builtin_amdgcn_ballot_w64(m8 != 0xffu);
+}
+// The cell1's atoms and box from the lanes' atoms p and types ty (lane & 7).
+template <int FORM>
+__device__ __forceinline__ void og_set_cell1(const og_dev_sys &s, const og_f4 p, const int ty, og_cell1 &c) {
+    // charge x 332.06378 (x 1/eps_r under Debye-Hueckel)
+    const float qc = FORM == 2 ? p.w * OG_CHARGE_COEFF * s.dh_diel_inv : p.w * OG_CHARGE_COEFF;
+#pragma unroll
+    for (int i = 0; i < OG_NAC; i++) {
+        c.x[i]   = og_rlane(p.x, i);
+        c.y[i]   = og_rlane(p.y, i);
+        c.z[i]   = og_rlane(p.z, i);
+        c.q[i]   = og_rlane(qc, i);
+        c.row[i] = (unsigned)__builtin_amdgcn_readlane(ty, i) * (unsigned)s.n_types;
+    }
+    // bounding box: minima and maxima over the eight lanes
+    float lo[3] = {p.x, p.y, p.z}, hi[3] = {p.x, p.y, p.z};
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        lo[k]   = fminf(lo[k], og_dpp<0xB1>(lo[k]));
+        hi[k]   = fmaxf(hi[k], og_dpp<0xB1>(hi[k]));
+        lo[k]   = fminf(lo[k], og_dpp<0x4E>(lo[k]));
+        hi[k]   = fmaxf(hi[k], og_dpp<0x4E>(hi[k]));
+        c.lo[k] = fminf(lo[k], og_dpp<0x141>(lo[k]));
+        c.hi[k] = og_rlane(fmaxf(hi[k], og_dpp<0x141>(hi[k])), 0);  // one scalar operand per instruction
+    }
+}
+
+// What a work unit starts from.
+struct og_unit {
+    int   c1, p0, p1;  // its cell and records (scalar)
+    og_f4 p;           // the cell's atom of the lane (lane & 7)
+    int   ty;
+    bool  run, energy;
+};
+// Work unit u of a system with n cells: cells 0 .. n-m-1 whole, then the last
+// m cells as two units each (first and second half of their records).  run is
+// false past the last unit, for a frozen system and after a list overflow.
+// The list head, the cell's atoms and the counters are read together (a unit
+// is a chain of memory round trips of about a microsecond each: block map,
+// system record, these, the records, their atoms); only a unit of the split
+// tail, whose cell follows from the cell count, reads its own again.
+__device__ __forceinline__ og_unit og_unit_start(const og_dev_sys &s, const int u) {
+    const int jl = threadIdx.x & 7;
+    og_unit   t;
+    t.c1 = min(u, s.head_cells - 1);
+    int             a = s.cp_head[t.c1], b = s.cp_head[t.c1 + 1];
+    const OG_GLOBAL(og_f4) *X  = (const OG_GLOBAL(og_f4) *)s.gxyzq;
+    const OG_GLOBAL(int) *TY   = (const OG_GLOBAL(int) *)s.gtype;
+    t.p  = X[t.c1 * OG_NAC + jl];
+    t.ty = TY[t.c1 * OG_NAC + jl];
+    const og_dev_counters &c = *s.cnt;
+    const int              n = c.n_cells, m = og_pair_split_cells(s.pair_split, n);
+    // keeps these loads ahead of the branches on the counters
+    asm volatile("" ::"v"(t.p.x), "v"(t.ty), "s"(a), "s"(b));
+    t.run    = !og_frozen_c(c) && !(c.flags & OG_F_CP_OVERFLOW) && u < n + m;
+    t.energy = og_energy_step_c(s, c);
+    if (u >= n - m && t.run) {
+        const int half = (u - (n - m)) & 1;
+        t.c1 = n - m + ((u - (n - m)) >> 1);
+        a    = s.cp_head[t.c1], b = s.cp_head[t.c1 + 1];
+        t.p  = X[t.c1 * OG_NAC + jl];
+        t.ty = TY[t.c1 * OG_NAC + jl];
+        const int mid = a + ((b - a + 1) >> 1);
+        if (half == 0) b = mid;
+        else a = mid;
+    }
+    // scalar bounds: the record loop counts and addresses on the scalar unit
+    t.c1 = __builtin_amdgcn_readfirstlane(t.c1);
+    t.p0 = __builtin_amdgcn_readfirstlane(a);
+    t.p1 = __builtin_amdgcn_readfirstlane(b);
+    return t;
 }
 
 // Halves of two registers exchanged and added: lanes of the lower half (of
@@ -316,15 +453,24 @@ __device__ __forceinline__ double og_wave_sum64(double v) {
     return (r[0] + r[1]) + (r[2] + r[3]);
 }
 
+// One energy of the cell (per-lane partial sums v, scaled) into its accumulator slot.
+__device__ __forceinline__ void og_cell_energy(const og_dev_sys &s, const int c1, const int term, double v,
+                                               const double scale) {
+    v = og_wave_sum64(v);
+    if ((threadIdx.x & 63) == 0)
+        og_atomic_add_fx_g((OG_GLOBAL(long long) *)s.e_acc + (c1 % OG_EACC_SLOTS) * OG_EACC_STRIDE + term,
+                           og_to_fixed(v * scale));
+}
+
 // One cell1 (one wave), its cell-pair records [p0, p1) (all of them, or
 // half of them for a split cell).  ENERGY = false on steps whose energies
 // are not logged: forces and the pair count only.  LJ_LDS: the cell1's LJ rows are in
 // the block's LDS copy ljl of the table's leading rows.
 template <int FORM, bool ENERGY, bool LJ_LDS>
-__device__ __forceinline__ void og_pair_cell(const og_dev_sys &s, const int c1, const int p0, const int p1,
-                                             const og_f4 *__restrict__ shift,
+__device__ __forceinline__ void og_pair_cell(const og_dev_sys &s, const og_unit &un, const og_f4 *__restrict__ shift,
                                              const typename og_ljt<FORM>::type *__restrict__ ljl, og_f4 *qp,
                                              int2 *qa) {
+    const int c1 = un.c1, p0 = un.p0, p1 = un.p1;
     const int lane = threadIdx.x & 63;
     const int jl   = lane & 7;
 
@@ -333,11 +479,8 @@ __device__ __forceinline__ void og_pair_cell(const og_dev_sys &s, const int c1, 
     const OG_GLOBAL(char) *__restrict__ TY = (const OG_GLOBAL(char) *)s.gtype;
     const OG_GLOBAL(ljt) *__restrict__ LJP =
         (const OG_GLOBAL(ljt) *)(FORM == 2 ? (const void *)s.lj_hps : (const void *)s.lj_pair);
-    const OG_GLOBAL(unsigned) *__restrict__ CP = (const OG_GLOBAL(unsigned) *)s.cp_c2;
-    const OG_GLOBAL(uint64_t) *__restrict__ CM = (const OG_GLOBAL(uint64_t) *)s.cp_mask;
     OG_GLOBAL(long long) *__restrict__ FX      = (OG_GLOBAL(long long) *)s.fx;
     const int cap = s.cap_atom_array;
-    const int nt  = s.n_types;
     // j-side words of the gradient: packed (x, y) and z, per slot
     OG_GLOBAL(char) *FXJ = (OG_GLOBAL(char) *)(FX + OG_FX_XY(cap));
     OG_GLOBAL(char) *FXZ = (OG_GLOBAL(char) *)(FX + OG_FX_Z(cap));
@@ -345,67 +488,16 @@ __device__ __forceinline__ void og_pair_cell(const og_dev_sys &s, const int c1, 
     // distance can never drop a row that holds an in-range pair
     const float rcb2 = s.cutoff2 * 1.00001f;
 
-    // Cell-pair records of the group of eight at base (lane = 8 * record + j
-    // atom): cell2 | image << 24 and the j atom's mask byte.  Uniform base plus
-    // a lane offset that is constant but for the last group, where lanes past
-    // the end read its last record.
-    struct rec_t {
-        unsigned cp, m8;
-    };
-    auto load_rec = [&](const int base) {
-        const int b = min(base, p1 - 1), r = p1 - b;
-        unsigned  k = (unsigned)lane >> 3;
-        if (r < OG_NAC) k = min(k, (unsigned)(r - 1));
-        rec_t t;
-        t.cp = *(const OG_GLOBAL(unsigned) *)((const OG_GLOBAL(char) *)(CP + b) + 4u * k);
-        t.m8 = *((const OG_GLOBAL(unsigned char) *)(CM + b) + (8u * k + (unsigned)jl));
-        return t;
-    };
-    struct atom_t {
-        og_f4    p;
-        unsigned ty;
-    };
-    auto load_atom = [&](const unsigned cp) {
-        const unsigned off = ((cp << 7) & 0x7fffffffu) | ((unsigned)jl << 4);  // 16 bytes per slot
-        atom_t t;
-        t.p  = *(const OG_GLOBAL(og_f4) *)(X + off);
-        t.ty = *(const OG_GLOBAL(unsigned) *)(TY + (off >> 2));
-        return t;
-    };
-
+    const og_list L{X, TY, (const OG_GLOBAL(char) *)s.cp_c2, (const OG_GLOBAL(char) *)s.cp_mask};
     // the first groups' records load with the cell1 atoms
-    rec_t rec{0u, 0xffu}, rec1{0u, 0xffu};
+    og_rec rec{0u, 0xffu}, rec1{0u, 0xffu};
     if (p0 < p1) {
-        rec  = load_rec(p0);
-        rec1 = load_rec(p0 + OG_NAC);
+        rec  = og_load_rec(L, p0, p1);
+        rec1 = og_load_rec(L, p0 + OG_NAC, p1);
     }
 
     og_cell1 c;
-    {
-        const og_f4 p  = *(const OG_GLOBAL(og_f4) *)(X + (16u * (unsigned)(c1 * OG_NAC + jl)));
-        const int   ty = *(const OG_GLOBAL(int) *)(TY + (4u * (unsigned)(c1 * OG_NAC + jl)));
-        // charge x 332.06378 (x 1/eps_r under Debye-Hueckel)
-        const float qc = FORM == 2 ? p.w * OG_CHARGE_COEFF * s.dh_diel_inv : p.w * OG_CHARGE_COEFF;
-#pragma unroll
-        for (int i = 0; i < OG_NAC; i++) {
-            c.x[i]   = og_rlane(p.x, i);
-            c.y[i]   = og_rlane(p.y, i);
-            c.z[i]   = og_rlane(p.z, i);
-            c.q[i]   = og_rlane(qc, i);
-            c.row[i] = (unsigned)__builtin_amdgcn_readlane(ty, i) * (unsigned)nt;
-        }
-        // bounding box: minima and maxima over the eight lanes
-        float lo[3] = {p.x, p.y, p.z}, hi[3] = {p.x, p.y, p.z};
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            lo[k]   = fminf(lo[k], og_dpp<0xB1>(lo[k]));
-            hi[k]   = fmaxf(hi[k], og_dpp<0xB1>(hi[k]));
-            lo[k]   = fminf(lo[k], og_dpp<0x4E>(lo[k]));
-            hi[k]   = fmaxf(hi[k], og_dpp<0x4E>(hi[k]));
-            c.lo[k] = fminf(lo[k], og_dpp<0x141>(lo[k]));
-            c.hi[k] = og_rlane(fmaxf(hi[k], og_dpp<0x141>(hi[k])), 0);  // one scalar operand per instruction
-        }
-    }
+    og_set_cell1<FORM>(s, un.p, un.ty, c);
 
     float  fi[3 * OG_NAC];
 #pragma unroll
@@ -418,31 +510,19 @@ __device__ __forceinline__ void og_pair_cell(const og_dev_sys &s, const int c1, 
 
     // Two groups in flight: the next group's atoms and the records after them
     // load while this group is filtered (and its full pass evaluated).
-    atom_t at{og_f4{0.0f, 0.0f, 0.0f, 0.0f}, 0u};
-    if (p0 < p1) at = load_atom(rec.cp);
+    og_jatom at{og_f4{0.0f, 0.0f, 0.0f, 0.0f}, 0u};
+    if (p0 < p1) at = og_load_atom(L, rec.cp);
     for (int base = p0; base < p1; base += OG_NAC) {
-        const atom_t at1  = load_atom(rec1.cp);
-        const rec_t  rec2 = load_rec(base + 2 * OG_NAC);
-        unsigned     m8   = rec.m8;
+        const og_jatom at1  = og_load_atom(L, rec1.cp);
+        const og_rec   rec2 = og_load_rec(L, base + 2 * OG_NAC, p1);
+        unsigned       m8   = rec.m8;
         if (p1 - base < OG_NAC) m8 = (lane >> 3) < p1 - base ? m8 : 0xffu;  // lanes past the last record
-        float px = at.p.x, py = at.p.y, pz = at.p.z;
-        if (__builtin_amdgcn_ballot_w64(rec.cp > 0xffffffu)) {  // a periodic image among the group's pairs
-            const og_f4 sh = shift[(rec.cp >> 24) & 63u];
-            px += sh.x;
-            py += sh.y;
-            pz += sh.z;
-        }
-        // distance to the cell1 box
-        const float    gx = px - __builtin_amdgcn_fmed3f(px, c.lo[0], c.hi[0]);
-        const float    gy = py - __builtin_amdgcn_fmed3f(py, c.lo[1], c.hi[1]);
-        const float    gz = pz - __builtin_amdgcn_fmed3f(pz, c.lo[2], c.hi[2]);
-        const uint64_t ub = __builtin_amdgcn_ballot_w64(fmaf(gz, gz, fmaf(gx, gx, gy * gy)) < rcb2) &
-                            __builtin_amdgcn_ballot_w64(m8 != 0xffu);
+        const uint64_t ub = og_keep(c.lo, c.hi, rcb2, shift, rec.cp, m8, at.p);
         if (__builtin_amdgcn_inverse_ballot_w64(ub)) {
             const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(ub >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)ub, 0u));
             const int slot = (qn + rank) & (OG_QCAP - 1);
             const int a2   = (int)(rec.cp & 0xffffffu) * OG_NAC + jl;
-            qp[slot]       = og_f4{px, py, pz, at.p.w};
+            qp[slot]       = at.p;
             qa[slot]       = make_int2(a2, (int)(at.ty | (m8 << 24)));
         }
         qn += __builtin_popcountll(ub);
@@ -475,16 +555,12 @@ __device__ __forceinline__ void og_pair_cell(const og_dev_sys &s, const int c1, 
         og_add_fx3(FX, cap, og_fx_slot(a1), (double)h3[0], (double)h3[1], (double)h3[2]);
     }
     if (!ENERGY) return;
-    ev  = og_wave_sum64(ev);
-    ee  = og_wave_sum64(ee);
-    vir = og_wave_sum64(vir);
-    if (lane == 0) {
-        OG_GLOBAL(long long) *A = (OG_GLOBAL(long long) *)s.e_acc + (c1 % OG_EACC_SLOTS) * OG_EACC_STRIDE;
-        og_atomic_add_fx_g(A + OG_EACC_VDW, og_to_fixed(FORM == 2 ? ev : ev * (-1.0 / 12.0)));
-        og_atomic_add_fx_g(A + OG_EACC_ELE, og_to_fixed(ee));
-        og_atomic_add_fx_g(A + OG_EACC_VIR, og_to_fixed(vir));
-        og_atomic_add_fx_g(A + OG_EACC_PAIRS, (long long)npair);
-    }
+    og_cell_energy(s, c1, OG_EACC_VDW, ev, FORM == 2 ? 1.0 : -1.0 / 12.0);
+    og_cell_energy(s, c1, OG_EACC_ELE, ee, 1.0);
+    og_cell_energy(s, c1, OG_EACC_VIR, vir, 1.0);
+    if (lane == 0)
+        og_atomic_add_fx_g((OG_GLOBAL(long long) *)s.e_acc + (c1 % OG_EACC_SLOTS) * OG_EACC_STRIDE + OG_EACC_PAIRS,
+                           (long long)npair);
 }
 
 // The block's table of image shifts and its LDS copy of the leading rows of
@@ -508,62 +584,275 @@ __device__ __forceinline__ int og_pair_tables(const og_dev_sys &s, og_f4 *shift,
     return rows;
 }
 
-// One work unit: cell c1, half -1 (whole), 0 or 1 (first or second half of
-// its records).  A cell1 whose types are all in the block's LDS rows reads LJ
-// pairs from LDS, otherwise from the global table.
-template <int FORM>
-__device__ __forceinline__ void og_pair_unit(const og_dev_sys &s, const int c1, const int half, const int rows,
-                                             const og_f4 *shift, const typename og_ljt<FORM>::type *ljl, og_f4 *qp,
-                                             int2 *qa) {
-    int p0 = __builtin_amdgcn_readfirstlane(s.cp_head[c1]);
-    int p1 = __builtin_amdgcn_readfirstlane(s.cp_head[c1 + 1]);
-    if (half >= 0) {
-        const int pm = p0 + ((p1 - p0 + 1) >> 1);
-        if (half == 0) p1 = pm;
-        else p0 = pm;
-    }
-    // scalar bounds: the record loop counts and addresses on the scalar unit
-    p0 = __builtin_amdgcn_readfirstlane(p0);
-    p1 = __builtin_amdgcn_readfirstlane(p1);
-    const bool lds = __builtin_amdgcn_readfirstlane(__all(s.gtype[c1 * OG_NAC + (threadIdx.x & 7)] < rows)) != 0;
-    if (og_energy_step(s)) {
-        if (lds) og_pair_cell<FORM, true, true>(s, c1, p0, p1, shift, ljl, qp, qa);
-        else og_pair_cell<FORM, true, false>(s, c1, p0, p1, shift, ljl, qp, qa);
-    } else {
-        if (lds) og_pair_cell<FORM, false, true>(s, c1, p0, p1, shift, ljl, qp, qa);
-        else og_pair_cell<FORM, false, false>(s, c1, p0, p1, shift, ljl, qp, qa);
-    }
-}
-
 // WAVES waves (one work unit each: a cell, or half of one of the last
 // cells) per block.  The block size is a launch shape the autotuner chooses
-// (results do not depend on it).
+// (results do not depend on it).  Five waves per SIMD: the kernel needs 99
+// vector registers when left free (four waves), and holding it to 96 costs a
+// few spills and gains 5% at 450,000 atoms (400 to 380 us with energies; the
+// same at 99,200); the HPS form would spill more.
 template <int FORM, int WAVES>
-__global__ void __launch_bounds__(64 * WAVES) k_pair(const og_dev_sys *__restrict__ S, const int2 *__restrict__ map) {
+__global__ void __launch_bounds__(64 * WAVES, FORM == 2 ? 4 : 5) k_pair(const og_dev_sys *__restrict__ S,
+                                                                       const int2 *__restrict__ map) {
     typedef typename og_ljt<FORM>::type ljt;
     __shared__ og_f4 shift[64];              // image code -> shift of cell2
     __shared__ ljt   ljl[OG_LJ_LDS_ENTRIES(FORM)];
     __shared__ og_f4 qpos[WAVES][OG_QCAP];  // row queue: shifted x, y, z, charge
     __shared__ int2  qaux[WAVES][OG_QCAP];  // grid slot, LJ column | mask byte << 24
-    const int2        bm = map[blockIdx.x];
+    const int2        bm = map ? map[blockIdx.x] : make_int2(0, (int)blockIdx.x);
     const og_dev_sys &s  = S[bm.x];
-    // block-uniform exits (one system per block; this kernel never sets the overflow flag)
-    if (og_frozen(s) || (s.cnt->flags & OG_F_CP_OVERFLOW)) return;
+    const int         w  = threadIdx.x >> 6;
+    const og_unit     un = og_unit_start(s, __builtin_amdgcn_readfirstlane(bm.y * WAVES + w));
     const int rows = og_pair_tables<FORM, 64 * WAVES>(s, shift, ljl);
     __syncthreads();
-    // work unit u of the system: cells 0 .. n-m-1 whole, then the last m
-    // cells as two units each (first and second half of their records)
-    const int w  = threadIdx.x >> 6;
-    const int n  = s.cnt->n_cells;
-    const int m  = og_pair_split_cells(s.pair_split, n);
-    const int u  = __builtin_amdgcn_readfirstlane(bm.y * WAVES + w);
-    if (u >= n + m) return;
-    int c1 = u, half = -1;
-    if (u >= n - m) {
-        c1   = n - m + ((u - (n - m)) >> 1);
-        half = (u - (n - m)) & 1;
+    if (!un.run) return;
+    // a cell1 whose types are all in the block's LDS rows reads LJ pairs from LDS, otherwise from the global table
+    if (un.energy) {
+        if (__all(un.ty < rows)) og_pair_cell<FORM, true, true>(s, un, shift, ljl, qpos[w], qaux[w]);
+        else og_pair_cell<FORM, true, false>(s, un, shift, ljl, qpos[w], qaux[w]);
+    } else {
+        if (__all(un.ty < rows)) og_pair_cell<FORM, false, true>(s, un, shift, ljl, qpos[w], qaux[w]);
+        else og_pair_cell<FORM, false, false>(s, un, shift, ljl, qpos[w], qaux[w]);
     }
-    og_pair_unit<FORM>(s, c1, half, rows, shift, ljl, qpos[w], qaux[w]);
+}
+
+// ------------------------------------------------------ team of waves --
+// The same work unit by a team of four waves (one block), for launches that do
+// not fill the chip: a lone wave issues one VALU instruction per 8 cycles and
+// waits out every load, and takes about 24 us for a unit (6,000 atoms: 784
+// units on 1,024 SIMDs).
+//  * filter: the waves take the groups of eight records in turn and queue
+//    their rows at the positions the one-wave filter would give them (ballot
+//    counts exchanged through LDS);
+//  * rows: the waves evaluate four passes at a time, one each: the j-gradients go
+//    out, the pairs' gradient coefficients and the rows' energies to LDS;
+//  * i side: wave w then sums atoms 2 w and 2 w + 1 over those passes in pass
+//    order, waves 0 to 2 one energy each.
+// Every sum is taken over the same values in the same order as by one wave,
+// so the results are the same bits.  (Dividing the atoms instead, each wave
+// continuing the rows' sums of the one before it a pass behind, measured
+// 24.4 us at 6,000 atoms against 25.6 for one wave: too many steps.)
+// Kernel time, a wave per unit / a team: 3,000 atoms 23.7 / 18.2 us, 6,000
+// 25.0 / 21.9.  What is left: four to six dependent memory round trips before
+// the first pass (about 4 us), and per four passes one of 2,400 cycles and a
+// sum of 1,300.
+#define OG_TEAM 4                                  // waves
+#define OG_TEAM_NI (OG_NAC / OG_TEAM)              // cell1 atoms per wave on the i side
+#define OG_TEAM_NG 2                               // groups per wave and batch
+#define OG_TEAM_G (OG_TEAM_NG * OG_TEAM)           // groups per batch (64 candidate rows each)
+struct og_team {
+    og_f4 qp[OG_TEAM_G * 64 + 64];                 // queue: one batch and a remainder
+    int2  qa[OG_TEAM_G * 64 + 64];
+    float coef[OG_TEAM][OG_NAC][64];               // by pass: gradient coefficients of the row's pairs
+    float en[OG_TEAM][3][64];                      // by pass: the rows' LJ and electrostatic energy and virial
+    int   cnt[2][OG_TEAM_G];                       // rows kept by each group of a batch, by batch parity
+    og_f4 shift[64];
+};
+
+// LDS written by the block's waves is visible after it (no wait for memory)
+__device__ __forceinline__ void og_lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <int FORM, bool ENERGY, bool LJ_LDS>
+__device__ __forceinline__ void og_team_cell(const og_dev_sys &s, const og_unit &un, const int w, og_team &T,
+                                             const typename og_ljt<FORM>::type *__restrict__ ljl) {
+    typedef typename og_ljt<FORM>::type ljt;
+    constexpr int NI = OG_TEAM_NI, NG = OG_TEAM_NG, G = OG_TEAM_G;
+    const int     c1 = un.c1, p0 = un.p0, p1 = un.p1;
+    const int     lane = threadIdx.x & 63, jl = lane & 7, i0 = w * NI;
+    const OG_GLOBAL(ljt) *__restrict__ LJP =
+        (const OG_GLOBAL(ljt) *)(FORM == 2 ? (const void *)s.lj_hps : (const void *)s.lj_pair);
+    const og_list L{(const OG_GLOBAL(char) *)s.gxyzq, (const OG_GLOBAL(char) *)s.gtype,
+                    (const OG_GLOBAL(char) *)s.cp_c2, (const OG_GLOBAL(char) *)s.cp_mask};
+    OG_GLOBAL(long long) *FX = (OG_GLOBAL(long long) *)s.fx;
+    const int   cap  = s.cap_atom_array;
+    OG_GLOBAL(char) *FXJ = (OG_GLOBAL(char) *)(FX + OG_FX_XY(cap));
+    OG_GLOBAL(char) *FXZ = (OG_GLOBAL(char) *)(FX + OG_FX_Z(cap));
+    const float rcb2 = s.cutoff2 * 1.00001f;
+
+    // this wave's groups of the first batch, and the records of the second
+    og_rec   rec[NG], rec1[NG];
+    og_jatom at[NG];
+    if (p0 < p1) {
+#pragma unroll
+        for (int j = 0; j < NG; j++) {
+            rec[j]  = og_load_rec(L, p0 + OG_NAC * (j * OG_TEAM + w), p1);
+            rec1[j] = og_load_rec(L, p0 + OG_NAC * (G + j * OG_TEAM + w), p1);
+        }
+#pragma unroll
+        for (int j = 0; j < NG; j++) at[j] = og_load_atom(L, rec[j].cp);
+    }
+    og_cell1 c;
+    og_set_cell1<FORM>(s, un.p, un.ty, c);
+    float xi[NI], yi[NI], zi[NI];  // the atoms this wave sums
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+        xi[i] = og_vgpr(og_rlane(un.p.x, i0 + i));
+        yi[i] = og_vgpr(og_rlane(un.p.y, i0 + i));
+        zi[i] = og_vgpr(og_rlane(un.p.z, i0 + i));
+    }
+
+    float fi[3 * NI];
+#pragma unroll
+    for (int k = 0; k < 3 * NI; k++) fi[k] = 0.0f;
+    double en = 0.0;  // waves 0, 1, 2: -12 x the LJ energy (except under HPS), electrostatic energy, virial
+    int    npair = 0, qn = 0, parity = 0;
+    float  vmax = 0.0f, vsum = 0.0f;
+    for (int base = p0;;) {
+        if (base < p1) {
+            uint64_t ub[NG];
+#pragma unroll
+            for (int j = 0; j < NG; j++) {
+                const int left = p1 - (base + OG_NAC * (j * OG_TEAM + w));  // records from the group's first to the end
+                if (left < OG_NAC) rec[j].m8 = (lane >> 3) < left ? rec[j].m8 : 0xffu;
+                ub[j] = og_keep(c.lo, c.hi, rcb2, T.shift, rec[j].cp, rec[j].m8, at[j].p);
+                if (lane == 0) T.cnt[parity][j * OG_TEAM + w] = __builtin_popcountll(ub[j]);
+            }
+            og_lds_barrier();
+            // running counts of the batch's groups (lanes 0 .. G - 1): row shifts by 1, 2, 4 lanes
+            static_assert(G == 8, "one row of lanes, three shifts");
+            int sum = T.cnt[parity][lane & (G - 1)];
+            sum += __builtin_amdgcn_update_dpp(0, sum, 0x111, 0xf, 0xf, true);
+            sum += __builtin_amdgcn_update_dpp(0, sum, 0x112, 0xf, 0xf, true);
+            sum += __builtin_amdgcn_update_dpp(0, sum, 0x114, 0xf, 0xf, true);
+#pragma unroll
+            for (int j = 0; j < NG; j++) {
+                const int at0 = qn + __builtin_amdgcn_readlane(sum, j * OG_TEAM + w) - __builtin_popcountll(ub[j]);
+                if (__builtin_amdgcn_inverse_ballot_w64(ub[j])) {
+                    const int slot = at0 + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(ub[j] >> 32),
+                                                                          __builtin_amdgcn_mbcnt_lo((unsigned)ub[j], 0u));
+                    T.qp[slot] = at[j].p;
+                    T.qa[slot] = make_int2((int)(rec[j].cp & 0xffffffu) * OG_NAC + jl, (int)(at[j].ty | (rec[j].m8 << 24)));
+                }
+            }
+            qn += __builtin_amdgcn_readlane(sum, G - 1);
+            base += G * OG_NAC;
+            parity ^= 1;
+            // the next batch's atoms and the records after them load while this batch's passes run
+#pragma unroll
+            for (int j = 0; j < NG; j++) {
+                rec[j]  = rec1[j];
+                at[j]   = og_load_atom(L, rec[j].cp);
+                rec1[j] = og_load_rec(L, base + OG_NAC * (G + j * OG_TEAM + w), p1);
+            }
+        }
+        // a pass per wave at a time: wave w evaluates pass q + w, then sums its atoms over the passes in order
+        const bool last = base >= p1;
+        const int  np   = last ? (qn + 63) >> 6 : qn >> 6;
+        for (int q = 0; q < np; q += OG_TEAM) {
+            og_lds_barrier();  // the queue is written, the last passes' coefficients are read
+            const int p = q + w;
+            if (p < np) {
+                const int  cnt  = min(qn - 64 * p, 64);
+                const bool live = lane < cnt;
+                og_f4      pj   = T.qp[64 * p + lane];
+                const int2 ax   = T.qa[64 * p + lane];
+                unsigned   m8 = (unsigned)ax.y >> 24, tj = (unsigned)ax.y & 0xffffffu;
+                if (cnt < 64) {  // idle lanes: finite coordinates, LJ column 0, every pair masked
+                    if (!live) pj = og_f4{0.0f, 0.0f, 0.0f, 0.0f};
+                    m8 = live ? m8 : 0xffu;
+                    tj = live ? tj : 0u;
+                }
+                float    g[OG_NAC];
+                og_chain ch;
+                og_rows<FORM, ENERGY, LJ_LDS, true>(s, c, pj, tj, m8, ljl, LJP, g, npair, ch);
+#pragma unroll
+                for (int i = 0; i < OG_NAC; i++) T.coef[w][i][lane] = g[i];
+                if (ENERGY) T.en[w][0][lane] = ch.e, T.en[w][1][lane] = ch.q, T.en[w][2][lane] = ch.v;
+                og_range(ch, vmax, vsum);
+                og_jpend pend{ch.x, ch.y, ch.z, ax.x, live};
+                og_flush_j(FXJ, FXZ, pend);
+            }
+            og_lds_barrier();
+            // the passes' rows and coefficients load together; a pass past the last adds coefficient 0
+            og_f4 pj[OG_TEAM];
+            float g[OG_TEAM][NI];
+#pragma unroll
+            for (int k = 0; k < OG_TEAM; k++) {
+                const bool in = lane < qn - 64 * (q + k) && q + k < np;
+                pj[k] = T.qp[64 * min(q + k, np - 1) + lane];
+                if (!in) pj[k] = og_f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int i = 0; i < NI; i++) {
+                    const float v = T.coef[k][i0 + i][lane];
+                    g[k][i]       = in ? v : 0.0f;
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < OG_TEAM; k++)
+#pragma unroll
+                for (int i = 0; i < NI; i++) {
+                    fi[3 * i]     = fmaf(g[k][i], xi[i] - pj[k].x, fi[3 * i]);
+                    fi[3 * i + 1] = fmaf(g[k][i], yi[i] - pj[k].y, fi[3 * i + 1]);
+                    fi[3 * i + 2] = fmaf(g[k][i], zi[i] - pj[k].z, fi[3 * i + 2]);
+                }
+            if (ENERGY && w < 3) {
+                float e[OG_TEAM];
+#pragma unroll
+                for (int k = 0; k < OG_TEAM; k++) e[k] = T.en[k][w][lane];
+#pragma unroll
+                for (int k = 0; k < OG_TEAM; k++) en += q + k < np ? (double)e[k] : 0.0;
+            }
+        }
+        if (last) break;
+        // the rows short of a pass lead the next batch's queue (its rows are written after another barrier)
+        const int rem = qn - 64 * np;
+        if (np > 0) {
+            og_lds_barrier();
+            if (w == 0 && lane < rem) {
+                const og_f4 mp = T.qp[64 * np + lane];
+                const int2  ma = T.qa[64 * np + lane];
+                T.qp[lane]     = mp;
+                T.qa[lane]     = ma;
+            }
+        }
+        qn = rem;
+    }
+    // i-gradients: sums over the wave in the order of the one-wave reduction, lanes 0-31 and 32-63 an atom each
+    static_assert(NI == 2, "two atoms per wave");
+    float h3[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        float v = og_fold32(fi[k], fi[3 + k]);
+        v       = og_fold16(v, v);
+        h3[k]   = og_dpp_sum8(v + og_dpp<0x128>(v));
+    }
+    if (!(vmax <= OG_FXJ_ROW_LIMIT) || !(fabsf(vsum) < INFINITY)) atomicOr(&s.cnt->flags, OG_F_NAN);
+    if ((lane & 31) == 0) {
+        const int a1 = c1 * OG_NAC + i0 + (lane >> 5);
+        if (!(fabsf(h3[0]) + fabsf(h3[1]) + fabsf(h3[2]) <= (float)OG_FX_LIMIT)) atomicOr(&s.cnt->flags, OG_F_NAN);
+        og_add_fx3(FX, cap, og_fx_slot(a1), (double)h3[0], (double)h3[1], (double)h3[2]);
+    }
+    if (!ENERGY) return;
+    if (w < 3) og_cell_energy(s, c1, OG_EACC_VDW + w, en, w == 0 && FORM != 2 ? -1.0 / 12.0 : 1.0);
+    if (lane == 0)
+        og_atomic_add_fx_g((OG_GLOBAL(long long) *)s.e_acc + (c1 % OG_EACC_SLOTS) * OG_EACC_STRIDE + OG_EACC_PAIRS,
+                           (long long)npair);
+}
+
+// One work unit per block; the map lists units (one per block).
+template <int FORM>
+__global__ void __launch_bounds__(64 * OG_TEAM) k_pair_team(const og_dev_sys *__restrict__ S,
+                                                           const int2 *__restrict__ map) {
+    typedef typename og_ljt<FORM>::type ljt;
+    __shared__ og_team T;
+    __shared__ ljt     ljl[OG_LJ_LDS_ENTRIES(FORM)];
+    const int2        bm = map ? map[blockIdx.x] : make_int2(0, (int)blockIdx.x);
+    const og_dev_sys &s  = S[bm.x];
+    const og_unit     un = og_unit_start(s, bm.y);
+    const int rows = og_pair_tables<FORM, 64 * OG_TEAM>(s, T.shift, ljl);
+    og_lds_barrier();
+    if (!un.run) return;  // block-uniform
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (un.energy) {
+        if (__all(un.ty < rows)) og_team_cell<FORM, true, true>(s, un, w, T, ljl);
+        else og_team_cell<FORM, true, false>(s, un, w, T, ljl);
+    } else {
+        if (__all(un.ty < rows)) og_team_cell<FORM, false, true>(s, un, w, T, ljl);
+        else og_team_cell<FORM, false, false>(s, un, w, T, ljl);
+    }
 }
 
 // Per atom: fixed-point pair gradient -> FP64 "work" with the atom's
@@ -610,6 +899,20 @@ void og_launch_pair(const og_launch &a, int form, int waves) {
     case OG_FORM_ZM_ALPHA: og_launch_pair_form<4>(a, waves); break;
     case OG_FORM_ZD_ALPHA: og_launch_pair_form<1>(a, waves); break;
     default: og_launch_pair_form<0>(a, waves); break;
+    }
+}
+
+template <int FORM>
+static void og_launch_team_form(const og_launch &a) {
+    hipLaunchKernelGGL((k_pair_team<FORM>), dim3(a.n_blocks), dim3(64 * OG_TEAM), 0, a.stream, a.sys, a.map);
+}
+void og_launch_pair_team(const og_launch &a, int form) {
+    switch (form) {
+    case OG_FORM_HPS_DH: og_launch_team_form<2>(a); break;
+    case OG_FORM_ZM: og_launch_team_form<3>(a); break;
+    case OG_FORM_ZM_ALPHA: og_launch_team_form<4>(a); break;
+    case OG_FORM_ZD_ALPHA: og_launch_team_form<1>(a); break;
+    default: og_launch_team_form<0>(a); break;
     }
 }
 void og_launch_forces_to_work(const og_launch &a) {
