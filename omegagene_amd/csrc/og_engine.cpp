@@ -252,13 +252,16 @@ struct og_system {
     long long           step_end      = OG_NO_STEP_END;  // host mirror of og_dev_counters::step_end
     struct og_exec     *ctx = nullptr;   // private batch-of-one
     uint64_t            dev_bytes = 0;   // device memory allocated for the system
+    void               *pt_host = nullptr;  // pinned: a single-point call's og_point_out, then its gradient
+    size_t              pt_bytes = 0;       // bytes of it
     og_status           status = OG_OK;  // outcome of the system's last run or evaluation
 };
 
 struct og_exec {
     std::vector<og_system *> members;
     og_dev_sys              *d_sys = nullptr;
-    int2                    *d_map[KIND_N]{};
+    int2                    *d_maps = nullptr;  // the block maps, one after the other
+    int2                    *d_map[KIND_N]{};   // each kind's part of them
     int                      n_blocks[KIND_N]{};
     hipStream_t              stream = nullptr;
     bool                     dirty  = true;
@@ -291,8 +294,7 @@ og_status exec_release(og_exec &x) {
     free_graphs(x);
     for (auto &e : x.ev) hipEventDestroy(e);
     x.ev.clear();
-    for (int k = 0; k < KIND_N; k++)
-        if (x.d_map[k]) hipFree(x.d_map[k]), x.d_map[k] = nullptr;
+    if (x.d_maps) hipFree(x.d_maps), x.d_maps = nullptr;
     if (x.d_sys) hipFree(x.d_sys), x.d_sys = nullptr;
     if (x.stream) hipStreamDestroy(x.stream), x.stream = nullptr;
     return OG_OK;
@@ -304,8 +306,7 @@ og_status exec_prepare(og_exec &x) {
     free_graphs(x);
     if (!x.stream) OG_HIP(hipStreamCreateWithFlags(&x.stream, hipStreamNonBlocking));
     if (x.d_sys) hipFree(x.d_sys), x.d_sys = nullptr;
-    for (int k = 0; k < KIND_N; k++)
-        if (x.d_map[k]) hipFree(x.d_map[k]), x.d_map[k] = nullptr;
+    if (x.d_maps) hipFree(x.d_maps), x.d_maps = nullptr;
     const int ns = (int)x.members.size();
     if (ns == 0) {
         x.dirty = false;
@@ -420,13 +421,18 @@ og_status exec_prepare(og_exec &x) {
     }
     OG_HIP(hipMalloc((void **)&x.d_sys, sizeof(og_dev_sys) * ns));
     OG_HIP(hipMemcpy(x.d_sys, hs.data(), sizeof(og_dev_sys) * ns, hipMemcpyHostToDevice));
+    std::vector<int2> all;
     for (int k = 0; k < KIND_N; k++) {
         x.n_blocks[k] = (int)maps[k].size();
-        if (x.n_blocks[k]) {
-            OG_HIP(hipMalloc((void **)&x.d_map[k], sizeof(int2) * maps[k].size()));
-            OG_HIP(hipMemcpy(x.d_map[k], maps[k].data(), sizeof(int2) * maps[k].size(), hipMemcpyHostToDevice));
-        }
+        all.insert(all.end(), maps[k].begin(), maps[k].end());
     }
+    // one allocation and one copy for all maps: 30 of each were most of a new context's first call
+    if (!all.empty()) {
+        OG_HIP(hipMalloc((void **)&x.d_maps, sizeof(int2) * all.size()));
+        OG_HIP(hipMemcpy(x.d_maps, all.data(), sizeof(int2) * all.size(), hipMemcpyHostToDevice));
+    }
+    int2 *at = x.d_maps;
+    for (int k = 0; k < KIND_N; at += x.n_blocks[k++]) x.d_map[k] = at;
     x.dirty = false;
     return OG_OK;
 }
@@ -453,9 +459,8 @@ void launch_pair(const og_exec &x, int shape) {
     else og_launch_pair(a, x.pair_form, 1 << (shape & 3));
 }
 
-// reduce: reduce the energies now (a single-point call); an MD step reduces
-// them in its closing kernel instead
-void enqueue_forces(og_exec &x, hipEvent_t e0, hipEvent_t e1, bool reduce = false) {
+// point: a single-point call, which always takes the gradient
+void enqueue_forces(og_exec &x, hipEvent_t e0, hipEvent_t e1, bool point = false) {
     if (e0) hipEventRecord(e0, x.stream);
     launch_pair(x, x.pair_shape);
     if (e1) hipEventRecord(e1, x.stream);
@@ -463,8 +468,7 @@ void enqueue_forces(og_exec &x, hipEvent_t e0, hipEvent_t e1, bool reduce = fals
     // the fused step kernel)
     if (x.any_bonded) og_launch_bonded(L(x, KIND_BTERM));
     // an MD step of a fused context converts the gradient inside its step kernel
-    if (reduce || !x.fused) og_launch_forces_to_work(L(x, KIND_ATOM));
-    if (reduce) og_launch_energy_reduce(L(x, KIND_SYS));
+    if (point || !x.fused) og_launch_forces_to_work(L(x, KIND_ATOM));
 }
 
 void enqueue_integrate(og_exec &x) {
@@ -494,6 +498,13 @@ void enqueue_integrate(og_exec &x) {
     og_launch_finish(L(x, KIND_ATOM));
     og_launch_step_close(L(x, KIND_SYS));
 }
+
+// Most bytes a single-point call returns through pinned memory of the system
+// (its kernel writes them, the host copies them on); a larger gradient is
+// copied from the device.  Pinned / copied, us per call: 960 atoms 91 / 99,
+// 4,230 116 / 126, 12,000 130 / 138, 25,041 158 / 165, 99,200 433 / 443; but
+// pinning costs the first call 0.2 ms up to 300 KB and 0.9 ms at 2.4 MB.
+constexpr size_t OG_POINT_PINNED = 512 << 10;
 
 // Ask for a grid rebuild of this system before its next step whatever its
 // phase (a new system, new coordinates, an explicit rebuild); the step's
@@ -549,40 +560,48 @@ og_status get_graph(og_exec &x, const std::string &pattern, hipGraphExec_t *out)
 // faulted member stands still on the device (og_frozen); its sticky state is
 // cleared here so it can be run again once the caller has acted on the
 // error, and its grid is rebuilt first.  Returns the first member's error.
+og_status check_flags(og_system *s, const og_dev_counters &c) {
+    s->host_step = c.step;
+    og_status st = OG_OK;
+    char      msg[256];
+    if (c.flags & (OG_F_CP_OVERFLOW | OG_F_CELL_OVERFLOW | OG_F_COL_OVERFLOW)) {
+        st = OG_E_CAPACITY;
+        snprintf(msg, sizeof msg, "device list overflow (flags 0x%x): cells %d, cell pairs cap %d", c.flags,
+                 c.n_cells, s->h.cap_cell_pairs);
+    } else if (c.flags & OG_F_NAN) {
+        st = OG_E_NAN;
+        snprintf(msg, sizeof msg, "non-finite coordinate or force (flags 0x%x) at step %lld", c.flags, c.step);
+    } else if (c.shake_fail) {
+        st = OG_E_NOCONV;
+        snprintf(msg, sizeof msg, "SHAKE did not converge for %d constraint groups", c.shake_fail);
+    }
+    s->status = st;
+    // the device flags are sticky: clear them once reported
+    if (c.flags & ~OG_F_OUTSIDE_BOX) OG_HIP(hipMemset(&s->d_cnt->flags, 0, sizeof(int)));
+    if (c.shake_fail) OG_HIP(hipMemset(&s->d_cnt->shake_fail, 0, sizeof(int)));
+    if (st == OG_E_CAPACITY || st == OG_E_NAN) {
+        // a step stopped part-way: drop its partial sums, rebuild before the next one
+        OG_HIP(hipMemset(s->h.fx, 0, sizeof(long long) * OG_FX_WORDS(s->h.cap_atom_array)));
+        OG_HIP(hipMemset(s->h.e_acc, 0, sizeof(long long) * OG_EACC_SLOTS * OG_EACC_STRIDE));
+        s->grid_valid = false;
+    }
+    if (st != OG_OK) set_err("%s", msg);
+    return st;
+}
+
 og_status check_flags(og_exec &x) {
     og_status first = OG_OK;
+    std::string err;
     for (og_system *s : x.members) {
         og_dev_counters c;
         OG_HIP(hipMemcpy(&c, s->d_cnt, sizeof c, hipMemcpyDeviceToHost));
-        s->host_step = c.step;
-        og_status st = OG_OK;
-        char      msg[256];
-        if (c.flags & (OG_F_CP_OVERFLOW | OG_F_CELL_OVERFLOW | OG_F_COL_OVERFLOW)) {
-            st = OG_E_CAPACITY;
-            snprintf(msg, sizeof msg, "device list overflow (flags 0x%x): cells %d, cell pairs cap %d", c.flags,
-                     c.n_cells, s->h.cap_cell_pairs);
-        } else if (c.flags & OG_F_NAN) {
-            st = OG_E_NAN;
-            snprintf(msg, sizeof msg, "non-finite coordinate or force (flags 0x%x) at step %lld", c.flags, c.step);
-        } else if (c.shake_fail) {
-            st = OG_E_NOCONV;
-            snprintf(msg, sizeof msg, "SHAKE did not converge for %d constraint groups", c.shake_fail);
-        }
-        s->status = st;
-        // the device flags are sticky: clear them once reported
-        if (c.flags & ~OG_F_OUTSIDE_BOX) OG_HIP(hipMemset(&s->d_cnt->flags, 0, sizeof(int)));
-        if (c.shake_fail) OG_HIP(hipMemset(&s->d_cnt->shake_fail, 0, sizeof(int)));
-        if (st == OG_E_CAPACITY || st == OG_E_NAN) {
-            // a step stopped part-way: drop its partial sums, rebuild before the next one
-            OG_HIP(hipMemset(s->h.fx, 0, sizeof(long long) * OG_FX_WORDS(s->h.cap_atom_array)));
-            OG_HIP(hipMemset(s->h.e_acc, 0, sizeof(long long) * OG_EACC_SLOTS * OG_EACC_STRIDE));
-            s->grid_valid = false;
-        }
+        const og_status st = check_flags(s, c);
         if (st != OG_OK && first == OG_OK) {
             first = st;
-            set_err("%s", msg);
+            err   = g_last_error;
         }
     }
+    if (first != OG_OK) g_last_error = err;
     return first;
 }
 
@@ -1531,6 +1550,7 @@ og_status og_system_destroy(og_system *s) {
         delete s->ctx;
     }
     for (void *p : s->allocs) hipFree(p);
+    if (s->pt_host) hipHostFree(s->pt_host);
     delete s;
     return OG_OK;
 }
@@ -1554,26 +1574,31 @@ og_status og_calc_energy_force(og_system *s, int rebuild, double *work_atom, dou
     og_status st = ensure_ctx(s);
     if (st != OG_OK) return st;
     og_exec &x = *s->ctx;
+    const size_t nw = sizeof(double) * 3 * (size_t)s->h.n_atoms, need = sizeof(og_point_out) + (work_atom ? nw : 0);
+    const bool   pinned = need <= OG_POINT_PINNED;  // the gradient too, otherwise the status alone
+    if (s->pt_bytes < (pinned ? need : sizeof(og_point_out))) {
+        if (s->pt_host) hipHostFree(s->pt_host);
+        s->pt_host = nullptr, s->pt_bytes = 0;
+        OG_HIP(hipHostMalloc(&s->pt_host, pinned ? need : sizeof(og_point_out), hipHostMallocDefault));
+        s->pt_bytes = pinned ? need : sizeof(og_point_out);
+    }
+    og_point_out *out   = (og_point_out *)s->pt_host;
+    double       *wpin  = pinned && work_atom ? (double *)(out + 1) : nullptr;
+    const bool    fresh = rebuild || !s->grid_valid;
     // a single-point evaluation always carries its energies
-    const int one = 1, zero = 0;
-    OG_HIP(hipMemcpy(&s->d_cnt->force_energy, &one, sizeof(int), hipMemcpyHostToDevice));
-    if (rebuild || !s->grid_valid) {
-        st = request_rebuild(s);  // cleared by the energy reduction
-        if (st != OG_OK) return st;
-        enqueue_rebuild(x);
-    }
+    og_launch_point_begin(s->d_cnt, fresh, x.stream);
+    if (fresh) enqueue_rebuild(x);
     enqueue_forces(x, nullptr, nullptr, true);
+    og_launch_point_end(L(x, KIND_SYS), out, wpin, s->h.n_atoms);
+    OG_HIP(hipGetLastError());
     OG_HIP(hipStreamSynchronize(x.stream));
-    OG_HIP(hipMemcpy(&s->d_cnt->force_energy, &zero, sizeof(int), hipMemcpyHostToDevice));
     s->grid_valid = true;
-    st            = check_flags(x);
+    st            = check_flags(s, out->cnt);
     if (st != OG_OK) return st;
-    if (work_atom) OG_HIP(hipMemcpy(work_atom, s->h.work, sizeof(double) * 3 * s->h.n_atoms, hipMemcpyDeviceToHost));
-    if (energies) {
-        double e[OG_E_NTERMS];
-        OG_HIP(hipMemcpy(e, s->h.energy, sizeof e, hipMemcpyDeviceToHost));
-        for (int k = 0; k < OG_NTERMS; k++) energies[k] = e[k];
-    }
+    if (wpin) std::memcpy(work_atom, wpin, nw);
+    else if (work_atom) OG_HIP(hipMemcpy(work_atom, s->h.work, nw, hipMemcpyDeviceToHost));
+    if (energies)
+        for (int k = 0; k < OG_NTERMS; k++) energies[k] = out->energy[k];
     return OG_OK;
 }
 

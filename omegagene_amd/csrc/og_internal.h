@@ -509,6 +509,13 @@ constexpr long long OG_TEAM_CELLS = 900;
 void og_launch_pair_team(const og_launch &units, int form);
 void og_launch_forces_to_work(const og_launch &atoms);
 void og_launch_energy_reduce(const og_launch &sys);
+// a single-point evaluation of one system: its requests, and its outcome to pinned host memory
+struct alignas(16) og_point_out {
+    og_dev_counters cnt;
+    double          energy[OG_E_NTERMS];
+};
+void og_launch_point_begin(og_dev_counters *cnt, int rebuild, hipStream_t stream);
+void og_launch_point_end(const og_launch &sys, og_point_out *out, double *work, int n_atoms);
 // integration
 void og_launch_leapfrog_vel(const og_launch &atoms);
 void og_launch_com_sum(const og_launch &sys);
