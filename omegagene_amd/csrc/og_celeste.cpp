@@ -264,8 +264,6 @@ int og_alloc_atom_info(int max_n_atoms_exbox, int max_n_cells, int max_n_cell_pa
     CS_TRY(cs_alloc(&h.comp, max_n_atoms_exbox));
     CS_TRY(cs_alloc(&h.head_cell, (size_t)n_columns + 1));
     CS_TRY(cs_alloc(&h.n_cells_z, (size_t)n_columns + 1));
-    CS_TRY(cs_alloc(&h.n_atoms_col, (size_t)n_columns + 1));
-    CS_TRY(cs_alloc(&h.col_fill, (size_t)n_columns + 1));
     CS_TRY(cs_alloc(&h.cell_col, h.cap_cells));
     CS_TRY(cs_alloc(&h.cell_z, h.cap_cells));
     CS_TRY(cs_alloc(&h.cell_zmin, h.cap_cells));
@@ -275,6 +273,7 @@ int og_alloc_atom_info(int max_n_atoms_exbox, int max_n_cells, int max_n_cell_pa
     CS_TRY(cs_alloc(&h.cp_count, (size_t)h.cap_cells + 1));
     CS_TRY(cs_alloc(&h.cp_stage, (size_t)h.cap_cells * OG_ENUM_STAGE));
     CS_TRY(cs_alloc(&h.cp_head, (size_t)h.cap_cells + 1));
+    CS_TRY(cs_alloc(&h.cp_bsum, (size_t)h.cap_cells / 1024 + 1));
     CS_TRY(cs_alloc(&h.cp_c2, max_n_cell_pairs));
     CS_TRY(cs_alloc(&h.cp_mask, max_n_cell_pairs));
     CS_TRY(cs_alloc(&h.fx, OG_FX_WORDS(cap)));
@@ -595,12 +594,11 @@ int og_enumerate_cell_pairs(int **h_atomids, int n_cells, int n_neighbor_col, co
     c.n_cells  = n_cells;
     c.step_end = OG_NO_STEP_END;
     CS_HIP(hipMemcpy(g_cs.d_cnt, &c, sizeof c, hipMemcpyHostToDevice));
-    og_launch_grid_clear(cs_launch(g_cs.map_slot, g_cs.nb_slot), cs_launch(g_cs.map_slot, g_cs.nb_slot));
+    og_launch_grid_clear(cs_launch(g_cs.map_slot, g_cs.nb_slot));
     og_launch_cells_from_grid(cs_launch(g_cs.map_col, g_cs.nb_col));
     og_launch_enum_count(cs_launch(g_cs.map_cellw, g_cs.nb_cellw));
-    og_launch_enum_scan(cs_launch(g_cs.map_sys, 1));
-    og_launch_enum_write(cs_launch(g_cs.map_cellw, g_cs.nb_cellw));
-    og_launch_masks(cs_launch(g_cs.map_cellw, g_cs.nb_cellw));
+    og_launch_enum_scan(cs_launch(nullptr, g_cs.n_cells / 1024 + 1));
+    og_launch_list(cs_launch(g_cs.map_cellw, g_cs.nb_cellw));
     CS_HIP(hipGetLastError());
     CS_HIP(hipStreamSynchronize(g_cs.stream));
     CS_HIP(hipMemcpy(&c, g_cs.d_cnt, sizeof c, hipMemcpyDeviceToHost));

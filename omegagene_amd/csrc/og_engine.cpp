@@ -221,7 +221,7 @@ og_status wrap_inbox(const GridGeom &g, int n, double *crd) {
 void og_set_error(const char *msg) { g_last_error = msg; }
 
 // ----------------------------------------------------------------- types --
-enum { KIND_ATOM = 0, KIND_SLOT, KIND_CELLW, KIND_COL, KIND_SYS, KIND_MISC, KIND_TRIO, KIND_COMA, KIND_LSTEP,
+enum { KIND_ATOM = 0, KIND_CELLW, KIND_COL, KIND_SYS, KIND_MISC, KIND_TRIO, KIND_COMA, KIND_LSTEP,
        KIND_BTERM,  // OG_THREADS threads per block over the bonded terms (angles, torsions, impropers, 1-4)
        KIND_QUAD,   // OG_QUAD_THREADS threads per block over the four-atom SHAKE groups
        KIND_SCANB,  // blocks of 1024 cells over cap_cells + 1 (multi-block offset scan)
@@ -344,10 +344,8 @@ og_status exec_prepare(og_exec &x) {
         x.any_quad |= d.constraint != 0 && d.n_quads > 0;
         x.fused &= d.integrator == 1 && d.n_water_blocks > 0;
         x.cells += cdiv(d.n_atoms, OG_NAC);
-        const int n_bins = (d.n_columns + 1) * d.n_uni_z;
         int       cnt[KIND_N];
         cnt[KIND_ATOM]  = cdiv(d.n_atoms, OG_THREADS);
-        cnt[KIND_SLOT]  = cdiv(std::max(d.n_columns, n_bins), OG_THREADS);
         cnt[KIND_CELLW] = cdiv(d.cap_cells, OG_THREADS / 64);
         cnt[KIND_COL]   = d.n_columns;
         cnt[KIND_SYS]   = 1;
@@ -440,15 +438,13 @@ og_status exec_prepare(og_exec &x) {
 og_launch L(const og_exec &x, int kind) { return og_launch{x.d_sys, x.d_map[kind], x.n_blocks[kind], x.stream}; }
 
 void enqueue_rebuild(og_exec &x) {
-    og_launch_grid_clear(L(x, KIND_SLOT), L(x, KIND_SLOT));
     og_launch_grid_bin(L(x, KIND_ATOM));
     og_launch_grid_scan(L(x, KIND_SYS));
     og_launch_grid_scatter(L(x, KIND_ATOM));
     og_launch_grid_sort(L(x, KIND_COL));
     og_launch_enum_count(L(x, KIND_CELLW));
-    og_launch_enum_scan_blocks(L(x, KIND_SCANB));
-    og_launch_enum_write(L(x, KIND_CELLW));
-    og_launch_masks(L(x, KIND_CELLW));
+    og_launch_enum_scan(L(x, KIND_SCANB));
+    og_launch_list(L(x, KIND_CELLW));
 }
 
 void launch_pair(const og_exec &x, int shape) {
@@ -583,6 +579,7 @@ og_status check_flags(og_system *s, const og_dev_counters &c) {
         // a step stopped part-way: drop its partial sums, rebuild before the next one
         OG_HIP(hipMemset(s->h.fx, 0, sizeof(long long) * OG_FX_WORDS(s->h.cap_atom_array)));
         OG_HIP(hipMemset(s->h.e_acc, 0, sizeof(long long) * OG_EACC_SLOTS * OG_EACC_STRIDE));
+        OG_HIP(hipMemset(s->h.n_atoms_col, 0, sizeof(int) * s->h.n_columns));
         s->grid_valid = false;
     }
     if (st != OG_OK) set_err("%s", msg);

@@ -9,22 +9,22 @@
 #include "og_internal.h"
 
 // ---------------------------------------------------------------- clear --
-// Zero per-column counters and the uniform-z bin table of each system.
+// Empties thread t's share (every n-th) of the uniform-z bin table.
+__device__ __forceinline__ void og_clear_bins(const og_dev_sys &s, const int t, const int n) {
+    const int n_bins = (s.n_columns + 1) * s.n_uni_z;
+    for (int k = t; k < n_bins; k += n) {
+        s.u2c_min[k] = OG_EMPTY_BIN;
+        s.u2c_max[k] = -1;
+    }
+}
+// The bin table of the reference call points (an engine's rebuild empties it
+// in k_grid_bin).
 __global__ void __launch_bounds__(OG_THREADS) k_grid_clear(const og_dev_sys *__restrict__ S,
                                                            const int2 *__restrict__ map) {
     const int2        bm = map[blockIdx.x];
     const og_dev_sys &s  = S[bm.x];
     if (og_rebuild_skip(s)) return;
-    const int         t  = bm.y * OG_THREADS + threadIdx.x;
-    if (t < s.n_columns) {
-        s.n_atoms_col[t] = 0;
-        s.col_fill[t]    = 0;
-    }
-    const int n_bins = (s.n_columns + 1) * s.n_uni_z;
-    if (t < n_bins) {
-        s.u2c_min[t] = OG_EMPTY_BIN;
-        s.u2c_max[t] = -1;
-    }
+    og_clear_bins(s, blockIdx.x * OG_THREADS + threadIdx.x, gridDim.x * OG_THREADS);
     // overflow flags stay set until the host has read them (check_flags), so a
     // failed rebuild inside a multi-step graph is never hidden by a later one
 }
@@ -37,22 +37,27 @@ __global__ void __launch_bounds__(OG_THREADS) k_grid_clear(const og_dev_sys *__r
 // (atoms in input order are mostly spatial neighbours, so a wave touches a
 // few columns).  Returns the old counter value plus the lane's rank among
 // the lanes of its key, i.e. what a per-lane atomicAdd(ctr + key, 1) could
-// have returned.
+// have returned.  The keys' atomics go out together: one after the other, a
+// wave of chain atoms (ten columns) waited ten round trips (the scatter of
+// 4,230 atoms 10.5 us, now 4.1).
 __device__ __forceinline__ int og_wave_count_add(int *ctr, int key, bool active) {
-    const int lane = threadIdx.x & 63;
-    uint64_t  todo = __ballot(active);
-    int       res  = 0;
+    const int lane   = threadIdx.x & 63;
+    uint64_t  todo   = __ballot(active);
+    int       leader = lane, rank = 0, count = 0;
     while (todo) {
-        const int      leader = __builtin_ctzll(todo);
-        const int      lkey   = __builtin_amdgcn_readlane(key, leader);
-        const uint64_t m      = __ballot(active && key == lkey) & todo;
-        int            base   = 0;
-        if (lane == leader) base = atomicAdd(ctr + lkey, __builtin_popcountll(m));
-        base = __builtin_amdgcn_readlane(base, leader);
-        if ((m >> lane) & 1ull) res = base + __builtin_popcountll(m & ((1ull << lane) - 1ull));
+        const int      l    = __builtin_ctzll(todo);
+        const int      lkey = __builtin_amdgcn_readlane(key, l);
+        const uint64_t m    = __ballot(active && key == lkey) & todo;
+        if ((m >> lane) & 1ull) {
+            leader = l;
+            rank   = __builtin_popcountll(m & ((1ull << lane) - 1ull));
+            count  = __builtin_popcountll(m);
+        }
         todo &= ~m;
     }
-    return res;
+    int base = 0;
+    if (active && leader == lane) base = atomicAdd(ctr + key, count);
+    return __shfl(base, leader, 64) + rank;
 }
 
 __global__ void __launch_bounds__(OG_THREADS) k_grid_bin(const og_dev_sys *__restrict__ S,
@@ -62,6 +67,7 @@ __global__ void __launch_bounds__(OG_THREADS) k_grid_bin(const og_dev_sys *__res
     if (og_rebuild_skip(s)) return;
     const int         i  = bm.y * OG_THREADS + threadIdx.x;
     const bool        in = i < s.n_atoms;
+    og_clear_bins(s, i, s.n_atom_blocks * OG_THREADS);  // read by the last rebuild only, filled by the sort
     int  c[2] = {0, 0};
     bool bad = false;
     if (in) {
@@ -165,8 +171,6 @@ __global__ void __launch_bounds__(OG_THREADS) k_grid_scatter(const og_dev_sys *_
     if (in) s.tmp_ids[s.head_atom[col] + slot] = i;
 }
 
-__device__ void og_column_cells(const og_dev_sys &s, int col, int nz);
-
 // ----------------------------------------------------------------- sort --
 // One block per column.  Ascending float z with the atom id as tie-break
 // (the reference Hoare quicksort, MiniCell.cpp:636-691, orders distinct z
@@ -175,20 +179,79 @@ __device__ void og_column_cells(const og_dev_sys &s, int col, int nz);
 // (MiniCell.cpp:574-580), grid-order coordinates rounded through float
 // (MiniCell.cpp:414-415), cell z extents and uniform-z bins
 // (MiniCell.cpp:884-936).
-__global__ void __launch_bounds__(OG_THREADS) k_grid_sort(const og_dev_sys *__restrict__ S,
+//
+// A column of at most a block's threads (any at liquid density in a box below
+// 150 A) has an atom per thread: it loads its atom while it counts the smaller
+// keys (its place), and leaves its z in LDS for the cells.  A longer column is
+// sorted in LDS by a bitonic network.  The kernel is a chain of memory round
+// trips; the count takes 3 cycles per key and wave against the network's 28
+// barriers for 128 atoms (4,230 atoms 10.0 -> 6.2 us).
+struct og_slot_atom {
+    float x, y, z, q;
+    int   type, comp;
+};
+__device__ __forceinline__ og_slot_atom og_load_slot_atom(const og_dev_sys &s, const int id) {
+    return og_slot_atom{(float)s.crd[3 * id], (float)s.crd[3 * id + 1], (float)s.crd[3 * id + 2],
+                        s.charge[id], s.atom_type[id], s.comp[id]};
+}
+// id < 0: a dummy at atom a's place
+__device__ __forceinline__ void og_store_slot(const og_dev_sys &s, const int slot, const int id,
+                                              const og_slot_atom &a) {
+    s.atomids[slot]      = id;
+    s.gcrd[3 * slot]     = (double)a.x;
+    s.gcrd[3 * slot + 1] = (double)a.y;
+    s.gcrd[3 * slot + 2] = (double)a.z;
+    s.gxyzq[slot]        = make_float4(a.x, a.y, a.z, id >= 0 ? a.q : 0.0f);
+    s.gtype[slot]        = id >= 0 ? a.type : 0;
+    s.gcomp[slot]        = id >= 0 ? a.comp : -1;
+    if (id >= 0) s.rev[id] = slot;
+}
+
+__device__ void og_column_cells(const og_dev_sys &s, int col, int nz, const float *z);
+
+__global__ void __launch_bounds__(OG_THREADS, 8) k_grid_sort(const og_dev_sys *__restrict__ S,
                                                           const int2 *__restrict__ map) {
     const int2        bm  = map[blockIdx.x];
     const og_dev_sys &s   = S[bm.x];
     if (og_rebuild_skip(s)) return;
     const int         col = bm.y;
     __shared__ uint64_t keys[OG_SORT_CAP];
+    __shared__ float    zs[OG_THREADS + OG_NAC];
+    const int n = s.n_atoms_col[col], nz = s.n_cells_z[col], base = s.head_atom[col];
     if (s.cnt->n_cells == 0) return;
-    const int n = s.n_atoms_col[col];
     if (n == 0) return;
-    const int base = s.head_atom[col];
-    int       P    = 1;
+    const int tid = threadIdx.x;
+    if (n <= OG_THREADS) {
+        const int    id = tid < n ? s.tmp_ids[base + tid] : 0;
+        og_slot_atom a{};
+        uint64_t     key = ~0ull;
+        if (tid < n) {
+            key = ((uint64_t)s.zkey[id] << 32) | (uint32_t)id;
+            a   = og_load_slot_atom(s, id);
+        }
+        keys[tid] = key;  // past the column: above every key, as far as the unrolled count reads
+        __syncthreads();
+        if (tid == 0) s.n_atoms_col[col] = 0;  // the next rebuild's binning counts from zero
+        if (tid < n) {
+            int rank = 0;
+            for (int k = 0; k < n; k += 8)
+#pragma unroll
+                for (int j = 0; j < 8; j++) rank += keys[k + j] < key ? 1 : 0;
+            og_store_slot(s, base + rank, id, a);
+            zs[rank] = a.z;
+            if (rank == n - 1)
+                for (int t = n; t < nz * OG_NAC; t++) {
+                    og_store_slot(s, base + t, -1, a);
+                    zs[t] = a.z;
+                }
+        }
+        __syncthreads();
+        og_column_cells(s, col, nz, zs);
+        return;
+    }
+    int P = 1;
     while (P < n) P <<= 1;
-    for (int t = threadIdx.x; t < P; t += blockDim.x) {
+    for (int t = tid; t < P; t += OG_THREADS) {
         if (t < n) {
             const int id = s.tmp_ids[base + t];
             keys[t]      = ((uint64_t)s.zkey[id] << 32) | (uint32_t)id;
@@ -197,9 +260,10 @@ __global__ void __launch_bounds__(OG_THREADS) k_grid_sort(const og_dev_sys *__re
         }
     }
     __syncthreads();
+    if (tid == 0) s.n_atoms_col[col] = 0;
     for (int k = 2; k <= P; k <<= 1) {
         for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int t = threadIdx.x; t < P; t += blockDim.x) {
+            for (int t = tid; t < P; t += OG_THREADS) {
                 const int u = t ^ j;
                 if (u > t) {
                     const uint64_t a = keys[t], b = keys[u];
@@ -213,39 +277,27 @@ __global__ void __launch_bounds__(OG_THREADS) k_grid_sort(const og_dev_sys *__re
             __syncthreads();
         }
     }
-    const int nz    = s.n_cells_z[col];
-    const int last  = (int)(keys[n - 1] & 0xffffffffu);
-    const int cap   = s.cap_atom_array;
-    for (int t = threadIdx.x; t < nz * OG_NAC; t += blockDim.x) {
-        const int slot = base + t;
-        const int id   = t < n ? (int)(keys[t] & 0xffffffffu) : -1;
-        const int src  = t < n ? id : last;
-        const float x = (float)s.crd[3 * src], y = (float)s.crd[3 * src + 1], z = (float)s.crd[3 * src + 2];
-        s.atomids[slot]      = id;
-        s.gcrd[3 * slot]     = (double)x;
-        s.gcrd[3 * slot + 1] = (double)y;
-        s.gcrd[3 * slot + 2] = (double)z;
-        s.gxyzq[slot]        = make_float4(x, y, z, id >= 0 ? s.charge[src] : 0.0f);
-        s.gtype[slot]        = id >= 0 ? s.atom_type[src] : 0;
-        s.gcomp[slot]        = id >= 0 ? s.comp[src] : -1;
-        if (id >= 0) s.rev[id] = slot;
-        (void)cap;
+    const int last = (int)(keys[n - 1] & 0xffffffffu);
+    for (int t = tid; t < nz * OG_NAC; t += OG_THREADS) {
+        const int id = t < n ? (int)(keys[t] & 0xffffffffu) : -1;
+        og_store_slot(s, base + t, id, og_load_slot_atom(s, t < n ? id : last));
     }
     __syncthreads();
-    og_column_cells(s, col, nz);
+    og_column_cells(s, col, nz, nullptr);
 }
 
 // Cells of one grid column from grid-order coordinates: cell -> column and z
 // index, z extents from the first and last slot of each cell (dummies copy
 // the last real atom, so the last slot holds the top), and the uniform-z bins
 // the cell overlaps (MiniCell::set_uniform_grid, MiniCell.cpp:884-936).
-// Called by one block per column after the column's slots are written.
-__device__ void og_column_cells(const og_dev_sys &s, int col, int nz) {
+// Called by one block per column after the column's slots are written; z: the
+// slots' z in LDS, or null.
+__device__ void og_column_cells(const og_dev_sys &s, int col, int nz, const float *z) {
     const int hc = s.head_cell[col];
     for (int c = threadIdx.x; c < nz; c += blockDim.x) {
         const int   cell = hc + c;
-        const float zmin = (float)s.gcrd[3 * (cell * OG_NAC) + 2];
-        const float zmax = (float)s.gcrd[3 * (cell * OG_NAC + OG_NAC - 1) + 2];
+        const float zmin = z ? z[c * OG_NAC] : (float)s.gcrd[3 * (cell * OG_NAC) + 2];
+        const float zmax = z ? z[c * OG_NAC + OG_NAC - 1] : (float)s.gcrd[3 * (cell * OG_NAC + OG_NAC - 1) + 2];
         s.cell_col[cell]  = col;
         s.cell_z[cell]    = c;
         s.cell_zmin[cell] = zmin;
@@ -278,7 +330,7 @@ __global__ void __launch_bounds__(OG_THREADS) k_cells_from_grid(const og_dev_sys
     if (og_rebuild_skip(s)) return;
     const int         col = bm.y;
     if (s.head_cell[col] < 0) return;
-    og_column_cells(s, col, s.n_cells_z[col]);
+    og_column_cells(s, col, s.n_cells_z[col], nullptr);
 }
 
 // ---------------------------------------------------------- enumeration --
@@ -311,10 +363,12 @@ __device__ __forceinline__ float og_zgap2(float z2t, float z2b, float z1b, float
 
 // MODE 1: count the cell's pairs and stage them (cell2 | image << 24, list
 // order) in cp_stage[c1 * OG_ENUM_STAGE ...] as far as they fit;
-// MODE 2: write them at cp_head[c1] (cells whose pairs did not fit).
+// MODE 2: write them at p0 (cells whose pairs did not fit).
+// Bound by its about 900 vector instructions per cell (147 us at 450,000
+// atoms): reading a lane's bins and candidates in batches of eight and four
+// independent loads cost 189 us there.
 template <int MODE>
-__device__ void og_enum_cell(const og_dev_sys &s, int c1, int *out_count) {
-    constexpr bool WRITE = MODE != 0;
+__device__ void og_enum_cell(const og_dev_sys &s, int c1, int p0, int *out_count) {
     const int lane  = threadIdx.x & 63;
     const int col1  = s.cell_col[c1];
     const int x1    = col1 % s.nx, y1 = col1 / s.nx;
@@ -343,7 +397,7 @@ __device__ void og_enum_cell(const og_dev_sys &s, int c1, int *out_count) {
         fz[2] = lz[2] = -1;
         lz[1]         = tl;
     }
-    int carry = MODE == 2 ? s.cp_head[c1] : 0;
+    int carry = MODE == 2 ? p0 : 0;
     int total = 0;
     for (int r0 = 0; r0 < ncand; r0 += 64) {
         const int k     = r0 + lane;
@@ -404,7 +458,7 @@ __device__ void og_enum_cell(const og_dev_sys &s, int c1, int *out_count) {
                 }
                 if (f < 0) continue;
                 // a cell top rounding onto the upper face spills into the next
-                // column's first bin (see k_grid_sort); keep the range in this column
+                // column's first bin (see og_column_cells); keep the range in this column
                 const int zc0 = s.u2c_min[f], zc1 = min(s.u2c_max[l], s.n_cells_z[col2] - 1);
                 if (zc0 > zc1) continue;
                 c2lo[ii] = head2 + zc0;
@@ -429,7 +483,7 @@ __device__ void og_enum_cell(const og_dev_sys &s, int c1, int *out_count) {
             if (lane >= off) incl += v;
         }
         const int round_total = __shfl(incl, 63, 64);
-        if (WRITE && mine) {
+        if (mine) {
             int p = carry + incl - mine;
             for (int ii = 0; ii < 3; ii++) {
                 const float sh = (float)(ii - 1) * s.L[2];
@@ -469,36 +523,15 @@ __global__ void __launch_bounds__(OG_THREADS) k_enum_count(const og_dev_sys *__r
     if (og_rebuild_skip(s)) return;
     const int         c1 = __builtin_amdgcn_readfirstlane(bm.y * (OG_THREADS / 64) + (threadIdx.x >> 6));
     if (c1 >= s.cnt->n_cells) return;
-    og_enum_cell<1>(s, c1, &s.cp_count[c1]);
+    og_enum_cell<1>(s, c1, 0, &s.cp_count[c1]);
 }
 
-__global__ void __launch_bounds__(OG_THREADS) k_enum_write(const og_dev_sys *__restrict__ S,
-                                                           const int2 *__restrict__ map) {
-    const int2        bm = map[blockIdx.x];
-    const og_dev_sys &s  = S[bm.x];
-    if (og_rebuild_skip(s)) return;
-    const int         c1 = __builtin_amdgcn_readfirstlane(bm.y * (OG_THREADS / 64) + (threadIdx.x >> 6));
-    if (c1 >= s.cnt->n_cells) return;
-    const int n = s.cp_count[c1];
-    if (n > OG_ENUM_STAGE) {  // did not fit the stage: enumerate again, writing in place
-        og_enum_cell<2>(s, c1, nullptr);
-        return;
-    }
-    const int  lane = threadIdx.x & 63;
-    const int  p0   = s.cp_head[c1];
-    const int *src  = s.cp_stage + (size_t)c1 * OG_ENUM_STAGE;
-    for (int k = lane; k < n; k += 64)
-        if (p0 + k < s.cap_cell_pairs) s.cp_c2[p0 + k] = src[k];
-}
-
-// Exclusive scan of per-cell pair counts -> cp_head (one 1024-thread block per system).
-// The same scan over many blocks of 1024 cells (a large system has 150 k
-// cells): k_enum_scan_part writes each cell's exclusive prefix within its
-// block and the block total; k_enum_scan_add adds the sum of the earlier
-// blocks' totals, clamps to the list capacity and records the total.
-__global__ void __launch_bounds__(1024) k_enum_scan_part(const og_dev_sys *__restrict__ S,
+// Exclusive scan of the cells' pair counts, blocks of 1024 cells: each cell's
+// prefix within its block to cp_head, the block's total to cp_bsum.  k_list
+// adds the totals of the blocks before a cell's.
+__global__ void __launch_bounds__(1024) k_enum_scan(const og_dev_sys *__restrict__ S,
                                                          const int2 *__restrict__ map) {
-    const int2        bm = map[blockIdx.x];
+    const int2        bm = map ? map[blockIdx.x] : make_int2(0, (int)blockIdx.x);
     const og_dev_sys &s  = S[bm.x];
     if (og_rebuild_skip(s)) return;
     const int n = s.cnt->n_cells;
@@ -516,104 +549,74 @@ __global__ void __launch_bounds__(1024) k_enum_scan_part(const og_dev_sys *__res
     __syncthreads();
     int before = 0;
     for (int q = 0; q < w; q++) before += wsum[q];
-    if (k <= n) s.cp_head[k] = before + incl - v;
+    if (k < n) s.cp_head[k] = before + incl - v;
     if (threadIdx.x == 1023) s.cp_bsum[bm.y] = before + incl;
 }
 
-__global__ void __launch_bounds__(1024) k_enum_scan_add(const og_dev_sys *__restrict__ S,
-                                                        const int2 *__restrict__ map) {
-    const int2        bm = map[blockIdx.x];
-    const og_dev_sys &s  = S[bm.x];
-    if (og_rebuild_skip(s)) return;
-    const int n = s.cnt->n_cells;
-    if (bm.y * 1024 > n) return;
-    const int k    = bm.y * 1024 + threadIdx.x;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    __shared__ long long wsum[16];
-    long long o = 0;
-    for (int q = threadIdx.x; q < bm.y; q += 1024) o += s.cp_bsum[q];
-    for (int off = 32; off > 0; off >>= 1) o += __shfl_xor(o, off, 64);
-    if (lane == 0) wsum[w] = o;
-    __syncthreads();
-    long long offset = 0;
-    for (int q = 0; q < 16; q++) offset += wsum[q];
-    if (k > n) return;
-    const long long p = offset + s.cp_head[k];
-    s.cp_head[k]      = (int)min(p, (long long)s.cap_cell_pairs);
-    if (k == n) {
-        if (p > s.cap_cell_pairs) {
-            atomicOr(&s.cnt->flags, OG_F_CP_OVERFLOW);
-            s.cnt->n_cell_pairs = 0;
-        } else {
-            s.cnt->n_cell_pairs = (int)p;
-        }
-    }
-}
-
-__global__ void __launch_bounds__(1024) k_enum_scan(const og_dev_sys *__restrict__ S, const int2 *__restrict__ map) {
-    const og_dev_sys &s   = S[map[blockIdx.x].x];
-    if (og_rebuild_skip(s)) return;
-    const int         n   = s.cnt->n_cells;
-    const int         T   = blockDim.x;
-    const int         per = (n + T - 1) / T;
-    const int         k0  = threadIdx.x * per, k1 = min(k0 + per, n);
-    const int         lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    __shared__ long long wsum[16];
-    long long local = 0;
-    for (int k = k0; k < k1; k++) local += s.cp_count[k];
-    // inclusive scan within the wave (shuffles), then over the 16 wave totals
-    long long incl = local;
-    for (int off = 1; off < 64; off <<= 1) {
-        const long long v = __shfl_up(incl, off, 64);
-        if (lane >= off) incl += v;
-    }
-    if (lane == 63) wsum[w] = incl;
-    __syncthreads();
-    long long before = 0;
-    for (int q = 0; q < w; q++) before += wsum[q];
-    long long p = before + incl - local;
-    for (int k = k0; k < k1; k++) {
-        s.cp_head[k] = (int)min(p, (long long)s.cap_cell_pairs);
-        p += s.cp_count[k];
-    }
-    if (threadIdx.x == T - 1) {
-        const long long total = before + incl;
-        s.cp_head[n]          = (int)min(total, (long long)s.cap_cell_pairs);
-        if (total > s.cap_cell_pairs) {
-            atomicOr(&s.cnt->flags, OG_F_CP_OVERFLOW);
-            s.cnt->n_cell_pairs = 0;
-        } else {
-            s.cnt->n_cell_pairs = (int)total;
-        }
-    }
-}
-
-// ---------------------------------------------------------------- masks --
+// ----------------------------------------------------------------- list --
+// One wave per cell1: the cell's place in the list (its block prefix and the
+// totals before), its records from the stage, and their masks.
+//
 // MiniCell::set_cell_pair_bitmask (MiniCell.cpp:1198-1237): bit a2*8+a1 set
 // (= skip) for a dummy atom, the lower triangle of a self pair, or an nb15off
-// partner (the partner list read up to its first -1).  One wave per cell1.
+// partner (the partner list read up to its first -1).
 // The exclusion bits are found from the atoms' side: the cell's partner
 // lists are read once (lane = 8 * atom + partner) and each partner's grid
 // slot becomes a (cell2, bit) entry in LDS; each lane then builds the masks
-// of 64 of the cell's pairs from the dummy flags, the self-pair triangle and
-// the entries whose cell2 matches.  Same bits as testing every atom pair.
-__global__ void __launch_bounds__(OG_THREADS) k_masks(const og_dev_sys *__restrict__ S, const int2 *__restrict__ map) {
+// of its share of the cell's pairs from the dummy flags, the self-pair
+// triangle and the entries whose cell2 matches.  Same bits as testing every
+// atom pair.
+//
+// A wave is a chain of memory round trips, so what does not depend on each
+// other is read together: the counts, the first 64 staged records and the
+// cell's atoms; then the records' atoms and the partner lists.  Offsets,
+// records and masks took three kernels of such chains (450,000 atoms 110 us,
+// now 84; 4,230 atoms 15 us and two launches more, now 9).
+__global__ void __launch_bounds__(OG_THREADS, 8) k_list(const og_dev_sys *__restrict__ S, const int2 *__restrict__ map) {
     __shared__ int exq[OG_THREADS / 64][OG_NAC * OG_MAX_NB15];  // (cell2 << 6) | bit, per wave
     const int2        bm = map[blockIdx.x];
     const og_dev_sys &s  = S[bm.x];
     if (og_rebuild_skip(s)) return;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int c1   = __builtin_amdgcn_readfirstlane(bm.y * (OG_THREADS / 64) + w);
-    if (c1 >= s.cnt->n_cells || s.cnt->n_cell_pairs == 0) return;
-    int      *ex = exq[w];
-    const int p0 = __builtin_amdgcn_readfirstlane(s.cp_head[c1]);
-    const int p1 = __builtin_amdgcn_readfirstlane(s.cp_head[c1 + 1]);
+    const int n    = s.cnt->n_cells;
+    if (c1 >= n) return;
+    int       *ex  = exq[w];
+    const int *src = s.cp_stage + (size_t)c1 * OG_ENUM_STAGE;
+    const int  cnt = __builtin_amdgcn_readfirstlane(s.cp_count[c1]);
+    int        rec = src[lane];  // the stage of a cell is longer than a wave
+    static_assert(OG_ENUM_STAGE >= 64, "the first records are read before their count is known");
+    const int  a1  = lane >> 3;
+    const int  id1 = s.atomids[c1 * OG_NAC + a1];
+    const int  idl = s.atomids[c1 * OG_NAC + (lane & 7)];
+    long long  at  = 0;  // the list position of the cell's first record
+    for (int q = lane; q < (c1 >> 10); q += 64) at += s.cp_bsum[q];
+    for (int off = 32; off > 0; off >>= 1) at += __shfl_xor(at, off, 64);
+    at += s.cp_head[c1];
+    const long long end = at + cnt, cap = s.cap_cell_pairs;
+    if (lane == 0) {
+        s.cp_head[c1] = (int)min(at, cap);
+        if (c1 == n - 1) {
+            s.cp_head[n] = (int)min(end, cap);
+            if (end > cap) atomicOr(&s.cnt->flags, OG_F_CP_OVERFLOW);
+            s.cnt->n_cell_pairs = end > cap ? 0 : (int)end;
+        }
+    }
+    const int  p0     = __builtin_amdgcn_readfirstlane((int)min(at, cap));
+    const int  m1     = __builtin_amdgcn_readfirstlane((int)min(end, cap)) - p0;  // records that fit
+    const bool staged = cnt <= OG_ENUM_STAGE;
+    if (!staged) {  // did not fit the stage: enumerate again, writing in place
+        og_enum_cell<2>(s, c1, p0, nullptr);
+        __threadfence_block();
+        rec = lane < m1 ? s.cp_c2[p0 + lane] : 0;
+    }
+    const int4 *A4 = (const int4 *)s.atomids;
+    int4        u  = make_int4(0, 0, 0, 0), v = u;
+    if (lane < m1) u = A4[2 * (rec & 0xffffff)], v = A4[2 * (rec & 0xffffff) + 1];
 
     // exclusion entries: lane = 8 * a1 + (partner index within this round of 8)
-    const int a1  = lane >> 3;
-    const int id1 = s.atomids[c1 * OG_NAC + a1];
-    bool      open = id1 >= 0;  // a1's list has not ended yet
-    int       nex  = 0;
+    bool open = id1 >= 0;  // a1's list has not ended yet
+    int  nex  = 0;
     for (int kb = 0; kb < OG_MAX_NB15; kb += 8) {
         const int      k    = kb + (lane & 7);
         const int      t    = open ? s.nb15off[(size_t)id1 * OG_MAX_NB15 + k] : -1;
@@ -632,19 +635,17 @@ __global__ void __launch_bounds__(OG_THREADS) k_masks(const og_dev_sys *__restri
     }
 
     // dummy atoms of cell1: bit a1 of every row byte
-    const int      idl  = s.atomids[c1 * OG_NAC + (lane & 7)];
     const unsigned dmy1 = (unsigned)__ballot(idl < 0) & 0xffu;
     const uint64_t cols = (uint64_t)dmy1 * 0x0101010101010101ull;
     // self pair: a1 >= a2, i.e. bits a2..7 of row byte a2
     uint64_t self = 0;
     for (int a2 = 0; a2 < OG_NAC; a2++) self |= (uint64_t)((0xffu << a2) & 0xffu) << (8 * a2);
-    const int4 *A4 = (const int4 *)s.atomids;
-    for (int base = p0; base < p1; base += 64) {
-        const int p = base + lane;
-        if (p < p1) {
-            const int  c2 = s.cp_c2[p] & 0xffffff;
-            const int4 u = A4[2 * c2], v = A4[2 * c2 + 1];
-            uint64_t   m = cols | (c2 == c1 ? self : 0ull);
+    for (int base = 0; base < m1; base += 64) {
+        const int k = base + lane;
+        if (k < m1) {
+            const int p  = p0 + k;
+            const int c2 = rec & 0xffffff;
+            uint64_t  m  = cols | (c2 == c1 ? self : 0ull);
             // dummy atoms of cell2: the whole row byte
             m |= (u.x < 0 ? 0xffull : 0ull) | (u.y < 0 ? 0xffull << 8 : 0ull) | (u.z < 0 ? 0xffull << 16 : 0ull) |
                  (u.w < 0 ? 0xffull << 24 : 0ull) | (v.x < 0 ? 0xffull << 32 : 0ull) |
@@ -654,13 +655,18 @@ __global__ void __launch_bounds__(OG_THREADS) k_masks(const og_dev_sys *__restri
                 const int q = ex[e];
                 if ((q >> 6) == c2) m |= 1ull << (q & 63);
             }
+            if (staged) s.cp_c2[p] = rec;
             s.cp_mask[p] = m;
+        }
+        if (k + 64 < m1) {  // the next 64
+            rec = staged ? src[k + 64] : s.cp_c2[p0 + k + 64];
+            u   = A4[2 * (rec & 0xffffff)], v = A4[2 * (rec & 0xffffff) + 1];
         }
     }
 }
 
 // ------------------------------------------------------------- launchers --
-void og_launch_grid_clear(const og_launch &cols, const og_launch &) {
+void og_launch_grid_clear(const og_launch &cols) {
     hipLaunchKernelGGL(k_grid_clear, dim3(cols.n_blocks), dim3(OG_THREADS), 0, cols.stream, cols.sys, cols.map);
 }
 void og_launch_grid_bin(const og_launch &a) {
@@ -681,16 +687,9 @@ void og_launch_cells_from_grid(const og_launch &a) {
 void og_launch_enum_count(const og_launch &a) {
     hipLaunchKernelGGL(k_enum_count, dim3(a.n_blocks), dim3(OG_THREADS), 0, a.stream, a.sys, a.map);
 }
-void og_launch_enum_scan_blocks(const og_launch &a) {
-    hipLaunchKernelGGL(k_enum_scan_part, dim3(a.n_blocks), dim3(1024), 0, a.stream, a.sys, a.map);
-    hipLaunchKernelGGL(k_enum_scan_add, dim3(a.n_blocks), dim3(1024), 0, a.stream, a.sys, a.map);
-}
 void og_launch_enum_scan(const og_launch &a) {
     hipLaunchKernelGGL(k_enum_scan, dim3(a.n_blocks), dim3(1024), 0, a.stream, a.sys, a.map);
 }
-void og_launch_enum_write(const og_launch &a) {
-    hipLaunchKernelGGL(k_enum_write, dim3(a.n_blocks), dim3(OG_THREADS), 0, a.stream, a.sys, a.map);
-}
-void og_launch_masks(const og_launch &a) {
-    hipLaunchKernelGGL(k_masks, dim3(a.n_blocks), dim3(OG_THREADS), 0, a.stream, a.sys, a.map);
+void og_launch_list(const og_launch &a) {
+    hipLaunchKernelGGL(k_list, dim3(a.n_blocks), dim3(OG_THREADS), 0, a.stream, a.sys, a.map);
 }

@@ -199,7 +199,7 @@ struct og_dev_sys {
     // ---- grid ----
     int      *col_of_atom;  // [n_atoms]
     uint32_t *zkey;         // [n_atoms] order-preserving float-z bits
-    int      *n_atoms_col;  // [n_columns]
+    int      *n_atoms_col;  // [n_columns] zero between rebuilds (counted by the binning, cleared by the sort)
     int      *col_fill;     // [n_columns]
     int      *head_cell;    // [n_columns+1], -1 = empty column
     int      *head_atom;    // [n_columns+1], -1 = empty column
@@ -484,17 +484,15 @@ struct og_launch {
 };
 
 // grid build
-void og_launch_grid_clear(const og_launch &cols, const og_launch &bins);
+void og_launch_grid_clear(const og_launch &cols);
 void og_launch_grid_bin(const og_launch &atoms);
 void og_launch_grid_scan(const og_launch &sys);
 void og_launch_grid_scatter(const og_launch &atoms);
 void og_launch_grid_sort(const og_launch &cols);
 void og_launch_cells_from_grid(const og_launch &cols);
 void og_launch_enum_count(const og_launch &cellw);
-void og_launch_enum_scan(const og_launch &sys);
-void og_launch_enum_scan_blocks(const og_launch &blocks);  // blocks of 1024 cells (cap_cells + 1)
-void og_launch_enum_write(const og_launch &cellw);
-void og_launch_masks(const og_launch &cp);
+void og_launch_enum_scan(const og_launch &blocks);  // blocks of 1024 cells (cap_cells + 1); null map: one system
+void og_launch_list(const og_launch &cellw);
 // forces
 // pair forms of og_launch_pair
 enum { OG_FORM_ZD = 0, OG_FORM_ZD_ALPHA = 1, OG_FORM_HPS_DH = 2, OG_FORM_ZM = 3, OG_FORM_ZM_ALPHA = 4 };
