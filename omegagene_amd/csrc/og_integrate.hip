@@ -331,12 +331,13 @@ __device__ __forceinline__ void og_shake_trio(const og_dev_sys &s, int a1, int a
 
 // Analytic SETTLE (S. Miyamoto, P. A. Kollman, J. Comput. Chem. 13 (1992) 952-962)
 // for a rigid 3-site water (O, H1, H2); same arithmetic as the oracle's orc_settle.
-// Core on values: xO/xH1/xH2 are the unconstrained positions (moved to the
-// constrained ones), pO/pH1/pH2 the previous positions.  Returns false, with
-// the positions untouched, when there is no rigid solution.
+// Core on values: xO/xH1/xH2 are the unconstrained positions, pO/pH1/pH2 the
+// previous positions; D holds what each atom's position is to be moved by.
+// Returns false, with D unset, when there is no rigid solution.
 __device__ __forceinline__ bool og_settle_core(const og_dev_sys &s, double mO, double mH, double dOH, double dHH,
-                                               double *xO, double *xH1, double *xH2, const double *pO,
-                                               const double *pH1, const double *pH2) {
+                                               const double *xO, const double *xH1, const double *xH2,
+                                               const double *pO, const double *pH1, const double *pH2,
+                                               double (*D)[3]) {
     const double wt = mO + 2.0 * mH;
     const double rc = 0.5 * dHH;
     const double h  = sqrt(dOH * dOH - rc * rc);
@@ -404,9 +405,9 @@ __device__ __forceinline__ bool og_settle_core(const og_dev_sys &s, double mO, d
         const double ca = com[d] + X[d] * a3[0] + Y[d] * a3[1] + Z[d] * a3[2];
         const double cb = com[d] + X[d] * b3[0] + Y[d] * b3[1] + Z[d] * b3[2];
         const double cc = com[d] + X[d] * c3[0] + Y[d] * c3[1] + Z[d] * c3[2];
-        xO[d] += ca;
-        xH1[d] += cb - xb[d];
-        xH2[d] += cc - xc[d];
+        D[0][d] = ca;
+        D[1][d] = cb - xb[d];
+        D[2][d] = cc - xc[d];
     }
     return true;
 }
@@ -420,12 +421,13 @@ __device__ void og_settle(const og_dev_sys &s, int iO, int iH1, int iH2, double 
             x[a][d] = s.crd[3 * ia[a] + d];
             p[a][d] = s.crd_prev[3 * ia[a] + d];
         }
-    if (!og_settle_core(s, s.mass[iO], s.mass[iH1], dOH, dHH, x[0], x[1], x[2], p[0], p[1], p[2])) {
+    double D[3][3];
+    if (!og_settle_core(s, s.mass[iO], s.mass[iH1], dOH, dHH, x[0], x[1], x[2], p[0], p[1], p[2], D)) {
         atomicAdd(&s.cnt->shake_fail, 1);
         return;
     }
     for (int a = 0; a < 3; a++)
-        for (int d = 0; d < 3; d++) s.crd[3 * ia[a] + d] = x[a][d];
+        for (int d = 0; d < 3; d++) s.crd[3 * ia[a] + d] = x[a][d] + D[a][d];
 }
 
 __global__ void __launch_bounds__(OG_TRIO_THREADS) k_trio(const og_dev_sys *__restrict__ S,
@@ -658,52 +660,67 @@ __device__ __forceinline__ void og_water_lanes(const og_dev_sys &s, const int bl
         for (int d = 0; d < 3; d++) X[k][d] = __shfl(x[d], base + k, 64);
         Q[k] = __shfl(q, base + k, 64);
     }
-    // excluded pairs of the atom, in its list order (og_atom_work_calc)
-    auto excl = [&](const int4 en) {
-        const int   la = en.x == ia[0] ? 0 : (en.x == ia[1] ? 1 : 2);
-        const int   lb = en.y == ia[0] ? 0 : (en.y == ia[1] ? 1 : 2);
-        float       we[3];
-        const float ene = og_excess_pair(s, X[la], X[lb], Q[la], Q[lb], we);
-        if (la == ac) {
-            for (int d = 0; d < 3; d++) w[d] += (double)we[d];
-            if (live) e_ex += (double)ene;
-        } else {
-            for (int d = 0; d < 3; d++) w[d] -= (double)we[d];
+    // excluded pairs of the atom, in its list order (og_atom_work_calc); one copy of the pair's code
+#pragma unroll 1
+    for (int e = e0; e < e1; e++) {
+        const int4 en  = e == e0 ? ent[0] : e == e0 + 1 ? ent[1] : s.exc_at[e];
+        const bool own = en.x == i;
+        const int  la  = en.x == ia[0] ? 0 : (en.x == ia[1] ? 1 : 2);
+        const int  lb  = en.y == ia[0] ? 0 : (en.y == ia[1] ? 1 : 2);
+        double     a[3], b[3];
+        for (int d = 0; d < 3; d++) {
+            a[d] = la == 0 ? X[0][d] : la == 1 ? X[1][d] : X[2][d];
+            b[d] = lb == 0 ? X[0][d] : lb == 1 ? X[1][d] : X[2][d];
         }
-    };
-    for (int j = 0; j < 2; j++)
-        if (e0 + j < e1) excl(ent[j]);
-    for (int e = e0 + 2; e < e1; e++) excl(s.exc_at[e]);
+        float       we[3];
+        const float ene = og_excess_pair(s, a, b, la == 0 ? Q[0] : la == 1 ? Q[1] : Q[2],
+                                         lb == 0 ? Q[0] : lb == 1 ? Q[1] : Q[2], we);
+        for (int d = 0; d < 3; d++) w[d] += own ? (double)we[d] : -(double)we[d];
+        e_ex += own && live ? (double)ene : 0.0;
+    }
     double xn[3];
     og_langevin_core(s, i, step, x, xp, vn, w, (double)m, (double)mi, xn);
-    double XN[3][3];
-    for (int k = 0; k < 3; k++)
-        for (int d = 0; d < 3; d++) XN[k][d] = __shfl(xn[d], base + k, 64);
-    const double mO = __shfl((double)m, base, 64), mH = __shfl((double)m, base + 1, 64);
-    if (!og_settle_core(s, mO, mH, s.settle_dOH, s.settle_dHH, XN[0], XN[1], XN[2], X[0], X[1], X[2]) && live &&
-        ac == 0)
-        atomicAdd(&s.cnt->shake_fail, 1);
+    // what is final goes out here: fewer registers are held through SETTLE
+    if (live) {
+        og_fx_consume(s.fx, cap, og_fx_slot(g));
+        for (int d = 0; d < 3; d++) {
+            s.work[3 * i + d]      = w[d];
+            s.crd_prev2[3 * i + d] = xp[d];
+            s.crd_prev[3 * i + d]  = x[d];
+        }
+    }
+    double D[3][3];
+    bool   ok;
+    {
+        double XN[3][3];
+        for (int k = 0; k < 3; k++)
+            for (int d = 0; d < 3; d++) XN[k][d] = __shfl(xn[d], base + k, 64);
+        const double mO = __shfl((double)m, base, 64), mH = __shfl((double)m, base + 1, 64);
+        ok = og_settle_core(s, mO, mH, s.settle_dOH, s.settle_dHH, XN[0], XN[1], XN[2], X[0], X[1], X[2], D);
+    }
+    if (!ok && live && ac == 0) atomicAdd(&s.cnt->shake_fail, 1);
+    if (ok)
+        for (int d = 0; d < 3; d++) xn[d] += ac == 0 ? D[0][d] : ac == 1 ? D[1][d] : D[2][d];
     double v[3], xw[3];
     float  f[3];
-    const double ka = og_langevin_vel(s, step, XN[ac], xp, vn, v);
-    og_advance(s, XN[ac], x, gc, f, xw);
+    const double ka = og_langevin_vel(s, step, xn, xp, vn, v);
+    og_advance(s, xn, x, gc, f, xw);
     if (!live) return;
     ke += ka * (double)m;
-    og_fx_consume(s.fx, cap, og_fx_slot(g));
     for (int d = 0; d < 3; d++) {
-        s.work[3 * i + d]      = w[d];
-        s.crd_prev2[3 * i + d] = xp[d];
-        s.crd_prev[3 * i + d]  = x[d];
-        s.crd[3 * i + d]       = xw[d];
-        s.vel[3 * i + d]       = step == 0 ? vn[d] : v[d];
-        s.gcrd[3 * g + d]      = gc[d];
+        s.crd[3 * i + d]  = xw[d];
+        s.vel[3 * i + d]  = step == 0 ? vn[d] : v[d];
+        s.gcrd[3 * g + d] = gc[d];
     }
     s.gxyzq[g] = make_float4(f[0], f[1], f[2], gw);
 }
 
 __device__ void og_vcmd_block(const og_dev_sys &s, double *bias, int &active);  // VcMD section below
 
-__global__ void __launch_bounds__(OG_WATER_THREADS) k_langevin_step(const og_dev_sys *__restrict__ S,
+// Three waves per SIMD (168 registers): left free the kernel takes 203 (two
+// waves), held to 128 it spills (450,000 atoms 430 / 421 / 429 us per step at
+// two / three / four waves, sixteen walkers 303 / 297 / 299).
+__global__ void __launch_bounds__(OG_WATER_THREADS, 3) k_langevin_step(const og_dev_sys *__restrict__ S,
                                                                     const int2 *__restrict__ map) {
     const int2        bm = map[blockIdx.x];
     const og_dev_sys &s  = S[bm.x];

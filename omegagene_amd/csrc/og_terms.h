@@ -119,19 +119,17 @@ __device__ __forceinline__ double og_bond_pair(const og_dev_sys &s, double bk, d
     return coef * dif;
 }
 
-#ifndef OG_TERM_BATCH
-#define OG_TERM_BATCH 8  // list entries whose loads are issued together
-#endif
-
 // Atom i: fixed-point pair gradient (grid slot) -> FP64 "work" in atom order
 // (SubBox::add_work_from_minicell, SubBox.cpp:1398-1407), plus the atom's
 // excluded-pair ZD terms (SubBox::calc_energy_ele_excess SubBox.cpp:1347-1367)
 // and bonds through per-atom lists: every pair term is evaluated for both of
 // its atoms in the orientation of the reference list, so no atomics are
 // needed and the sums are deterministic.  Energies are counted on the pair's
-// first atom.  The lists are walked in batches: the entries, then the
-// partners' coordinates, are loaded for a whole batch before the terms are
-// added in list order.  Returns the work in w; stores nothing.
+// first atom.  The terms are added in list order; a term's partner loads
+// while the term before it is evaluated, its list entry one term earlier.
+// One copy of each term's code: batches of eight loads with their terms
+// unrolled ran 16 copies of the excluded pair, most of the time out of the
+// instruction cache (OG_F2W figures).  Returns the work in w; stores nothing.
 __device__ __forceinline__ void og_atom_work_calc(const og_dev_sys &s, const int i, double *w, double &e_ex,
                                                   double &e_b) {
 #pragma clang fp contract(off)
@@ -143,72 +141,56 @@ __device__ __forceinline__ void og_atom_work_calc(const og_dev_sys &s, const int
     for (int k = 0; k < 3; k++) xi[k] = s.crd[3 * i + k];
     const float qi = s.charge[i];
     og_fx_read(s.fx, cap, og_fx_slot(g), w);
-    for (int eb = x0; eb < x1; eb += OG_TERM_BATCH) {
-        const int n = min(OG_TERM_BATCH, x1 - eb);
-        int       other[OG_TERM_BATCH];
-        bool      first[OG_TERM_BATCH];
-#pragma unroll
-        for (int j = 0; j < OG_TERM_BATCH; j++)
-            if (j < n) {
-                const int4 ent = s.exc_at[eb + j];
-                first[j]       = ent.x == i;
-                other[j]       = first[j] ? ent.y : ent.x;
-            }
-        double xo[OG_TERM_BATCH][3];
-        float  qo[OG_TERM_BATCH];
-#pragma unroll
-        for (int j = 0; j < OG_TERM_BATCH; j++)
-            if (j < n) {
-                for (int k = 0; k < 3; k++) xo[j][k] = s.crd[3 * other[j] + k];
-                qo[j] = s.charge[other[j]];
-            }
-#pragma unroll
-        for (int j = 0; j < OG_TERM_BATCH; j++)
-            if (j < n) {
-                float we[3];
-                if (first[j]) {
-                    const float ene = og_excess_pair(s, xi, xo[j], qi, qo[j], we);
-                    for (int k = 0; k < 3; k++) w[k] += (double)we[k];
-                    e_ex += (double)ene;
-                } else {
-                    og_excess_pair(s, xo[j], xi, qo[j], qi, we);
-                    for (int k = 0; k < 3; k++) w[k] -= (double)we[k];
-                }
-            }
+    // the partner of list entry at[e] and its position; past the list's end nothing is read
+    auto partner = [&](const int4 ent, const bool in, double *x, bool &first) {
+        first       = ent.x == i;
+        const int o = first ? ent.y : ent.x;
+        if (in)
+            for (int k = 0; k < 3; k++) x[k] = s.crd[3 * o + k];
+        return o;
+    };
+    if (x0 < x1) {
+        int4   ent = s.exc_at[x0], nxt = s.exc_at[min(x0 + 1, x1 - 1)];
+        double xo[3];
+        bool   first;
+        float  qo = s.charge[partner(ent, true, xo, first)];
+#pragma unroll 1
+        for (int e = x0; e < x1; e++) {
+            double     xn[3] = {xo[0], xo[1], xo[2]};
+            bool       fn;
+            const int  on  = partner(nxt, e + 1 < x1, xn, fn);
+            const float qn = s.charge[on];
+            nxt            = s.exc_at[min(e + 2, x1 - 1)];
+            double a[3], b[3];
+            for (int k = 0; k < 3; k++) a[k] = first ? xi[k] : xo[k], b[k] = first ? xo[k] : xi[k];
+            float       we[3];
+            const float ene = og_excess_pair(s, a, b, first ? qi : qo, first ? qo : qi, we);
+            for (int k = 0; k < 3; k++) w[k] += first ? (double)we[k] : -(double)we[k];
+            e_ex += first ? (double)ene : 0.0;
+            for (int k = 0; k < 3; k++) xo[k] = xn[k];
+            qo = qn, first = fn;
+        }
     }
-    for (int eb = b0; eb < b1; eb += OG_TERM_BATCH) {
-        const int n = min(OG_TERM_BATCH, b1 - eb);
-        int       other[OG_TERM_BATCH], t[OG_TERM_BATCH];
-        bool      first[OG_TERM_BATCH];
-#pragma unroll
-        for (int j = 0; j < OG_TERM_BATCH; j++)
-            if (j < n) {
-                const int4 ent = s.bond_at[eb + j];
-                first[j]       = ent.x == i;
-                other[j]       = first[j] ? ent.y : ent.x;
-                t[j]           = ent.z;
-            }
-        double xo[OG_TERM_BATCH][3], bk[OG_TERM_BATCH], r0[OG_TERM_BATCH];
-#pragma unroll
-        for (int j = 0; j < OG_TERM_BATCH; j++)
-            if (j < n) {
-                for (int k = 0; k < 3; k++) xo[j][k] = s.crd[3 * other[j] + k];
-                bk[j] = s.bond_k[t[j]];
-                r0[j] = s.bond_r0[t[j]];
-            }
-#pragma unroll
-        for (int j = 0; j < OG_TERM_BATCH; j++)
-            if (j < n) {
-                double wb[3];
-                if (first[j]) {
-                    const double ene = og_bond_pair(s, bk[j], r0[j], xi, xo[j], wb);
-                    for (int k = 0; k < 3; k++) w[k] += wb[k];
-                    e_b += ene;
-                } else {
-                    og_bond_pair(s, bk[j], r0[j], xo[j], xi, wb);
-                    for (int k = 0; k < 3; k++) w[k] -= wb[k];
-                }
-            }
+    if (b0 < b1) {
+        int4   ent = s.bond_at[b0], nxt = s.bond_at[min(b0 + 1, b1 - 1)];
+        double xo[3], bk = s.bond_k[ent.z], r0 = s.bond_r0[ent.z];
+        bool   first;
+        partner(ent, true, xo, first);
+#pragma unroll 1
+        for (int e = b0; e < b1; e++) {
+            double       xn[3] = {xo[0], xo[1], xo[2]};
+            bool         fn;
+            const double bn = s.bond_k[nxt.z], rn = s.bond_r0[nxt.z];
+            partner(nxt, e + 1 < b1, xn, fn);
+            nxt = s.bond_at[min(e + 2, b1 - 1)];
+            double a[3], b[3], wb[3];
+            for (int k = 0; k < 3; k++) a[k] = first ? xi[k] : xo[k], b[k] = first ? xo[k] : xi[k];
+            const double ene = og_bond_pair(s, bk, r0, a, b, wb);
+            for (int k = 0; k < 3; k++) w[k] += first ? wb[k] : -wb[k];
+            e_b += first ? ene : 0.0;
+            for (int k = 0; k < 3; k++) xo[k] = xn[k];
+            bk = bn, r0 = rn, first = fn;
+        }
     }
     // angles, torsions, impropers and 1-4 pairs: the atom's shares, written
     // by k_bonded earlier in the evaluation, in ascending slot order
