@@ -352,7 +352,7 @@ og_status exec_prepare(og_exec &x) {
         cnt[KIND_MISC]  = cdiv(d.n_pairs_c, OG_THREADS);  // SHAKE pair constraints
         cnt[KIND_TRIO]  = cdiv(std::max(d.n_trios, d.n_settle), OG_TRIO_THREADS);
         cnt[KIND_COMA] = 0;  // filled below
-        cnt[KIND_LSTEP] = d.n_water_blocks ? d.n_water_blocks + 1 : 0;  // free-atom block + water blocks
+        cnt[KIND_LSTEP] = d.n_water_blocks ? og_lead_blocks(d) + d.n_water_blocks : 0;
         cnt[KIND_BTERM] = cdiv(d.n_bterms, OG_THREADS);
         cnt[KIND_QUAD]  = d.constraint ? cdiv(d.n_quads, OG_QUAD_THREADS) : 0;
         cnt[KIND_SCANB] = d.cap_cells / 1024 + 1;
@@ -469,8 +469,7 @@ void enqueue_forces(og_exec &x, hipEvent_t e0, hipEvent_t e1, bool point = false
 
 void enqueue_integrate(og_exec &x) {
     if (x.fused) {
-        og_launch_langevin_step(L(x, KIND_LSTEP));
-        og_launch_step_close(L(x, KIND_SYS));
+        og_launch_langevin_step(L(x, KIND_LSTEP));  // closes the step
         return;
     }
     // the extended-ensemble bias acts on the gradient of the step
@@ -1044,7 +1043,9 @@ og_status sys_alloc(og_system *s, const og_system_desc *d, const og_params *p) {
             if (!A(&h.free_ids, std::max<size_t>(free_ids.size(), 1))) return OG_E_DEVICE;
             if (!free_ids.empty())
                 OG_HIP(hipMemcpy(h.free_ids, free_ids.data(), sizeof(int) * free_ids.size(), hipMemcpyHostToDevice));
+            if (!A(&h.sync, 1)) return OG_E_DEVICE;
             h.n_free         = (int)free_ids.size();
+            h.n_free_blocks  = std::max(1, cdiv(h.n_free, OG_FREE_PER_BLOCK));
             h.n_water_blocks = nwb;
         }
     }
@@ -1313,7 +1314,7 @@ og_status og_system_footprint(const og_system_desc *d, const og_params *p, uint6
     b += cells * (6 * 4 + 4.0 * OG_ENUM_STAGE + 8) + (cells / 1024 + 1) * 8;
     b += pairs * 12;
     b += 8.0 * OG_EACC_SLOTS * OG_EACC_STRIDE + ke_parts * 8 + OG_E_NTERMS * 8 + log_rows * OG_E_NTERMS * 8;
-    b += std::min(n, (double)OG_FREE_MAX) * 4 + vc * 28 + vs * 32 + mcs * (4 + 8.0 * OG_MC_NPOLY + 32);
+    b += std::min(n, (double)OG_FREE_MAX) * 4 + sizeof(og_step_sync) + vc * 28 + vs * 32 + mcs * (4 + 8.0 * OG_MC_NPOLY + 32);
     {
         const double na = d->n_angles, ntr = (double)d->n_torsions + d->n_impros, n14 = d->n_nb14;
         const double nq = p->constraint ? d->n_shake_quads : 0;

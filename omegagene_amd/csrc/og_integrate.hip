@@ -459,7 +459,7 @@ __device__ __forceinline__ void og_ke_partial(const og_dev_sys &s, const int slo
     if (threadIdx.x == 0 && slot < s.n_ke_parts) {
         double t = 0.0;
         for (int k = 0; k < (int)(blockDim.x >> 6); k++) t += sh[k];
-        s.e_atom[slot] = t;
+        og_put(&s.e_atom[slot], t);
     }
 }
 
@@ -558,17 +558,19 @@ __global__ void __launch_bounds__(OG_THREADS) k_finish(const og_dev_sys *__restr
 // pair/excluded-pair/bond energies (on logged or requested steps), kinetic
 // energy from the per-block partials, the energy log entry, and the step
 // counter.  c: the system's counters as read at the start of the block.
-__device__ __forceinline__ void og_close_step(const og_dev_sys &s, const og_dev_counters &c) {
+// n_parts: the kinetic partials the step wrote.
+__device__ __forceinline__ void og_close_step(const og_dev_sys &s, const og_dev_counters &c, const int n_parts) {
     // the kinetic partials are read first (loads issued four strides at a
     // time, added in stride order) so they overlap the counter reads
     double t = 0.0;
-    for (int k = threadIdx.x; k < s.n_ke_parts; k += 4 * OG_STEP_THREADS) {
+    for (int k = threadIdx.x; k < n_parts; k += 4 * OG_STEP_THREADS) {
         double v[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++) v[j] = k + j * OG_STEP_THREADS < s.n_ke_parts ? s.e_atom[k + j * OG_STEP_THREADS] : 0.0;
+        for (int j = 0; j < 4; j++)
+            v[j] = k + j * OG_STEP_THREADS < n_parts ? og_take(&s.e_atom[k + j * OG_STEP_THREADS]) : 0.0;
 #pragma unroll
         for (int j = 0; j < 4; j++)
-            if (k + j * OG_STEP_THREADS < s.n_ke_parts) t += v[j];
+            if (k + j * OG_STEP_THREADS < n_parts) t += v[j];
     }
     // read with the partials, before the counters are known (one memory
     // round trip less): the accumulator slots and, in thread 0, the energy
@@ -577,7 +579,7 @@ __device__ __forceinline__ void og_close_step(const og_dev_sys &s, const og_dev_
     const long long ev = og_eacc_load<OG_STEP_THREADS>(s);
     double row[OG_E_NTERMS];
     if (threadIdx.x == 0)
-        for (int k = 0; k < OG_E_NTERMS; k++) row[k] = s.energy[k];
+        for (int k = 0; k < OG_E_NTERMS; k++) row[k] = og_take(&s.energy[k]);
     if (og_frozen_c(c)) return;
     __shared__ double    sh[OG_STEP_THREADS / 64];
     __shared__ long long she[16 * OG_EACC_STRIDE];
@@ -607,17 +609,25 @@ __device__ __forceinline__ void og_close_step(const og_dev_sys &s, const og_dev_
 // One launch for the whole integration step of a Langevin system whose
 // SETTLE waters interact with nothing but their own atoms through exclusions
 // and carry no bonds, VcMD groups or SHAKE groups:
-//  * block 0 of a system takes every other ("free") atom through the same
-//    sequence as the separate kernels -- gradient conversion, VcMD bias,
-//    Langevin positions, SHAKE pairs then trios, finish -- with a block
-//    barrier between the stages;
-//  * blocks 1.. take the waters, three lanes per water (og_water_lanes):
-//    gradient conversion, Langevin positions, SETTLE and finish.
+//  * the lead blocks of a system convert the gradient of every other ("free")
+//    atom, eight lanes per atom (og_free_work), and one more block finds the
+//    VcMD / V-AUS bias, which needs no gradient; the last of them to arrive
+//    takes the free atoms on -- bias, Langevin positions, SHAKE pairs then
+//    trios, finish -- with a block barrier between the stages;
+//  * the other blocks take the waters, three lanes per water
+//    (og_water_lanes): gradient conversion, Langevin positions, SETTLE and
+//    finish;
+//  * the last block to arrive closes the step (og_close_step).
 // Each atom goes through the same device functions, in the same order, as in
 // the separate kernels, so the trajectory is bitwise the same; only the
 // FP64 block partials of the kinetic, excluded-pair and bond energies are
-// grouped differently (block 0, then the water blocks; the remaining e_atom
-// slots are zeroed).
+// grouped differently (the free atoms, then the water blocks; the remaining
+// e_atom slots are not read).
+//
+// A launch of one walker is latency: one block for all free atoms took 17.3 us
+// of it (13,481 atoms, 200 of them free; a wave alone on its SIMD issues one
+// instruction per 8 cycles) against 11.5 for the water blocks, and a closing
+// kernel of its own 4.8.
 // SETTLE waters of the fused Langevin step, three lanes per water (lane
 // 3k + a holds atom a of the wave's water k; lane 63 is an idle copy): each
 // lane loads its atom, takes the other two atoms' positions by shuffles for
@@ -715,53 +725,135 @@ __device__ __forceinline__ void og_water_lanes(const og_dev_sys &s, const int bl
     s.gxyzq[g] = make_float4(f[0], f[1], f[2], gw);
 }
 
-__device__ void og_vcmd_block(const og_dev_sys &s, double *bias, int &active);  // VcMD section below
+// Gradient of the free atoms of lead block blk, eight lanes per atom: each
+// evaluates one term of the atom's lists at a time, then all add them in list
+// order (og_atom_work_calc's sums).  The work goes to another block.
+__device__ __forceinline__ void og_free_work(const og_dev_sys &s, const int blk, double &e_ex, double &e_b) {
+    if (s.n_free == 0) return;
+    const int  lane = threadIdx.x & 63, q = lane & 7, base = lane & ~7;
+    const int  k    = blk * OG_FREE_PER_BLOCK + (threadIdx.x >> 3);
+    const bool live = k < s.n_free;
+    const int  i    = s.free_ids[min(k, s.n_free - 1)];
+    const int  g    = s.rev[i];
+    const int  x0 = s.exc_off[i], nx = live ? s.exc_off[i + 1] - x0 : 0;
+    const int  b0 = s.bond_off[i], nb = live ? s.bond_off[i + 1] - b0 : 0;
+    double     xi[3], w[3];
+    for (int d = 0; d < 3; d++) xi[d] = s.crd[3 * i + d];
+    const float qi = s.charge[i];
+    og_fx_read(s.fx, s.cap_atom_array, og_fx_slot(g), w);
+    for (int r = 0; __any(r < nx); r += 8) {
+        float we[3] = {0.0f, 0.0f, 0.0f};
+        if (r + q < nx) {
+            const int4  en    = s.exc_at[x0 + r + q];
+            const bool  first = en.x == i;
+            const int   o     = first ? en.y : en.x;
+            const float qo    = s.charge[o];
+            double      a[3], b[3];
+            for (int d = 0; d < 3; d++) {
+                const double xo = s.crd[3 * o + d];
+                a[d] = first ? xi[d] : xo, b[d] = first ? xo : xi[d];
+            }
+            const float ene = og_excess_pair(s, a, b, first ? qi : qo, first ? qo : qi, we);
+            if (first) e_ex += (double)ene;
+            for (int d = 0; d < 3; d++) we[d] = first ? we[d] : -we[d];
+        }
+        for (int t = 0; t < 8 && __any(r + t < nx); t++)
+            for (int d = 0; d < 3; d++) {
+                const float v = __shfl(we[d], base + t, 64);
+                if (r + t < nx) w[d] += (double)v;
+            }
+    }
+    for (int r = 0; __any(r < nb); r += 8) {
+        double wb[3] = {0.0, 0.0, 0.0};
+        if (r + q < nb) {
+            const int4 en    = s.bond_at[b0 + r + q];
+            const bool first = en.x == i;
+            const int  o     = first ? en.y : en.x;
+            double     a[3], b[3];
+            for (int d = 0; d < 3; d++) {
+                const double xo = s.crd[3 * o + d];
+                a[d] = first ? xi[d] : xo, b[d] = first ? xo : xi[d];
+            }
+            const double ene = og_bond_pair(s, s.bond_k[en.z], s.bond_r0[en.z], a, b, wb);
+            if (first) e_b += ene;
+            for (int d = 0; d < 3; d++) wb[d] = first ? wb[d] : -wb[d];
+        }
+        for (int t = 0; t < 8 && __any(r + t < nb); t++)
+            for (int d = 0; d < 3; d++) {
+                const double v = __shfl(wb[d], base + t, 64);
+                if (r + t < nb) w[d] += v;
+            }
+    }
+    if (!live || q != 0) return;
+    og_atom_work_bonded(s, i, w);
+    og_fx_consume(s.fx, s.cap_atom_array, og_fx_slot(g));
+    for (int d = 0; d < 3; d++) og_put(&s.work[3 * i + d], w[d]);
+}
+
+__device__ void og_vcmd_lambda(const og_dev_sys &s, double *bias, int &active);  // VcMD section below
+__device__ void og_vcmd_apply(const og_dev_sys &s, const double *bias);
 
 // Three waves per SIMD (168 registers): left free the kernel takes 203 (two
 // waves), held to 128 it spills (450,000 atoms 430 / 421 / 429 us per step at
 // two / three / four waves, sixteen walkers 303 / 297 / 299).
 __global__ void __launch_bounds__(OG_WATER_THREADS, 3) k_langevin_step(const og_dev_sys *__restrict__ S,
-                                                                    const int2 *__restrict__ map) {
-    const int2        bm = map[blockIdx.x];
-    const og_dev_sys &s  = S[bm.x];
-    if (og_frozen(s)) return;
-    const long long step = s.cnt->step;
-    const int       tid  = threadIdx.x;
-    double          e_ex = 0.0, e_b = 0.0, ke = 0.0;
-    if (bm.y == 0) {
-        const int nf = s.n_free;
-        for (int k = tid; k < nf; k += OG_WATER_THREADS) og_atom_work(s, s.free_ids[k], e_ex, e_b);
-        __syncthreads();
-        if (s.vc_n_states || s.mc_mode == OG_MC_VAUS) {
-            __shared__ double bias[3];
-            __shared__ int    active;
-            og_vcmd_block(s, bias, active);
-            __syncthreads();
-        }
-        for (int k = tid; k < nf; k += OG_WATER_THREADS) {
-            const int    i     = s.free_ids[k];
-            const double wk[3] = {s.work[3 * i], s.work[3 * i + 1], s.work[3 * i + 2]};
-            og_langevin_atom(s, i, step, wk);
-        }
-        __syncthreads();
-        if (s.constraint) {
-            for (int t = tid; t < s.n_pairs_c; t += OG_WATER_THREADS) og_shake_pair(s, t);
-            __syncthreads();
-            for (int t = tid; t < s.n_trios; t += OG_WATER_THREADS)
-                og_shake_trio(s, s.trio_ids[3 * t], s.trio_ids[3 * t + 1], s.trio_ids[3 * t + 2], s.trio_d2 + 3 * t);
-            __syncthreads();
-        }
-        for (int k = tid; k < nf; k += OG_WATER_THREADS) ke += og_finish_atom(s, s.free_ids[k], step);
-        for (int k = s.n_water_blocks + 1 + tid; k < s.n_ke_parts; k += OG_WATER_THREADS) s.e_atom[k] = 0.0;
-    } else {
-        og_water_lanes(s, bm.y - 1, step, e_ex, ke);
-    }
+                                                                       const int2 *__restrict__ map) {
+    const int2            bm = map[blockIdx.x];
+    const og_dev_sys     &s  = S[bm.x];
+    const og_dev_counters c  = *s.cnt;
+    if (og_frozen_c(c)) return;
+    const long long   step = c.step;
+    const int         tid  = threadIdx.x;
+    const int         lead = og_lead_blocks(s);
+    double            e_ex = 0.0, e_b = 0.0, ke = 0.0;
     __shared__ double sh[2 * (OG_WATER_THREADS / 64)];
-    og_ke_partial(s, bm.y, ke, sh);
-    if (og_energy_step(s)) {
+    if (bm.y >= lead) {
+        og_water_lanes(s, bm.y - lead, step, e_ex, ke);
+        og_ke_partial(s, bm.y - lead + 1, ke, sh);
+    } else {
+        const bool        biased = lead > s.n_free_blocks;
+        __shared__ double bias[3];
+        __shared__ int    active;
+        if (bm.y < s.n_free_blocks) {
+            og_free_work(s, bm.y, e_ex, e_b);
+        } else {
+            og_vcmd_lambda(s, bias, active);
+            if (tid < 3) og_put(&s.sync->bias[tid], bias[tid]);
+            if (tid == 3) og_put(&s.sync->active, (double)active);
+        }
+        if (og_last_block(&s.sync->lead, lead)) {
+            const int nf = s.n_free;
+            if (biased) {
+                if (tid < 3) bias[tid] = og_take(&s.sync->bias[tid]);
+                const bool on = og_take(&s.sync->active) != 0.0;
+                __syncthreads();
+                if (on) og_vcmd_apply(s, bias);
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                __syncthreads();
+            }
+            for (int k = tid; k < nf; k += OG_WATER_THREADS) {
+                const int    i     = s.free_ids[k];
+                const double wk[3] = {og_take(&s.work[3 * i]), og_take(&s.work[3 * i + 1]), og_take(&s.work[3 * i + 2])};
+                og_langevin_atom(s, i, step, wk);
+            }
+            __syncthreads();
+            if (s.constraint) {
+                for (int t = tid; t < s.n_pairs_c; t += OG_WATER_THREADS) og_shake_pair(s, t);
+                __syncthreads();
+                for (int t = tid; t < s.n_trios; t += OG_WATER_THREADS)
+                    og_shake_trio(s, s.trio_ids[3 * t], s.trio_ids[3 * t + 1], s.trio_ids[3 * t + 2],
+                                  s.trio_d2 + 3 * t);
+                __syncthreads();
+            }
+            for (int k = tid; k < nf; k += OG_WATER_THREADS) ke += og_finish_atom(s, s.free_ids[k], step);
+            og_ke_partial(s, 0, ke, sh);
+        }
+    }
+    if (og_energy_step_c(s, c)) {
         __syncthreads();  // sh is reused
         og_add_misc_energies(s, bm.y, e_ex, e_b, sh);
     }
+    if (og_last_block(&s.sync->all, lead + s.n_water_blocks)) og_close_step(s, c, s.n_water_blocks + 1);
 }
 
 // One block per system, the step's last kernel.
@@ -771,7 +863,7 @@ __global__ void __launch_bounds__(OG_STEP_THREADS) k_step_close(const og_dev_sys
     // one batch of loads for the counters this kernel reads (a single block
     // runs per system, so every dependent round trip adds to the step)
     const og_dev_counters c = *s.cnt;
-    og_close_step(s, c);
+    og_close_step(s, c, s.n_ke_parts);
 }
 
 // ----------------------------------------------------------------- VcMD --
@@ -793,41 +885,51 @@ __global__ void __launch_bounds__(OG_STEP_THREADS) k_step_close(const og_dev_sys
 // V-AUS (mc_mode OG_MC_VAUS, ExtendedVAUS, Extend.cpp:366-540) takes the same
 // groups and lambda; its state moves first (og_mc_transition) and its force is
 // og_vaus_lane0's.
-// Called by every thread of a block (any size); bias and active live in LDS.
+// og_vcmd_lambda: the state, the reported terms and the bias (bias and active
+// in LDS), from the coordinates; og_vcmd_apply: the gradient of the group
+// atoms.  Called by every thread of a block of at most OG_THREADS.
 __device__ void og_vaus_lane0(const og_dev_sys &s, const double *diff, double lam, double *bias, int &active);
-__device__ void og_vcmd_block(const og_dev_sys &s, double *bias, int &active) {
+__device__ void og_vcmd_lambda(const og_dev_sys &s, double *bias, int &active) {
     const int lane = threadIdx.x, nt = blockDim.x;
     const int n    = s.vc_na + s.vc_nb;
-    for (int k = lane; k < n; k += nt) {
-        const int a = s.vc_atoms[k];
-        for (int d = 0; d < 3; d++) {
-            const double Lh   = (double)(s.L[d] * 0.5f);
-            double       tmp  = s.crd[3 * a + d];
-            double       diff = tmp - s.vc_crdg[3 * k + d];
-            while (diff > Lh) {
-                diff -= (double)s.L[d];
-                tmp -= (double)s.L[d];
+    // mass centres summed in group order, as the reference loop: a block's worth of products in LDS at a
+    // time, then a thread per direction (one thread that also loaded them took 3 us for 40 atoms)
+    __shared__ double prod[3][OG_THREADS], cen[2][3];
+    double            ca = 0.0, cb = 0.0;  // threads 0, 1, 2
+    for (int k0 = 0; k0 < n; k0 += nt) {
+        const int k = k0 + lane;
+        if (k < n) {
+            const int    a  = s.vc_atoms[k];
+            const double ms = (double)s.mass[a];
+            for (int d = 0; d < 3; d++) {
+                const double Lh   = (double)(s.L[d] * 0.5f);
+                double       tmp  = s.crd[3 * a + d];
+                double       diff = tmp - s.vc_crdg[3 * k + d];
+                while (diff > Lh) {
+                    diff -= (double)s.L[d];
+                    tmp -= (double)s.L[d];
+                }
+                while (-diff > Lh) {
+                    diff += (double)s.L[d];
+                    tmp += (double)s.L[d];
+                }
+                s.vc_crdg[3 * k + d] = tmp;
+                prod[d][lane]        = tmp * ms;
             }
-            while (-diff > Lh) {
-                diff += (double)s.L[d];
-                tmp += (double)s.L[d];
-            }
-            s.vc_crdg[3 * k + d] = tmp;
         }
+        __syncthreads();
+        if (lane < 3)
+            for (int j = 0; j < min(nt, n - k0); j++) {
+                if (k0 + j < s.vc_na) ca += prod[lane][j];
+                else cb += prod[lane][j];
+            }
+        __syncthreads();
     }
+    if (lane < 3) cen[0][lane] = ca, cen[1][lane] = cb;
     __syncthreads();
     if (lane == 0) {
-        // mass centres summed in group order, as the reference loop
-        double ca[3] = {0.0, 0.0, 0.0}, cb[3] = {0.0, 0.0, 0.0};
-        for (int k = 0; k < n; k++) {
-            const double ms = (double)s.mass[s.vc_atoms[k]];
-            for (int d = 0; d < 3; d++) {
-                if (k < s.vc_na) ca[d] += s.vc_crdg[3 * k + d] * ms;
-                else cb[d] += s.vc_crdg[3 * k + d] * ms;
-            }
-        }
         double diff[3];
-        for (int d = 0; d < 3; d++) diff[d] = og_mimg(ca[d] * s.vc_minv_a - cb[d] * s.vc_minv_b, s.L[d]);
+        for (int d = 0; d < 3; d++) diff[d] = og_mimg(cen[0][d] * s.vc_minv_a - cen[1][d] * s.vc_minv_b, s.L[d]);
         const double lam = sqrt(diff[0] * diff[0] + diff[1] * diff[1] + diff[2] * diff[2]);
         if (s.mc_mode == OG_MC_VAUS) {
             og_vaus_lane0(s, diff, lam, bias, active);
@@ -846,9 +948,9 @@ __device__ void og_vcmd_block(const og_dev_sys &s, double *bias, int &active) {
         for (int d = 0; d < 3; d++) bias[d] = diff[d] / lam;  // unit vector, scaled below
         for (int d = 0; d < 3; d++) bias[d] = dew * bias[d];
         active                = rec != 0.0;
-        s.energy[OG_E_EXTEND] = rec * ex;
-        s.energy[OG_E_LAMBDA] = lam;
-        s.energy[OG_E_VSTATE] = (double)vs;
+        og_put(&s.energy[OG_E_EXTEND], rec * ex);
+        og_put(&s.energy[OG_E_LAMBDA], lam);
+        og_put(&s.energy[OG_E_VSTATE], (double)vs);
         // visit count and transition trial
         const long long step     = s.cnt->step;
         const bool      in_range = lam >= lo && lam < hi;
@@ -872,14 +974,19 @@ __device__ void og_vcmd_block(const og_dev_sys &s, double *bias, int &active) {
         }
     }
     __syncthreads();
-    if (!active) return;
-    // gradient ("work") of the group atoms; the groups are disjoint
-    for (int k = lane; k < n; k += nt) {
+}
+// gradient ("work") of the group atoms; the groups are disjoint
+__device__ void og_vcmd_apply(const og_dev_sys &s, const double *bias) {
+    const int n = s.vc_na + s.vc_nb;
+    for (int k = threadIdx.x; k < n; k += blockDim.x) {
         const int    a    = s.vc_atoms[k];
         const bool   ga   = k < s.vc_na;
         const double minv = ga ? s.vc_minv_a : s.vc_minv_b;
         const double dir  = ga ? 1.0 : -1.0;
-        for (int d = 0; d < 3; d++) s.work[3 * a + d] += dir * (bias[d] * minv) * (double)s.mass[a];
+        for (int d = 0; d < 3; d++) {
+            double *w = &s.work[3 * a + d];
+            og_put(w, og_take(w) + dir * (bias[d] * minv) * (double)s.mass[a]);
+        }
     }
 }
 
@@ -943,9 +1050,9 @@ __device__ void og_vaus_lane0(const og_dev_sys &s, const double *diff, double la
     for (int d = 0; d < 3; d++) bias[d] = diff[d] / lam;
     for (int d = 0; d < 3; d++) bias[d] = dew * bias[d];
     active                = 1;
-    s.energy[OG_E_EXTEND] = 0.0;
-    s.energy[OG_E_LAMBDA] = lam;
-    s.energy[OG_E_VSTATE] = (double)vs;
+    og_put(&s.energy[OG_E_EXTEND], 0.0);
+    og_put(&s.energy[OG_E_LAMBDA], lam);
+    og_put(&s.energy[OG_E_VSTATE], (double)vs);
 }
 
 // V-McMD (ExtendedVMcMD::apply_bias + scale_force, Extend.cpp:126-200), one
@@ -975,9 +1082,9 @@ __global__ void __launch_bounds__(64) k_vmcmd(const og_dev_sys *__restrict__ S, 
     const double lo = s.mc_lo[vs], hi = s.mc_hi[vs];
     const double param = lam <= lo ? lo : (lam >= hi ? hi : lam);
     s.cnt->mc_scale       = s.mc_constk * og_mc_dlnp(s, vs, param);
-    s.energy[OG_E_EXTEND] = 0.0;
-    s.energy[OG_E_LAMBDA] = lam;
-    s.energy[OG_E_VSTATE] = (double)vs;
+    og_put(&s.energy[OG_E_EXTEND], 0.0);
+    og_put(&s.energy[OG_E_LAMBDA], lam);
+    og_put(&s.energy[OG_E_VSTATE], (double)vs);
 }
 __global__ void __launch_bounds__(OG_THREADS) k_vmcmd_scale(const og_dev_sys *__restrict__ S,
                                                             const int2 *__restrict__ map) {
@@ -1000,7 +1107,8 @@ __global__ void __launch_bounds__(64) k_vcmd(const og_dev_sys *__restrict__ S, c
     if (s.vc_n_states == 0 && s.mc_mode != OG_MC_VAUS) return;
     __shared__ double bias[3];
     __shared__ int    active;
-    og_vcmd_block(s, bias, active);
+    og_vcmd_lambda(s, bias, active);
+    if (active) og_vcmd_apply(s, bias);
 }
 
 // ------------------------------------------------------------- launchers --

@@ -84,6 +84,14 @@ struct og_dev_counters {
     double    mc_scale;    // V-McMD: the gradient factor of the current step
 };
 
+// Blocks of a fused step that have arrived (zero between launches; a line
+// each), and the bias its group block hands to the block that goes on.
+struct og_step_sync {
+    int    lead, pad0[31];
+    int    all, pad1[31];
+    double bias[3], active;
+};
+
 struct og_dev_sys {
     // ---- sizes ----
     int n_atoms;
@@ -97,6 +105,7 @@ struct og_dev_sys {
     int n_bterms;          // n_angles + n_torsions + n_impros + n_nb14: one thread each
     int n_quads;           // SHAKE four-atom groups
     int n_free;            // atoms outside SETTLE waters (fused Langevin step)
+    int n_free_blocks;     // fused Langevin step: blocks of OG_FREE_PER_BLOCK of them, at least one
     int n_water_blocks;    // fused Langevin step: blocks of OG_WATERS_PER_BLOCK waters; 0 = not fusable
     int pair_split;        // pair kernel: at most this many of the last cells run as two half-cell waves each
     int n_com_groups;
@@ -194,6 +203,7 @@ struct og_dev_sys {
     double *pairc_d2;
     int    *settle_ids;     // [n_settle*3]
     int    *free_ids;       // [n_free] atoms outside SETTLE waters
+    og_step_sync *sync;     // arrivals of the fused step's blocks
     int    *com_off, *com_atoms;   // COM-cancel groups
     float  *com_minv;
     // ---- grid ----
@@ -238,6 +248,11 @@ struct og_dev_sys {
     og_dev_counters *cnt;
 };
 
+// blocks of a fused step ahead of its water blocks: the free atoms' and the one that finds the groups' bias
+__host__ __device__ __forceinline__ int og_lead_blocks(const og_dev_sys &s) {
+    return s.n_free_blocks + (s.vc_n_states || s.mc_mode == OG_MC_VAUS ? 1 : 0);
+}
+
 // ---- block maps ----
 enum og_map_kind {
     OG_MAP_ATOM = 0,   // 256 threads per block over atoms
@@ -268,6 +283,7 @@ __host__ __device__ __forceinline__ int og_pair_split_cells(int split, int n_cel
 #define OG_WATER_THREADS 256  // fused Langevin step: threads per block
 #define OG_WATERS_PER_WAVE 21  // fused Langevin step: three lanes per water
 #define OG_WATERS_PER_BLOCK (OG_WATERS_PER_WAVE * (OG_WATER_THREADS / 64))
+#define OG_FREE_PER_BLOCK (OG_WATER_THREADS / 8)  // fused Langevin step: eight lanes per free atom
 #define OG_FREE_MAX 4096      // fused Langevin step: most atoms outside SETTLE waters (one block takes them)
 #define OG_CP_BLOCKS_PER_SYS_MIN 64
 
@@ -395,12 +411,36 @@ enum { OG_EACC_VDW, OG_EACC_ELE, OG_EACC_VIR, OG_EACC_PAIRS, OG_EACC_EXCESS, OG_
 // thread's loads in flight together), so each thread sums one term
 // (t % OG_EACC_STRIDE) over a share of the slots.
 #define OG_EACC_WORDS (OG_EACC_SLOTS * OG_EACC_STRIDE)
+// Values that blocks of one launch hand to each other: stored and loaded past
+// the caches that other blocks do not share.
+__device__ __forceinline__ void og_put(double *p, double v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double og_take(const double *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// True in every thread of the last of n blocks to arrive at ctr (it resets the
+// counter).  What a block handed over with og_put or an atomic add has reached
+// memory before its arrival counts.  No block waits for another.
+__device__ __forceinline__ bool og_last_block(int *ctr, int n) {
+    __shared__ int arrived;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        arrived = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (arrived == n - 1) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    return arrived == n - 1;
+}
+
 template <int NT>
 __device__ __forceinline__ long long og_eacc_load(const og_dev_sys &s) {
     static_assert(NT % 64 == 0 && NT <= 1024 && OG_EACC_WORDS % NT == 0, "block shape");
     long long w[OG_EACC_WORDS / NT];
 #pragma unroll
-    for (int k = 0; k < OG_EACC_WORDS / NT; k++) w[k] = s.e_acc[threadIdx.x + k * NT];
+    for (int k = 0; k < OG_EACC_WORDS / NT; k++)
+        w[k] = __hip_atomic_load(&s.e_acc[threadIdx.x + k * NT], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     long long v = 0;
 #pragma unroll
     for (int k = 0; k < OG_EACC_WORDS / NT; k++) v += w[k];

@@ -119,6 +119,17 @@ __device__ __forceinline__ double og_bond_pair(const og_dev_sys &s, double bk, d
     return coef * dif;
 }
 
+// Angles, torsions, impropers and 1-4 pairs: atom i's shares, written by
+// k_bonded earlier in the evaluation, added to w in ascending slot order.
+__device__ __forceinline__ void og_atom_work_bonded(const og_dev_sys &s, const int i, double *w) {
+    if (!s.n_bterms) return;
+    const int c0 = s.bc_off[i], c1 = s.bc_off[i + 1];
+    for (int e = c0; e < c1; e++) {
+        const double *c = s.bcontrib + 3 * (size_t)s.bc_at[e];
+        for (int k = 0; k < 3; k++) w[k] += c[k];
+    }
+}
+
 // Atom i: fixed-point pair gradient (grid slot) -> FP64 "work" in atom order
 // (SubBox::add_work_from_minicell, SubBox.cpp:1398-1407), plus the atom's
 // excluded-pair ZD terms (SubBox::calc_energy_ele_excess SubBox.cpp:1347-1367)
@@ -192,15 +203,7 @@ __device__ __forceinline__ void og_atom_work_calc(const og_dev_sys &s, const int
             bk = bn, r0 = rn, first = fn;
         }
     }
-    // angles, torsions, impropers and 1-4 pairs: the atom's shares, written
-    // by k_bonded earlier in the evaluation, in ascending slot order
-    if (s.n_bterms) {
-        const int c0 = s.bc_off[i], c1 = s.bc_off[i + 1];
-        for (int e = c0; e < c1; e++) {
-            const double *c = s.bcontrib + 3 * (size_t)s.bc_at[e];
-            for (int k = 0; k < 3; k++) w[k] += c[k];
-        }
-    }
+    og_atom_work_bonded(s, i, w);
 }
 
 // Stores atom i's work and clears its fixed-point accumulators for the next
