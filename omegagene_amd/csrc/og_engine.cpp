@@ -272,7 +272,8 @@ struct og_exec {
     bool                     any_vcmd = false, any_thermo = false;
     bool                     any_vmcmd = false;  // a member runs V-McMD
     bool                     any_bonded = false, any_quad = false;
-    bool                     fused = false;       // every member takes the fused Langevin step
+    bool                     fused = false;       // every member takes the fused step, in one form
+    int                      fused_form = 0;
     int                      pair_shape = OG_PAIR_DEFAULT;  // pair-kernel launch shape (KIND_PAIR + pair_shape)
     long long                cells = 0;           // cells of all members, at most a few per cent short
     int                      intvl = 1;
@@ -301,6 +302,12 @@ og_status exec_release(og_exec &x) {
 }
 
 // (re)build the descriptor array and block maps of an execution context
+int fused_form(const og_dev_sys &h) {
+    const bool shake = h.n_settle == 0;  // the waters are SHAKE trios
+    return h.integrator == 1 ? (shake ? OG_FUSED_LANGEVIN_SHAKE : OG_FUSED_LANGEVIN_SETTLE)
+                             : (shake ? OG_FUSED_LEAPFROG_SHAKE : OG_FUSED_LEAPFROG_SETTLE);
+}
+
 og_status exec_prepare(og_exec &x) {
     if (!x.dirty) return OG_OK;
     free_graphs(x);
@@ -342,7 +349,9 @@ og_status exec_prepare(og_exec &x) {
         x.any_thermo |= d.thermostat == OG_THERMOSTAT_SCALING;
         x.any_bonded |= d.n_bterms > 0;
         x.any_quad |= d.constraint != 0 && d.n_quads > 0;
-        x.fused &= d.integrator == 1 && d.n_water_blocks > 0;
+        const int form = fused_form(d);
+        if (si == 0) x.fused_form = form;
+        x.fused &= d.n_water_blocks > 0 && form == x.fused_form;
         x.cells += cdiv(d.n_atoms, OG_NAC);
         int       cnt[KIND_N];
         cnt[KIND_ATOM]  = cdiv(d.n_atoms, OG_THREADS);
@@ -469,7 +478,7 @@ void enqueue_forces(og_exec &x, hipEvent_t e0, hipEvent_t e1, bool point = false
 
 void enqueue_integrate(og_exec &x) {
     if (x.fused) {
-        og_launch_langevin_step(L(x, KIND_LSTEP));  // closes the step
+        og_launch_fused_step(L(x, KIND_LSTEP), x.fused_form);
         return;
     }
     // the extended-ensemble bias acts on the gradient of the step
@@ -849,7 +858,7 @@ og_status sys_alloc(og_system *s, const og_system_desc *d, const og_params *p) {
     if (h.n_quads && !(A(&h.quad_ids, 4 * (size_t)h.n_quads) && A(&h.quad_d2, 6 * (size_t)h.n_quads)))
         return OG_E_DEVICE;
     h.n_atom_blocks = cdiv(n, OG_THREADS);
-    h.n_ke_parts    = std::max(h.n_atom_blocks, cdiv(h.n_settle, OG_WATERS_PER_BLOCK) + 1);
+    h.n_ke_parts    = std::max(h.n_atom_blocks, cdiv(std::max(h.n_settle, h.n_trios), OG_WATERS_PER_BLOCK) + 1);
     if (h.thermostat == OG_THERMOSTAT_SCALING && !A(&h.th_part, h.n_atom_blocks)) return OG_E_DEVICE;
     ok = A(&h.e_atom, std::max(h.n_ke_parts, 1)) &&
          A(&h.com_mom, 3 * (size_t)(h.n_com_groups + 1)) && A(&h.energy, OG_E_NTERMS) &&
@@ -1000,54 +1009,84 @@ og_status sys_alloc(og_system *s, const og_system_desc *d, const og_params *p) {
         OG_HIP(hipMemcpy(h.quad_ids, d->shake_quad_ids, sizeof(int) * 4 * h.n_quads, hipMemcpyHostToDevice));
         OG_HIP(hipMemcpy(h.quad_d2, d->shake_quad_d2, sizeof(double) * 6 * h.n_quads, hipMemcpyHostToDevice));
     }
-    if (h.n_trios) {
-        OG_HIP(hipMemcpy(h.trio_ids, d->shake_trio_ids, sizeof(int) * 3 * h.n_trios, hipMemcpyHostToDevice));
-        OG_HIP(hipMemcpy(h.trio_d2, d->shake_trio_d2, sizeof(double) * 3 * h.n_trios, hipMemcpyHostToDevice));
-    }
     if (h.n_pairs_c) {
         OG_HIP(hipMemcpy(h.pairc_ids, d->shake_pair_ids, sizeof(int) * 2 * h.n_pairs_c, hipMemcpyHostToDevice));
         OG_HIP(hipMemcpy(h.pairc_d2, d->shake_pair_d2, sizeof(double) * h.n_pairs_c, hipMemcpyHostToDevice));
     }
     if (h.n_settle) OG_HIP(hipMemcpy(h.settle_ids, d->settle_ids, sizeof(int) * 3 * h.n_settle, hipMemcpyHostToDevice));
-    // The fused Langevin step (one kernel per MD step after the pair kernel)
-    // takes SETTLE waters one per thread, so each water must interact with no
-    // other atom through exclusions and carry no bond, SHAKE or VcMD group;
-    // the other atoms (at most OG_FREE_MAX) go through one block.
-    h.n_free         = 0;
-    h.n_water_blocks = 0;
-    if (h.integrator == 1 && h.n_settle > 0 && !p->split_step) {
-        std::vector<int> water(n, -1);
-        bool             fuse = true;
-        for (int t = 0; t < h.n_settle && fuse; t++)
-            for (int k = 0; k < 3 && fuse; k++) {
-                int &w = water[d->settle_ids[3 * t + k]];
-                fuse   = w < 0;
-                w      = t;
-            }
-        auto outside = [&](const int *ids, long long cnt) {
-            for (long long k = 0; k < cnt; k++)
-                if (water[ids[k]] >= 0) return false;
-            return true;
+    // The fused step (one kernel per MD step after the pair kernel) takes
+    // waters three lanes each, so each water must interact with no other atom
+    // through exclusions and carry no bond, VcMD group or other constraint;
+    // the other atoms (at most OG_FREE_MAX) go through one block.  Its waters
+    // are the SETTLE waters (all of them, or the step is not fused) or, with
+    // none, the SHAKE trios that qualify, which are moved to the end of the
+    // trio list (the trios are independent of each other).
+    h.n_free = h.n_free_blocks = h.n_waters = h.n_water_blocks = 0;
+    h.n_free_trios = h.n_trios;
+    std::vector<int>    trio_ids(d->shake_trio_ids, d->shake_trio_ids + 3 * (size_t)h.n_trios);
+    std::vector<double> trio_d2(d->shake_trio_d2, d->shake_trio_d2 + 3 * (size_t)h.n_trios);
+    const bool          steps = h.integrator == 1 || (h.thermostat == OG_THERMOSTAT_NONE && !h.com_cancel);
+    if (steps && h.constraint && (h.n_settle || h.n_trios) && !p->split_step &&
+        h.n_quads == 0) {  // the step kernel runs no four-atom SHAKE
+        const bool       settle = h.n_settle > 0;
+        const int        nt     = settle ? h.n_settle : h.n_trios;
+        const int       *ids    = settle ? d->settle_ids : d->shake_trio_ids;
+        std::vector<int> water(n, -1);  // the atom's water
+        std::vector<char> good(nt, 1);  // which of them qualify
+        auto              drop = [&](int a) {
+            if (water[a] >= 0) good[water[a]] = 0;
         };
-        for (int t = 0; t < h.n_excess && fuse; t++) fuse = water[d->excess[2 * t]] == water[d->excess[2 * t + 1]];
-        fuse = fuse && outside(d->bond_ids, 2LL * h.n_bonds) && outside(d->shake_pair_ids, 2LL * h.n_pairs_c) &&
-               outside(d->shake_trio_ids, 3LL * h.n_trios) && outside(d->vc_atoms_a, h.vc_na) &&
-               outside(d->vc_atoms_b, h.vc_nb) && outside(d->angle_ids, 3LL * h.n_angles) &&
-               outside(d->torsion_ids, 4LL * h.n_torsions) && outside(d->impro_ids, 4LL * h.n_impros) &&
-               outside(d->nb14_ids, 2LL * h.n_nb14) && h.n_quads == 0;  // the step kernel runs no four-atom SHAKE
+        for (int t = 0; t < nt; t++)
+            for (int k = 0; k < 3; k++) {
+                int &w = water[ids[3 * t + k]];
+                if (w >= 0) good[w] = good[t] = 0;  // an atom of two waters, or twice of one
+                w = t;
+            }
+        auto drop_all = [&](const int *at, long long cnt) {
+            for (long long k = 0; k < cnt; k++) drop(at[k]);
+        };
+        for (int e = 0; e < h.n_excess; e++)
+            if (water[d->excess[2 * e]] != water[d->excess[2 * e + 1]]) drop(d->excess[2 * e]), drop(d->excess[2 * e + 1]);
+        drop_all(d->bond_ids, 2LL * h.n_bonds);
+        drop_all(d->shake_pair_ids, 2LL * h.n_pairs_c);
+        if (settle) drop_all(d->shake_trio_ids, 3LL * h.n_trios);
+        drop_all(d->vc_atoms_a, h.vc_na);
+        drop_all(d->vc_atoms_b, h.vc_nb);
+        drop_all(d->angle_ids, 3LL * h.n_angles);
+        drop_all(d->torsion_ids, 4LL * h.n_torsions);
+        drop_all(d->impro_ids, 4LL * h.n_impros);
+        drop_all(d->nb14_ids, 2LL * h.n_nb14);
+        const int nw = (int)std::count(good.begin(), good.end(), 1);
         std::vector<int> free_ids;
-        for (int i = 0; i < n && fuse; i++)
-            if (water[i] < 0) free_ids.push_back(i);
-        const int nwb = cdiv(h.n_settle, OG_WATERS_PER_BLOCK);
-        if (fuse && (int)free_ids.size() <= OG_FREE_MAX) {
-            if (!A(&h.free_ids, std::max<size_t>(free_ids.size(), 1))) return OG_E_DEVICE;
+        for (int i = 0; i < n; i++)
+            if (water[i] < 0 || !good[water[i]]) free_ids.push_back(i);
+        if (nw > 0 && (nw == nt || !settle) && (int)free_ids.size() <= OG_FREE_MAX) {
+            if (!A(&h.free_ids, std::max<size_t>(free_ids.size(), 1)) || !A(&h.sync, 1)) return OG_E_DEVICE;
             if (!free_ids.empty())
                 OG_HIP(hipMemcpy(h.free_ids, free_ids.data(), sizeof(int) * free_ids.size(), hipMemcpyHostToDevice));
-            if (!A(&h.sync, 1)) return OG_E_DEVICE;
             h.n_free         = (int)free_ids.size();
             h.n_free_blocks  = std::max(1, cdiv(h.n_free, OG_FREE_PER_BLOCK));
-            h.n_water_blocks = nwb;
+            h.n_waters       = nw;
+            h.n_water_blocks = cdiv(nw, OG_WATERS_PER_BLOCK);
+            h.water_ids      = h.settle_ids;
+            if (!settle) {
+                size_t at = 0;
+                for (int pass = 0; pass < 2; pass++)  // the other trios, then the waters
+                    for (int t = 0; t < nt; t++)
+                        if (good[t] == pass) {
+                            std::copy_n(d->shake_trio_ids + 3 * (size_t)t, 3, trio_ids.begin() + at);
+                            std::copy_n(d->shake_trio_d2 + 3 * (size_t)t, 3, trio_d2.begin() + at);
+                            at += 3;
+                        }
+                h.n_free_trios = nt - nw;
+                h.water_ids    = h.trio_ids + 3 * (size_t)h.n_free_trios;
+                h.water_d2     = h.trio_d2 + 3 * (size_t)h.n_free_trios;
+            }
         }
+    }
+    if (h.n_trios) {
+        OG_HIP(hipMemcpy(h.trio_ids, trio_ids.data(), sizeof(int) * trio_ids.size(), hipMemcpyHostToDevice));
+        OG_HIP(hipMemcpy(h.trio_d2, trio_d2.data(), sizeof(double) * trio_d2.size(), hipMemcpyHostToDevice));
     }
     if (h.n_com_groups) {
         const int ng = h.n_com_groups;
@@ -1299,7 +1338,7 @@ og_status og_system_footprint(const og_system_desc *d, const og_params *p, uint6
     const double settle = p->constraint == OG_CONSTRAINT_SHAKE_SETTLE ? d->n_settle : 0;
     const double ng = p->com_cancel ? d->n_com_groups : 0;
     const double ng_atoms = ng > 0 ? d->com_group_off[d->n_com_groups] : 1;
-    const double ke_parts = std::max(std::ceil(n / OG_THREADS), std::floor(settle / OG_WATERS_PER_BLOCK) + 2);
+    const double ke_parts = std::max(std::ceil(n / OG_THREADS), std::floor(std::max(settle, trios) / OG_WATERS_PER_BLOCK) + 2);
     const double vc = (d->vc_n_states || d->mc_mode == OG_EXT_VAUS) ? d->vc_n_a + d->vc_n_b : 0, vs = d->vc_n_states;
     const double mcs = d->mc_mode ? d->mc_n_states : 0;
     const double log_rows = std::max(1, p->log_cap);
@@ -1826,7 +1865,7 @@ og_status og_system_device_bytes(og_system *s, uint64_t *bytes) {
 
 og_status og_step_fused(og_system *s, int *fused) {
     if (!s || !fused) return OG_E_ARG;
-    *fused = s->h.integrator == 1 && s->h.n_water_blocks > 0;
+    *fused = s->h.n_water_blocks > 0 && fused_form(s->h) == OG_FUSED_LANGEVIN_SETTLE;
     return OG_OK;
 }
 

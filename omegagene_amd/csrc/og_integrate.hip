@@ -36,7 +36,12 @@ __device__ __forceinline__ double2 og_gauss2(uint32_t a, uint32_t b) {
 }
 
 // --------------------------------------------------- leapfrog velocities --
-// SubBox::cpy_vel_prev + update_velocities (SubBox.cpp:1427-1454)
+// SubBox::cpy_vel_prev + update_velocities (SubBox.cpp:1427-1454): the
+// velocity after the step from v before it and the gradient component wk.
+__device__ __forceinline__ double og_leapfrog_vel(const og_dev_sys &s, const double v, const double wk,
+                                                  const double minv) {
+    return v + (((s.dt * -OG_FORCE_VEL) * wk) * minv);
+}
 __global__ void __launch_bounds__(OG_THREADS) k_leapfrog_vel(const og_dev_sys *__restrict__ S,
                                                              const int2 *__restrict__ map) {
     const int2        bm = map[blockIdx.x];
@@ -48,7 +53,7 @@ __global__ void __launch_bounds__(OG_THREADS) k_leapfrog_vel(const og_dev_sys *_
     for (int d = 0; d < 3; d++) {
         const double v    = s.vel_next[3 * i + d];
         s.vel[3 * i + d]  = v;
-        s.vel_next[3 * i + d] = v + (((s.dt * -OG_FORCE_VEL) * s.work[3 * i + d]) * minv);
+        s.vel_next[3 * i + d] = og_leapfrog_vel(s, v, s.work[3 * i + d], minv);
     }
 }
 
@@ -172,6 +177,20 @@ __global__ void __launch_bounds__(OG_THREADS) k_positions(const og_dev_sys *__re
     }
 }
 
+// One atom's leapfrog velocity and position with gradient wk.
+__device__ __forceinline__ void og_leapfrog_atom(const og_dev_sys &s, const int i, const double *wk) {
+    const double minv = (double)s.mass_inv[i];
+    for (int d = 0; d < 3; d++) {
+        const double v = s.vel_next[3 * i + d], x = s.crd[3 * i + d];
+        const double vn = og_leapfrog_vel(s, v, wk[d], minv);
+        s.vel[3 * i + d]      = v;
+        s.vel_next[3 * i + d] = vn;
+        s.crd_prev[3 * i + d] = x;
+        const double diff     = vn * s.dt;
+        s.crd[3 * i + d]      = x + diff;
+    }
+}
+
 // ----------------------------------------------------- Langevin positions --
 // DynamicsModeLangevin::calc_in_each_step (DynamicsMode.cpp:798-899):
 // crd_prev2 <- crd_prev <- crd; first step x1 = x0 + dt v0; later steps
@@ -272,20 +291,24 @@ __global__ void __launch_bounds__(OG_THREADS) k_shake_pair(const og_dev_sys *__r
     og_shake_pair(s, t);
 }
 
-// ConstraintShake::shake_trio (ConstraintShake.cpp:51-149), one thread per trio.
-// inlined: as a called function it takes 248 VGPRs, which would set every caller's count
-__device__ __forceinline__ void og_shake_trio(const og_dev_sys &s, int a1, int a2, int a3, const double *D) {
+// ConstraintShake::shake_trio (ConstraintShake.cpp:51-149).  Core on values:
+// x1..x3 unconstrained, p1..p3 previous positions, inverse masses m1..m3,
+// squared lengths D; M holds what each atom's position is to be moved by.
+// Returns false (M set all the same) when the loop did not converge.
+__device__ __forceinline__ bool og_shake_core(const og_dev_sys &s, const double *x1, const double *x2,
+                                              const double *x3, const double *p1, const double *p2, const double *p3,
+                                              const double m1, const double m2, const double m3, const double *D,
+                                              double (*M)[3]) {
     double d12[3], d23[3], d31[3], p12[3], p23[3], p31[3];
     double g[6] = {0, 0, 0, 0, 0, 0};
     for (int k = 0; k < 3; k++) {
-        d12[k] = og_mimg(s.crd[3 * a1 + k] - s.crd[3 * a2 + k], s.L[k]);
-        p12[k] = og_mimg(s.crd_prev[3 * a1 + k] - s.crd_prev[3 * a2 + k], s.L[k]);
-        d23[k] = og_mimg(s.crd[3 * a2 + k] - s.crd[3 * a3 + k], s.L[k]);
-        p23[k] = og_mimg(s.crd_prev[3 * a2 + k] - s.crd_prev[3 * a3 + k], s.L[k]);
-        d31[k] = og_mimg(s.crd[3 * a3 + k] - s.crd[3 * a1 + k], s.L[k]);
-        p31[k] = og_mimg(s.crd_prev[3 * a3 + k] - s.crd_prev[3 * a1 + k], s.L[k]);
+        d12[k] = og_mimg(x1[k] - x2[k], s.L[k]);
+        p12[k] = og_mimg(p1[k] - p2[k], s.L[k]);
+        d23[k] = og_mimg(x2[k] - x3[k], s.L[k]);
+        p23[k] = og_mimg(p2[k] - p3[k], s.L[k]);
+        d31[k] = og_mimg(x3[k] - x1[k], s.L[k]);
+        p31[k] = og_mimg(p3[k] - p1[k], s.L[k]);
     }
-    const double m1 = s.mass_inv[a1], m2 = s.mass_inv[a2], m3 = s.mass_inv[a3];
     const double c11 = m1 + m2, c12 = -m2, c13 = -m1;
     const double c21 = -m2, c22 = m2 + m3, c23 = -m3;
     const double c31 = -m1, c32 = -m3, c33 = m3 + m1;
@@ -321,12 +344,26 @@ __device__ __forceinline__ void og_shake_trio(const og_dev_sys &s, int a1, int a
         g[4] += g[1];
         g[5] += g[2];
     }
-    if (!conv) atomicAdd(&s.cnt->shake_fail, 1);
     for (int k = 0; k < 3; k++) {
-        s.crd[3 * a1 + k] += m1 * (g[3] * p12[k] - g[5] * p31[k]);
-        s.crd[3 * a2 + k] += m2 * (-g[3] * p12[k] + g[4] * p23[k]);
-        s.crd[3 * a3 + k] += m3 * (-g[4] * p23[k] + g[5] * p31[k]);
+        M[0][k] = m1 * (g[3] * p12[k] - g[5] * p31[k]);
+        M[1][k] = m2 * (-g[3] * p12[k] + g[4] * p23[k]);
+        M[2][k] = m3 * (-g[4] * p23[k] + g[5] * p31[k]);
     }
+    return conv;
+}
+// One thread per trio.  Inlined: as a called function it takes 248 VGPRs, which would set every caller's count.
+__device__ __forceinline__ void og_shake_trio(const og_dev_sys &s, int a1, int a2, int a3, const double *D) {
+    double    x[3][3], p[3][3], M[3][3];
+    const int a[3] = {a1, a2, a3};
+    for (int j = 0; j < 3; j++)
+        for (int k = 0; k < 3; k++) {
+            x[j][k] = s.crd[3 * a[j] + k];
+            p[j][k] = s.crd_prev[3 * a[j] + k];
+        }
+    if (!og_shake_core(s, x[0], x[1], x[2], p[0], p[1], p[2], s.mass_inv[a1], s.mass_inv[a2], s.mass_inv[a3], D, M))
+        atomicAdd(&s.cnt->shake_fail, 1);
+    for (int j = 0; j < 3; j++)
+        for (int k = 0; k < 3; k++) s.crd[3 * a[j] + k] += M[j][k];  // read again: the positions are not held through the loop
 }
 
 // Analytic SETTLE (S. Miyamoto, P. A. Kollman, J. Comput. Chem. 13 (1992) 952-962)
@@ -573,49 +610,55 @@ __device__ __forceinline__ void og_close_step(const og_dev_sys &s, const og_dev_
             if (k + j * OG_STEP_THREADS < n_parts) t += v[j];
     }
     // read with the partials, before the counters are known (one memory
-    // round trip less): the accumulator slots and, in thread 0, the energy
-    // row, whose pair, excluded-pair, bonded and kinetic terms this kernel
-    // replaces (the others come from earlier kernels of the step)
+    // round trip less): the accumulator slots and, in thread k, term k of the
+    // energy row, whose pair, excluded-pair, bonded and kinetic terms this
+    // kernel replaces (the others come from earlier kernels of the step)
     const long long ev = og_eacc_load<OG_STEP_THREADS>(s);
-    double row[OG_E_NTERMS];
-    if (threadIdx.x == 0)
-        for (int k = 0; k < OG_E_NTERMS; k++) row[k] = og_take(&s.energy[k]);
+    const int       k  = threadIdx.x;
+    double          e  = k < OG_E_NTERMS ? og_take(&s.energy[k]) : 0.0;
     if (og_frozen_c(c)) return;
     __shared__ double    sh[OG_STEP_THREADS / 64];
     __shared__ long long she[16 * OG_EACC_STRIDE];
-    if (og_energy_step_c(s, c)) {
-        og_eacc_clear<OG_STEP_THREADS>(s);
-        og_eacc_reduce<OG_STEP_THREADS>(s, ev, she, row);
-    }
     for (int off = 32; off > 0; off >>= 1) t += __shfl_down(t, off, 64);
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = t;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double ke = 0.0;
-        for (int w = 0; w < OG_STEP_THREADS / 64; w++) ke += sh[w];
-        row[OG_E_KIN]       = ke * OG_KINETIC_COEFF;
-        s.energy[OG_E_KIN]  = row[OG_E_KIN];
-        const long long stp = c.step;
-        if (s.log_cap > 0 && (stp % s.log_stride) == 0) {
-            double *e = s.elog + (size_t)((stp / s.log_stride) % s.log_cap) * OG_E_NTERMS;
-            for (int k = 0; k < OG_E_NTERMS; k++) e[k] = row[k];
+    bool fresh = false;
+    if (og_energy_step_c(s, c)) {
+        og_eacc_clear<OG_STEP_THREADS>(s);
+        fresh = og_eacc_term<OG_STEP_THREADS>(s, ev, she, e);
+    } else {
+        __syncthreads();
+    }
+    const long long stp = c.step;
+    if (k < OG_E_NTERMS) {
+        if (k == OG_E_KIN) {
+            double ke = 0.0;
+            for (int w = 0; w < OG_STEP_THREADS / 64; w++) ke += sh[w];
+            e     = ke * OG_KINETIC_COEFF;
+            fresh = true;
         }
+        if (fresh) s.energy[k] = e;
+        if (s.log_cap > 0 && og_step_mod(stp, s.log_stride) == 0)
+            s.elog[(size_t)og_step_mod(og_step_div(stp, s.log_stride), s.log_cap) * OG_E_NTERMS + k] = e;
+    }
+    if (k == 0) {
         s.cnt->rebuild_now = 0;
         s.cnt->step        = stp + 1;
     }
 }
 
-// ------------------------------------------------- fused Langevin step --
-// One launch for the whole integration step of a Langevin system whose
-// SETTLE waters interact with nothing but their own atoms through exclusions
-// and carry no bonds, VcMD groups or SHAKE groups:
+// ---------------------------------------------------------- fused step --
+// One launch for the whole integration step of a Langevin or leapfrog system
+// whose waters (SETTLE waters, or without any the SHAKE trios like them)
+// interact with nothing but their own atoms through exclusions and carry no
+// bonds, VcMD groups or other constraints; a leapfrog step has no thermostat
+// or COM removal, which need all velocities first:
 //  * the lead blocks of a system convert the gradient of every other ("free")
 //    atom, eight lanes per atom (og_free_work), and one more block finds the
 //    VcMD / V-AUS bias, which needs no gradient; the last of them to arrive
-//    takes the free atoms on -- bias, Langevin positions, SHAKE pairs then
+//    takes the free atoms on -- bias, positions, SHAKE pairs then
 //    trios, finish -- with a block barrier between the stages;
 //  * the other blocks take the waters, three lanes per water
-//    (og_water_lanes): gradient conversion, Langevin positions, SETTLE and
+//    (og_water_lanes): gradient conversion, positions, SETTLE or SHAKE and
 //    finish;
 //  * the last block to arrive closes the step (og_close_step).
 // Each atom goes through the same device functions, in the same order, as in
@@ -627,13 +670,15 @@ __device__ __forceinline__ void og_close_step(const og_dev_sys &s, const og_dev_
 // A launch of one walker is latency: one block for all free atoms took 17.3 us
 // of it (13,481 atoms, 200 of them free; a wave alone on its SIMD issues one
 // instruction per 8 cycles) against 11.5 for the water blocks, and a closing
-// kernel of its own 4.8.
-// SETTLE waters of the fused Langevin step, three lanes per water (lane
+// kernel of its own 4.8.  The leapfrog step of a SHAKE water box was six
+// kernels of 33 us together (6,000 atoms), now 14.3.
+// Waters of the fused step, three lanes per water (lane
 // 3k + a holds atom a of the wave's water k; lane 63 is an idle copy): each
 // lane loads its atom, takes the other two atoms' positions by shuffles for
-// the excluded pairs and for SETTLE (solved identically in all three lanes),
+// the excluded pairs and for SETTLE or SHAKE (solved identically in all three lanes),
 // runs the value cores shared with the separate kernels and stores its atom
 // once.  e_ex and ke collect the lane's contributions.
+template <bool LEAP, bool SHAKE>
 __device__ __forceinline__ void og_water_lanes(const og_dev_sys &s, const int blk, const long long step,
                                                double &e_ex, double &ke) {
     const int  lane = threadIdx.x & 63;
@@ -641,11 +686,11 @@ __device__ __forceinline__ void og_water_lanes(const og_dev_sys &s, const int bl
     const int  ac   = min(lane - 3 * grp, 2);
     const int  base = 3 * grp;
     const int  tr   = blk * OG_WATERS_PER_BLOCK + (threadIdx.x >> 6) * OG_WATERS_PER_WAVE + grp;
-    const bool live = lane < 3 * OG_WATERS_PER_WAVE && tr < s.n_settle;
-    const int  t    = min(tr, s.n_settle - 1);
+    const bool live = lane < 3 * OG_WATERS_PER_WAVE && tr < s.n_waters;
+    const int  t    = min(tr, s.n_waters - 1);
     const int  cap  = s.cap_atom_array;
     int        ia[3];
-    for (int k = 0; k < 3; k++) ia[k] = s.settle_ids[3 * t + k];
+    for (int k = 0; k < 3; k++) ia[k] = s.water_ids[3 * t + k];
     const int   i  = ia[ac];
     const int   g  = s.rev[i];
     const int   e0 = s.exc_off[i], e1 = s.exc_off[i + 1];
@@ -655,8 +700,8 @@ __device__ __forceinline__ void og_water_lanes(const og_dev_sys &s, const int bl
     double      x[3], xp[3], vn[3], w[3], gc[3];
     for (int d = 0; d < 3; d++) {
         x[d]  = s.crd[3 * i + d];
-        xp[d] = s.crd_prev[3 * i + d];
-        vn[d] = step == 0 ? s.vel_next[3 * i + d] : 0.0;
+        xp[d] = LEAP ? 0.0 : s.crd_prev[3 * i + d];
+        vn[d] = LEAP || step == 0 ? s.vel_next[3 * i + d] : 0.0;
         gc[d] = s.gcrd[3 * g + d];
     }
     og_fx_read(s.fx, cap, og_fx_slot(g), w);
@@ -689,13 +734,20 @@ __device__ __forceinline__ void og_water_lanes(const og_dev_sys &s, const int bl
         e_ex += own && live ? (double)ene : 0.0;
     }
     double xn[3];
-    og_langevin_core(s, i, step, x, xp, vn, w, (double)m, (double)mi, xn);
-    // what is final goes out here: fewer registers are held through SETTLE
+    if (LEAP) {
+        for (int d = 0; d < 3; d++) {
+            const double diff = og_leapfrog_vel(s, vn[d], w[d], (double)mi) * s.dt;
+            xn[d]             = x[d] + diff;
+        }
+    } else {
+        og_langevin_core(s, i, step, x, xp, vn, w, (double)m, (double)mi, xn);
+    }
+    // what is final goes out here: fewer registers are held through the constraint
     if (live) {
         og_fx_consume(s.fx, cap, og_fx_slot(g));
         for (int d = 0; d < 3; d++) {
             s.work[3 * i + d]      = w[d];
-            s.crd_prev2[3 * i + d] = xp[d];
+            if (!LEAP) s.crd_prev2[3 * i + d] = xp[d];
             s.crd_prev[3 * i + d]  = x[d];
         }
     }
@@ -705,21 +757,38 @@ __device__ __forceinline__ void og_water_lanes(const og_dev_sys &s, const int bl
         double XN[3][3];
         for (int k = 0; k < 3; k++)
             for (int d = 0; d < 3; d++) XN[k][d] = __shfl(xn[d], base + k, 64);
-        const double mO = __shfl((double)m, base, 64), mH = __shfl((double)m, base + 1, 64);
-        ok = og_settle_core(s, mO, mH, s.settle_dOH, s.settle_dHH, XN[0], XN[1], XN[2], X[0], X[1], X[2], D);
+        if (SHAKE) {
+            const double d2[3] = {s.water_d2[3 * t], s.water_d2[3 * t + 1], s.water_d2[3 * t + 2]};
+            ok = og_shake_core(s, XN[0], XN[1], XN[2], X[0], X[1], X[2], __shfl(mi, base, 64), __shfl(mi, base + 1, 64),
+                               __shfl(mi, base + 2, 64), d2, D);
+        } else {
+            const double mO = __shfl((double)m, base, 64), mH = __shfl((double)m, base + 1, 64);
+            ok = og_settle_core(s, mO, mH, s.settle_dOH, s.settle_dHH, XN[0], XN[1], XN[2], X[0], X[1], X[2], D);
+        }
     }
     if (!ok && live && ac == 0) atomicAdd(&s.cnt->shake_fail, 1);
-    if (ok)
+    if (SHAKE || ok)
         for (int d = 0; d < 3; d++) xn[d] += ac == 0 ? D[0][d] : ac == 1 ? D[1][d] : D[2][d];
     double v[3], xw[3];
     float  f[3];
-    const double ka = og_langevin_vel(s, step, xn, xp, vn, v);
+    double ka = 0.0;
+    if (LEAP) {  // the velocity from the constrained positions (og_finish_atom)
+        const double dt_inv = 1.0 / s.dt;
+        for (int d = 0; d < 3; d++) {
+            v[d]            = (xn[d] - x[d]) * dt_inv;
+            const double vj = (vn[d] + v[d]) * 0.5;
+            ka += vj * vj;
+        }
+    } else {
+        ka = og_langevin_vel(s, step, xn, xp, vn, v);
+    }
     og_advance(s, xn, x, gc, f, xw);
     if (!live) return;
     ke += ka * (double)m;
     for (int d = 0; d < 3; d++) {
         s.crd[3 * i + d]  = xw[d];
-        s.vel[3 * i + d]  = step == 0 ? vn[d] : v[d];
+        s.vel[3 * i + d]  = LEAP || step == 0 ? vn[d] : v[d];
+        if (LEAP) s.vel_next[3 * i + d] = v[d];
         s.gcrd[3 * g + d] = gc[d];
     }
     s.gxyzq[g] = make_float4(f[0], f[1], f[2], gw);
@@ -796,8 +865,9 @@ __device__ void og_vcmd_apply(const og_dev_sys &s, const double *bias);
 // Three waves per SIMD (168 registers): left free the kernel takes 203 (two
 // waves), held to 128 it spills (450,000 atoms 430 / 421 / 429 us per step at
 // two / three / four waves, sixteen walkers 303 / 297 / 299).
-__global__ void __launch_bounds__(OG_WATER_THREADS, 3) k_langevin_step(const og_dev_sys *__restrict__ S,
-                                                                       const int2 *__restrict__ map) {
+template <bool LEAP, bool SHAKE>
+__global__ void __launch_bounds__(OG_WATER_THREADS, 3) k_fused_step(const og_dev_sys *__restrict__ S,
+                                                                    const int2 *__restrict__ map) {
     const int2            bm = map[blockIdx.x];
     const og_dev_sys     &s  = S[bm.x];
     const og_dev_counters c  = *s.cnt;
@@ -808,7 +878,7 @@ __global__ void __launch_bounds__(OG_WATER_THREADS, 3) k_langevin_step(const og_
     double            e_ex = 0.0, e_b = 0.0, ke = 0.0;
     __shared__ double sh[2 * (OG_WATER_THREADS / 64)];
     if (bm.y >= lead) {
-        og_water_lanes(s, bm.y - lead, step, e_ex, ke);
+        og_water_lanes<LEAP, SHAKE>(s, bm.y - lead, step, e_ex, ke);
         og_ke_partial(s, bm.y - lead + 1, ke, sh);
     } else {
         const bool        biased = lead > s.n_free_blocks;
@@ -834,13 +904,14 @@ __global__ void __launch_bounds__(OG_WATER_THREADS, 3) k_langevin_step(const og_
             for (int k = tid; k < nf; k += OG_WATER_THREADS) {
                 const int    i     = s.free_ids[k];
                 const double wk[3] = {og_take(&s.work[3 * i]), og_take(&s.work[3 * i + 1]), og_take(&s.work[3 * i + 2])};
-                og_langevin_atom(s, i, step, wk);
+                if (LEAP) og_leapfrog_atom(s, i, wk);
+                else og_langevin_atom(s, i, step, wk);
             }
             __syncthreads();
             if (s.constraint) {
                 for (int t = tid; t < s.n_pairs_c; t += OG_WATER_THREADS) og_shake_pair(s, t);
                 __syncthreads();
-                for (int t = tid; t < s.n_trios; t += OG_WATER_THREADS)
+                for (int t = tid; t < s.n_free_trios; t += OG_WATER_THREADS)
                     og_shake_trio(s, s.trio_ids[3 * t], s.trio_ids[3 * t + 1], s.trio_ids[3 * t + 2],
                                   s.trio_d2 + 3 * t);
                 __syncthreads();
@@ -955,7 +1026,7 @@ __device__ void og_vcmd_lambda(const og_dev_sys &s, double *bias, int &active) {
         const long long step     = s.cnt->step;
         const bool      in_range = lam >= lo && lam < hi;
         if (in_range) s.vc_hist[vs] += 1.0;
-        if (step > 0 && step % s.vc_interval == 0 && in_range) {
+        if (step > 0 && og_step_mod(step, s.vc_interval) == 0 && in_range) {
             int cand[2] = {vs, -1};
             if (vs > 0) {
                 if (lam < s.vc_hi[vs - 1]) cand[1] = vs - 1;
@@ -1033,7 +1104,7 @@ __device__ double og_mc_dlnp(const og_dev_sys &s, int vs, double param) {
 __device__ void og_vaus_lane0(const og_dev_sys &s, const double *diff, double lam, double *bias, int &active) {
     const long long step = s.cnt->step;
     int             vs   = s.cnt->vs;
-    if (step > 0 && step % s.mc_interval == 0) {
+    if (step > 0 && og_step_mod(step, s.mc_interval) == 0) {
         vs        = og_mc_transition(s, vs, lam, step);
         s.cnt->vs = vs;
     }
@@ -1075,7 +1146,7 @@ __global__ void __launch_bounds__(64) k_vmcmd(const og_dev_sys *__restrict__ S, 
     const double    lam  = (double)v * OG_FX_INV + s.e_self;
     const long long step = s.cnt->step;
     int             vs   = s.cnt->vs;
-    if (step > 0 && step % s.mc_interval == 0) {
+    if (step > 0 && og_step_mod(step, s.mc_interval) == 0) {
         vs        = og_mc_transition(s, vs, lam, step);
         s.cnt->vs = vs;
     }
@@ -1140,8 +1211,14 @@ void og_launch_constraints(const og_launch &trio, const og_launch &misc) {
     if (trio.n_blocks)
         hipLaunchKernelGGL(k_trio, dim3(trio.n_blocks), dim3(OG_TRIO_THREADS), 0, trio.stream, trio.sys, trio.map);
 }
-void og_launch_langevin_step(const og_launch &a) {
-    hipLaunchKernelGGL(k_langevin_step, dim3(a.n_blocks), dim3(OG_WATER_THREADS), 0, a.stream, a.sys, a.map);
+void og_launch_fused_step(const og_launch &a, int form) {
+    const dim3 nb(a.n_blocks), nt(OG_WATER_THREADS);
+    switch (form) {
+    case OG_FUSED_LANGEVIN_SETTLE: hipLaunchKernelGGL((k_fused_step<false, false>), nb, nt, 0, a.stream, a.sys, a.map); break;
+    case OG_FUSED_LANGEVIN_SHAKE: hipLaunchKernelGGL((k_fused_step<false, true>), nb, nt, 0, a.stream, a.sys, a.map); break;
+    case OG_FUSED_LEAPFROG_SETTLE: hipLaunchKernelGGL((k_fused_step<true, false>), nb, nt, 0, a.stream, a.sys, a.map); break;
+    default: hipLaunchKernelGGL((k_fused_step<true, true>), nb, nt, 0, a.stream, a.sys, a.map); break;
+    }
 }
 void og_launch_finish(const og_launch &a) {
     hipLaunchKernelGGL(k_finish, dim3(a.n_blocks), dim3(OG_THREADS), 0, a.stream, a.sys, a.map);

@@ -104,9 +104,11 @@ struct og_dev_sys {
     int n_angles, n_torsions, n_impros, n_nb14;  // bonded terms beyond bonds (og_bonded.hip)
     int n_bterms;          // n_angles + n_torsions + n_impros + n_nb14: one thread each
     int n_quads;           // SHAKE four-atom groups
-    int n_free;            // atoms outside SETTLE waters (fused Langevin step)
-    int n_free_blocks;     // fused Langevin step: blocks of OG_FREE_PER_BLOCK of them, at least one
-    int n_water_blocks;    // fused Langevin step: blocks of OG_WATERS_PER_BLOCK waters; 0 = not fusable
+    int n_waters;          // fused step: waters taken three lanes each (SETTLE waters, or SHAKE trios like them)
+    int n_free_trios;      // fused step: SHAKE trios among the other atoms (the first ones of trio_ids)
+    int n_free;            // fused step: atoms outside the waters
+    int n_free_blocks;     // fused step: blocks of OG_FREE_PER_BLOCK of them, at least one
+    int n_water_blocks;    // fused step: blocks of OG_WATERS_PER_BLOCK waters; 0 = not fusable
     int pair_split;        // pair kernel: at most this many of the last cells run as two half-cell waves each
     int n_com_groups;
     int integrator;        // 0 leapfrog-presto, 1 langevin
@@ -202,7 +204,9 @@ struct og_dev_sys {
     int    *pairc_ids;      // [n_pairs_c*2]
     double *pairc_d2;
     int    *settle_ids;     // [n_settle*3]
-    int    *free_ids;       // [n_free] atoms outside SETTLE waters
+    int    *free_ids;       // [n_free] atoms outside the waters
+    int    *water_ids;      // [3*n_waters] settle_ids, or the waters' part of trio_ids
+    double *water_d2;       // [3*n_waters] their part of trio_d2 (SHAKE)
     og_step_sync *sync;     // arrivals of the fused step's blocks
     int    *com_off, *com_atoms;   // COM-cancel groups
     float  *com_minv;
@@ -280,11 +284,11 @@ enum og_map_kind {
 __host__ __device__ __forceinline__ int og_pair_split_cells(int split, int n_cells) {
     return n_cells >= 2 * split && n_cells < 8 * split ? split : 0;
 }
-#define OG_WATER_THREADS 256  // fused Langevin step: threads per block
-#define OG_WATERS_PER_WAVE 21  // fused Langevin step: three lanes per water
+#define OG_WATER_THREADS 256  // fused step: threads per block
+#define OG_WATERS_PER_WAVE 21  // fused step: three lanes per water
 #define OG_WATERS_PER_BLOCK (OG_WATERS_PER_WAVE * (OG_WATER_THREADS / 64))
-#define OG_FREE_PER_BLOCK (OG_WATER_THREADS / 8)  // fused Langevin step: eight lanes per free atom
-#define OG_FREE_MAX 4096      // fused Langevin step: most atoms outside SETTLE waters (one block takes them)
+#define OG_FREE_PER_BLOCK (OG_WATER_THREADS / 8)  // fused step: eight lanes per free atom
+#define OG_FREE_MAX 4096      // fused step: most atoms outside SETTLE waters (one block takes them)
 #define OG_CP_BLOCKS_PER_SYS_MIN 64
 
 // ---- small device helpers ----
@@ -297,17 +301,26 @@ __device__ __forceinline__ bool og_frozen_c(const og_dev_counters &c) {
     return c.step >= c.step_end || (c.flags & OG_F_FATAL) != 0;
 }
 __device__ __forceinline__ bool og_frozen(const og_dev_sys &s) { return og_frozen_c(*s.cnt); }
+// n mod d and n / d of a step number (n >= 0, d > 0): every kernel takes one
+// before its work, and the 64-bit division is some 150 instructions of a lone
+// wave (0.4 us) where the 32-bit one, right below 2^32 steps, is 20.
+__device__ __forceinline__ long long og_step_mod(long long n, int d) {
+    return (unsigned long long)n >> 32 ? n % d : (long long)((uint32_t)n % (uint32_t)d);
+}
+__device__ __forceinline__ long long og_step_div(long long n, int d) {
+    return (unsigned long long)n >> 32 ? n / d : (long long)((uint32_t)n / (uint32_t)d);
+}
 // The grid-rebuild kernels run for a system when its own step is a multiple
 // of its rebuild interval (DynamicsMode.cpp:480-486) or a rebuild is forced;
 // systems at other phases in the same launch skip them.
 __device__ __forceinline__ bool og_rebuild_skip(const og_dev_sys &s) {
-    return og_frozen(s) || (s.rebuild_intvl > 0 && (s.cnt->step % s.rebuild_intvl) != 0 && !s.cnt->rebuild_now);
+    return og_frozen(s) || (s.rebuild_intvl > 0 && og_step_mod(s.cnt->step, s.rebuild_intvl) != 0 && !s.cnt->rebuild_now);
 }
 // Energies (pair, virial) are evaluated on logged steps and on request; the
 // forces and the pair count on every step.
 __device__ __forceinline__ bool og_energy_step_c(const og_dev_sys &s, const og_dev_counters &c) {
     // V-McMD needs the potential energy of every step (its lambda)
-    return c.force_energy || (c.step % s.log_stride) == 0 || s.mc_mode == OG_MC_VMCMD;
+    return c.force_energy || og_step_mod(c.step, s.log_stride) == 0 || s.mc_mode == OG_MC_VMCMD;
 }
 __device__ __forceinline__ bool og_energy_step(const og_dev_sys &s) { return og_energy_step_c(s, *s.cnt); }
 
@@ -451,50 +464,46 @@ __device__ __forceinline__ void og_eacc_clear(const og_dev_sys &s) {
 #pragma unroll
     for (int k = 0; k < OG_EACC_WORDS / NT; k++) s.e_acc[threadIdx.x + k * NT] = 0;
 }
-// the block's loaded term sums into s.energy (and, when e is given, into
-// thread 0's copy e of the energy row)
+// Energy term k's accumulator, four bits each (15: none), so a thread finds its own.
+constexpr unsigned long long og_eacc_of(const int (&e)[OG_EACC]) {
+    unsigned long long p = ~0ull;
+    for (int a = 0; a < OG_EACC; a++) p = (p & ~(15ull << (4 * e[a]))) | ((unsigned long long)a << (4 * e[a]));
+    return p;
+}
+static_assert(OG_E_NTERMS <= 16 && OG_EACC <= 15, "four bits per term");
+// Sums the block's loaded accumulators; thread k < OG_E_NTERMS gets term k and
+// true if the accumulators (or the self energy) hold it.  A thread per term:
+// one thread taking all of them ran 600 instructions at the end of each step.
 template <int NT>
-__device__ __forceinline__ void og_eacc_reduce(const og_dev_sys &s, long long v, long long *sh, double *e) {
+__device__ __forceinline__ bool og_eacc_term(const og_dev_sys &s, long long v, long long *sh, double &val) {
     static_assert(OG_EACC_STRIDE == 16 && OG_EACC <= OG_EACC_STRIDE, "one term per lane of a 16-lane row");
+    constexpr int of[OG_EACC] = {OG_E_VDW, OG_E_ELE, OG_E_VIRIAL, OG_E_NPAIRS, OG_E_EXCESS, OG_E_BOND,
+                                 OG_E_ANGLE, OG_E_TORSION, OG_E_IMPRO, OG_E_VDW14, OG_E_ELE14};
+    static_assert(OG_EACC_VDW == 0 && OG_EACC_ELE == 1 && OG_EACC_VIR == 2 && OG_EACC_PAIRS == 3 &&
+                  OG_EACC_EXCESS == 4 && OG_EACC_BOND == 5 && OG_EACC_ANGLE == 6 && OG_EACC_TORSION == 7 &&
+                  OG_EACC_IMPRO == 8 && OG_EACC_VDW14 == 9 && OG_EACC_ELE14 == 10, "the order of the list above");
+    constexpr unsigned long long pack = og_eacc_of(of);
     v += __shfl_xor(v, 16, 64);
     v += __shfl_xor(v, 32, 64);
-    const int w = threadIdx.x >> 6;
+    const int w = threadIdx.x >> 6, k = threadIdx.x;
     if ((threadIdx.x & 63) < OG_EACC_STRIDE) sh[w * OG_EACC_STRIDE + (threadIdx.x & 63)] = v;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        long long t[OG_EACC];
-        for (int q = 0; q < OG_EACC; q++) t[q] = 0;
-        for (int k = 0; k < NT / 64; k++)
-            for (int q = 0; q < OG_EACC; q++) t[q] += sh[k * OG_EACC_STRIDE + q];
-        double r[OG_E_NTERMS];
-        r[OG_E_VDW]     = (double)t[OG_EACC_VDW] * OG_FX_INV;
-        r[OG_E_ELE]     = (double)t[OG_EACC_ELE] * OG_FX_INV;
-        r[OG_E_VIRIAL]  = (double)t[OG_EACC_VIR] * OG_FX_INV;
-        r[OG_E_NPAIRS]  = (double)t[OG_EACC_PAIRS];
-        r[OG_E_EXCESS]  = (double)t[OG_EACC_EXCESS] * OG_FX_INV;
-        r[OG_E_BOND]    = (double)t[OG_EACC_BOND] * OG_FX_INV;
-        r[OG_E_ANGLE]   = (double)t[OG_EACC_ANGLE] * OG_FX_INV;
-        r[OG_E_TORSION] = (double)t[OG_EACC_TORSION] * OG_FX_INV;
-        r[OG_E_IMPRO]   = (double)t[OG_EACC_IMPRO] * OG_FX_INV;
-        r[OG_E_VDW14]   = (double)t[OG_EACC_VDW14] * OG_FX_INV;
-        r[OG_E_ELE14]   = (double)t[OG_EACC_ELE14] * OG_FX_INV;
-        r[OG_E_SELF]    = s.e_self;
-        const int terms[] = {OG_E_VDW, OG_E_ELE, OG_E_VIRIAL, OG_E_NPAIRS, OG_E_EXCESS, OG_E_BOND, OG_E_ANGLE,
-                             OG_E_TORSION, OG_E_IMPRO, OG_E_VDW14, OG_E_ELE14, OG_E_SELF};
-        for (int k : terms) {
-            s.energy[k] = r[k];
-            if (e) e[k] = r[k];
-        }
-    }
-    __syncthreads();
+    const int acc = k < 16 ? (int)(pack >> (4 * k)) & 15 : 15;
+    if (k == OG_E_SELF) val = s.e_self;
+    if (acc == 15) return k == OG_E_SELF;
+    long long t = 0;
+    for (int j = 0; j < NT / 64; j++) t += sh[j * OG_EACC_STRIDE + acc];
+    val = k == OG_E_NPAIRS ? (double)t : (double)t * OG_FX_INV;
+    return true;
 }
 template <int NT>
 __device__ __forceinline__ void og_take_pair_energies(const og_dev_sys &s, long long *sh) {
     const long long v = og_eacc_load<NT>(s);
     og_eacc_clear<NT>(s);
-    og_eacc_reduce<NT>(s, v, sh, nullptr);
+    double val;
+    if (og_eacc_term<NT>(s, v, sh, val)) s.energy[threadIdx.x] = val;
+    __syncthreads();
 }
-
 
 __device__ __forceinline__ void og_atomic_add_fx(long long *p, long long v) {
     if (v != 0) atomicAdd((unsigned long long *)p, (unsigned long long)v);
@@ -565,7 +574,8 @@ void og_launch_constraints(const og_launch &trio, const og_launch &misc);
 // bonded terms beyond bonds and four-atom SHAKE (og_bonded.hip)
 void og_launch_bonded(const og_launch &terms);  // OG_THREADS threads per block over n_bterms
 void og_launch_shake_quad(const og_launch &quads);  // OG_QUAD_THREADS threads per block over n_quads
-void og_launch_langevin_step(const og_launch &a);
+enum { OG_FUSED_LANGEVIN_SETTLE, OG_FUSED_LANGEVIN_SHAKE, OG_FUSED_LEAPFROG_SETTLE, OG_FUSED_LEAPFROG_SHAKE };
+void og_launch_fused_step(const og_launch &a, int form);  // closes the step
 void og_launch_finish(const og_launch &atoms);
 void og_launch_step_close(const og_launch &sys);  // energies of the step, log entry, step counter
 void og_launch_vcmd(const og_launch &sys);  // VcMD and V-AUS group bias

@@ -904,11 +904,11 @@ __global__ void __launch_bounds__(OG_THREADS) k_point_end(const og_dev_sys *__re
         __shared__ long long sh[16 * OG_EACC_STRIDE];
         og_take_pair_energies<OG_THREADS>(s, sh);
     }
+    if (threadIdx.x < OG_E_NTERMS) out->energy[threadIdx.x] = s.energy[threadIdx.x];
     if (threadIdx.x) return;
     s.cnt->rebuild_now  = 0;
     s.cnt->force_energy = 0;
     out->cnt            = *s.cnt;
-    for (int k = 0; k < OG_E_NTERMS; k++) out->energy[k] = s.energy[k];
 }
 
 // ------------------------------------------------------------- launchers --
