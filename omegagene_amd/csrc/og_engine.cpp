@@ -448,7 +448,6 @@ og_launch L(const og_exec &x, int kind) { return og_launch{x.d_sys, x.d_map[kind
 
 void enqueue_rebuild(og_exec &x) {
     og_launch_grid_bin(L(x, KIND_ATOM));
-    og_launch_grid_scan(L(x, KIND_SYS));
     og_launch_grid_scatter(L(x, KIND_ATOM));
     og_launch_grid_sort(L(x, KIND_COL));
     og_launch_enum_count(L(x, KIND_CELLW));
@@ -464,7 +463,6 @@ void launch_pair(const og_exec &x, int shape) {
     else og_launch_pair(a, x.pair_form, 1 << (shape & 3));
 }
 
-// point: a single-point call, which always takes the gradient
 void enqueue_forces(og_exec &x, hipEvent_t e0, hipEvent_t e1, bool point = false) {
     if (e0) hipEventRecord(e0, x.stream);
     launch_pair(x, x.pair_shape);
@@ -472,8 +470,8 @@ void enqueue_forces(og_exec &x, hipEvent_t e0, hipEvent_t e1, bool point = false
     // angles, torsions, impropers, 1-4 pairs: each atom's shares, summed with its pair gradient below (or in
     // the fused step kernel)
     if (x.any_bonded) og_launch_bonded(L(x, KIND_BTERM));
-    // an MD step of a fused context converts the gradient inside its step kernel
-    if (point || !x.fused) og_launch_forces_to_work(L(x, KIND_ATOM));
+    // a fused context converts the gradient inside its step kernel, a single-point call in its last one
+    if (!point && !x.fused) og_launch_forces_to_work(L(x, KIND_ATOM));
 }
 
 void enqueue_integrate(og_exec &x) {
@@ -588,6 +586,7 @@ og_status check_flags(og_system *s, const og_dev_counters &c) {
         OG_HIP(hipMemset(s->h.fx, 0, sizeof(long long) * OG_FX_WORDS(s->h.cap_atom_array)));
         OG_HIP(hipMemset(s->h.e_acc, 0, sizeof(long long) * OG_EACC_SLOTS * OG_EACC_STRIDE));
         OG_HIP(hipMemset(s->h.n_atoms_col, 0, sizeof(int) * s->h.n_columns));
+        OG_HIP(hipMemset(s->h.sync, 0, sizeof(og_step_sync)));
         s->grid_valid = false;
     }
     if (st != OG_OK) set_err("%s", msg);
@@ -841,7 +840,7 @@ og_status sys_alloc(og_system *s, const og_system_desc *d, const og_params *p) {
               A(&h.cell_u1, h.cap_cells) && A(&h.u2c_min, (size_t)(h.n_columns + 2) * h.n_uni_z) &&
               A(&h.u2c_max, (size_t)(h.n_columns + 2) * h.n_uni_z) && A(&h.cp_count, h.cap_cells + 1) && A(&h.cp_stage, (size_t)h.cap_cells * OG_ENUM_STAGE) &&
               A(&h.cp_head, h.cap_cells + 1) && A(&h.cp_bsum, h.cap_cells / 1024 + 1) && A(&h.cp_c2, h.cap_cell_pairs) && A(&h.cp_mask, h.cap_cell_pairs) &&
-              A(&h.fx, OG_FX_WORDS(cap)) && A(&h.e_acc, (size_t)OG_EACC_SLOTS * OG_EACC_STRIDE);
+              A(&h.fx, OG_FX_WORDS(cap)) && A(&h.e_acc, (size_t)OG_EACC_SLOTS * OG_EACC_STRIDE) && A(&h.sync, 1);
     if (!ok) return OG_E_DEVICE;
     const int n_tor     = h.n_torsions + h.n_impros;
     const int n_contrib = 3 * h.n_angles + 4 * n_tor + 2 * h.n_nb14;
@@ -1061,7 +1060,7 @@ og_status sys_alloc(og_system *s, const og_system_desc *d, const og_params *p) {
         for (int i = 0; i < n; i++)
             if (water[i] < 0 || !good[water[i]]) free_ids.push_back(i);
         if (nw > 0 && (nw == nt || !settle) && (int)free_ids.size() <= OG_FREE_MAX) {
-            if (!A(&h.free_ids, std::max<size_t>(free_ids.size(), 1)) || !A(&h.sync, 1)) return OG_E_DEVICE;
+            if (!A(&h.free_ids, std::max<size_t>(free_ids.size(), 1))) return OG_E_DEVICE;
             if (!free_ids.empty())
                 OG_HIP(hipMemcpy(h.free_ids, free_ids.data(), sizeof(int) * free_ids.size(), hipMemcpyHostToDevice));
             h.n_free         = (int)free_ids.size();
@@ -1626,7 +1625,7 @@ og_status og_calc_energy_force(og_system *s, int rebuild, double *work_atom, dou
     og_launch_point_begin(s->d_cnt, fresh, x.stream);
     if (fresh) enqueue_rebuild(x);
     enqueue_forces(x, nullptr, nullptr, true);
-    og_launch_point_end(L(x, KIND_SYS), out, wpin, s->h.n_atoms);
+    og_launch_point_end(L(x, KIND_ATOM), out, wpin);
     OG_HIP(hipGetLastError());
     OG_HIP(hipStreamSynchronize(x.stream));
     s->grid_valid = true;

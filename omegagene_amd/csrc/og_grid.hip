@@ -60,6 +60,64 @@ __device__ __forceinline__ int og_wave_count_add(int *ctr, int key, bool active)
     return __shfl(base, leader, 64) + rank;
 }
 
+// ----------------------------------------------------------------- scan --
+// MiniCell::set_idx_xy_head (MiniCell.cpp:785-861): cells per column,
+// exclusive scan to head cell/atom, -1 heads for empty columns.  By the last
+// block of the binning, which reads the counts of all blocks (a launch of its
+// own took 4 us and the gap before it).
+__device__ __forceinline__ void og_scan_columns(const og_dev_sys &s) {
+    const int nc  = s.n_columns;
+    const int per = (nc + OG_THREADS - 1) / OG_THREADS;
+    const int k0  = threadIdx.x * per, k1 = min(k0 + per, nc);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    __shared__ int wsum[OG_THREADS / 64], big;
+    if (threadIdx.x == 0) big = 0;
+    auto count = [&](int k) {
+        return __hip_atomic_load(&s.n_atoms_col[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    int local = 0, mx = 0;
+#pragma unroll 4
+    for (int k = k0; k < k1; k++) {
+        const int n = count(k);
+        local += (n + OG_NAC - 1) / OG_NAC;
+        mx = max(mx, n);
+    }
+    int incl = local;
+    for (int off = 1; off < 64; off <<= 1) {
+        const int v = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += v;
+    }
+    if (lane == 63) wsum[w] = incl;
+    __syncthreads();
+    if (mx > OG_SORT_CAP) atomicOr(&big, 1);
+    __syncthreads();
+    int cell = incl - local;
+    for (int q = 0; q < w; q++) cell += wsum[q];
+#pragma unroll 4
+    for (int k = k0; k < k1; k++) {
+        const int n  = count(k);
+        const int nz = (n + OG_NAC - 1) / OG_NAC;
+        s.n_cells_z[k] = nz;
+        s.head_cell[k] = n ? cell : -1;
+        s.head_atom[k] = n ? cell * OG_NAC : -1;
+        s.col_fill[k]  = 0;
+        cell += nz;
+    }
+    if (threadIdx.x == OG_THREADS - 1) {
+        int total = cell;
+        s.head_cell[nc] = total;
+        s.head_atom[nc] = total * OG_NAC;
+        int fl = 0;
+        if (total > s.cap_cells) fl |= OG_F_CELL_OVERFLOW;
+        if (big) fl |= OG_F_COL_OVERFLOW;
+        if (fl) {
+            atomicOr(&s.cnt->flags, fl);
+            total = 0;  // nothing downstream runs on a grid that does not fit
+        }
+        s.cnt->n_cells = total;
+    }
+}
+
 __global__ void __launch_bounds__(OG_THREADS) k_grid_bin(const og_dev_sys *__restrict__ S,
                                                          const int2 *__restrict__ map) {
     const int2        bm = map[blockIdx.x];
@@ -100,61 +158,7 @@ __global__ void __launch_bounds__(OG_THREADS) k_grid_bin(const og_dev_sys *__res
         s.zkey[i]        = og_float_key(bad ? 0.0f : (float)z);
     }
     og_wave_count_add(s.n_atoms_col, c[0] + c[1] * s.nx, in);
-}
-
-// ----------------------------------------------------------------- scan --
-// MiniCell::set_idx_xy_head (MiniCell.cpp:785-861): cells per column,
-// exclusive scan to head cell/atom, -1 heads for empty columns.
-__global__ void __launch_bounds__(1024) k_grid_scan(const og_dev_sys *__restrict__ S, const int2 *__restrict__ map) {
-    const og_dev_sys &s  = S[map[blockIdx.x].x];
-    if (og_rebuild_skip(s)) return;
-    const int         nc = s.n_columns;
-    const int         T  = blockDim.x;
-    const int         per = (nc + T - 1) / T;
-    const int         k0  = threadIdx.x * per;
-    const int         k1  = min(k0 + per, nc);
-    __shared__ int    sh[1024];
-    __shared__ int    big;
-    if (threadIdx.x == 0) big = 0;
-    int local = 0, mx = 0;
-    for (int k = k0; k < k1; k++) {
-        const int n = s.n_atoms_col[k];
-        local += (n + OG_NAC - 1) / OG_NAC;
-        mx = max(mx, n);
-    }
-    sh[threadIdx.x] = local;
-    __syncthreads();
-    if (mx > OG_SORT_CAP) atomicOr(&big, 1);
-    // Hillis-Steele inclusive scan over 1024 partial sums
-    for (int off = 1; off < T; off <<= 1) {
-        const int v = threadIdx.x >= off ? sh[threadIdx.x - off] : 0;
-        __syncthreads();
-        sh[threadIdx.x] += v;
-        __syncthreads();
-    }
-    int cell = sh[threadIdx.x] - local;
-    for (int k = k0; k < k1; k++) {
-        const int n  = s.n_atoms_col[k];
-        const int nz = (n + OG_NAC - 1) / OG_NAC;
-        s.n_cells_z[k] = nz;
-        s.head_cell[k] = n ? cell : -1;
-        s.head_atom[k] = n ? cell * OG_NAC : -1;
-        s.col_fill[k]  = 0;
-        cell += nz;
-    }
-    if (threadIdx.x == T - 1) {
-        int total = sh[T - 1];
-        s.head_cell[nc] = total;
-        s.head_atom[nc] = total * OG_NAC;
-        int fl = 0;
-        if (total > s.cap_cells) fl |= OG_F_CELL_OVERFLOW;
-        if (big) fl |= OG_F_COL_OVERFLOW;
-        if (fl) {
-            atomicOr(&s.cnt->flags, fl);
-            total = 0;  // nothing downstream runs on a grid that does not fit
-        }
-        s.cnt->n_cells = total;
-    }
+    if (og_last_block(&s.sync->all, s.n_atom_blocks)) og_scan_columns(s);
 }
 
 // -------------------------------------------------------------- scatter --
@@ -671,9 +675,6 @@ void og_launch_grid_clear(const og_launch &cols) {
 }
 void og_launch_grid_bin(const og_launch &a) {
     hipLaunchKernelGGL(k_grid_bin, dim3(a.n_blocks), dim3(OG_THREADS), 0, a.stream, a.sys, a.map);
-}
-void og_launch_grid_scan(const og_launch &a) {
-    hipLaunchKernelGGL(k_grid_scan, dim3(a.n_blocks), dim3(1024), 0, a.stream, a.sys, a.map);
 }
 void og_launch_grid_scatter(const og_launch &a) {
     hipLaunchKernelGGL(k_grid_scatter, dim3(a.n_blocks), dim3(OG_THREADS), 0, a.stream, a.sys, a.map);

@@ -84,8 +84,9 @@ struct og_dev_counters {
     double    mc_scale;    // V-McMD: the gradient factor of the current step
 };
 
-// Blocks of a fused step that have arrived (zero between launches; a line
-// each), and the bias its group block hands to the block that goes on.
+// Blocks of a kernel that have arrived (zero between launches; a line each;
+// lead: the fused step's lead blocks), and the bias that the fused step's
+// group block hands to the block that goes on.
 struct og_step_sync {
     int    lead, pad0[31];
     int    all, pad1[31];
@@ -207,7 +208,7 @@ struct og_dev_sys {
     int    *free_ids;       // [n_free] atoms outside the waters
     int    *water_ids;      // [3*n_waters] settle_ids, or the waters' part of trio_ids
     double *water_d2;       // [3*n_waters] their part of trio_d2 (SHAKE)
-    og_step_sync *sync;     // arrivals of the fused step's blocks
+    og_step_sync *sync;     // arrivals of a kernel's blocks
     int    *com_off, *com_atoms;   // COM-cancel groups
     float  *com_minv;
     // ---- grid ----
@@ -535,7 +536,6 @@ struct og_launch {
 // grid build
 void og_launch_grid_clear(const og_launch &cols);
 void og_launch_grid_bin(const og_launch &atoms);
-void og_launch_grid_scan(const og_launch &sys);
 void og_launch_grid_scatter(const og_launch &atoms);
 void og_launch_grid_sort(const og_launch &cols);
 void og_launch_cells_from_grid(const og_launch &cols);
@@ -562,7 +562,7 @@ struct alignas(16) og_point_out {
     double          energy[OG_E_NTERMS];
 };
 void og_launch_point_begin(og_dev_counters *cnt, int rebuild, hipStream_t stream);
-void og_launch_point_end(const og_launch &sys, og_point_out *out, double *work, int n_atoms);
+void og_launch_point_end(const og_launch &atoms, og_point_out *out, double *work);  // takes the gradient too
 // integration
 void og_launch_leapfrog_vel(const og_launch &atoms);
 void og_launch_com_sum(const og_launch &sys);

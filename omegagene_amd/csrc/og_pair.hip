@@ -881,10 +881,12 @@ __global__ void __launch_bounds__(64) k_energy_reduce(const og_dev_sys *__restri
 }
 
 // A single-point evaluation of one system.  Its requests (energies, and a
-// grid rebuild) go into the counters before the first kernel, its outcome to
-// pinned host memory after the last: the counters, the energies and, when
-// work is given, the gradient.  One wait for the stream then delivers what
-// took six copies with a wait each (4,230 atoms: 208 us per call, now 116).
+// grid rebuild) go into the counters before the first kernel; the last kernel
+// is k_forces_to_work with its outcome sent to pinned host memory: the
+// gradient when work is given, and from the last block the counters and the
+// energies.  One wait for the stream then delivers what took six copies with a
+// wait each (4,230 atoms: 208 us per call, then 116; 5 of them the reduction's
+// own launch, now this last block).
 __global__ void k_point_begin(og_dev_counters *c, int rebuild) {
     c->force_energy = 1;
     if (rebuild) c->rebuild_now = 1;
@@ -892,15 +894,32 @@ __global__ void k_point_begin(og_dev_counters *c, int rebuild) {
 __global__ void __launch_bounds__(OG_THREADS) k_point_end(const og_dev_sys *__restrict__ S,
                                                           og_point_out *__restrict__ out,
                                                           double *__restrict__ work) {
-    const og_dev_sys &s = S[0];
-    if (blockIdx.x) {
-        const int k = 2 * ((blockIdx.x - 1) * OG_THREADS + threadIdx.x);
-        const int n = 3 * s.n_atoms;
-        if (k + 1 < n) *(double2 *)(work + k) = *(const double2 *)(s.work + k);
-        else if (k < n) work[k] = s.work[k];
-        return;
+    const og_dev_sys &s      = S[0];
+    const bool        run    = !og_frozen(s);
+    const bool        energy = run && og_energy_step(s);
+    const int         i0     = blockIdx.x * OG_THREADS, i = i0 + threadIdx.x;
+    double            e_ex = 0.0, e_b = 0.0, w[3] = {0.0, 0.0, 0.0};
+    if (i < s.n_atoms) {
+        if (run) {
+            og_atom_work_calc(s, i, w, e_ex, e_b);
+            og_atom_work_store(s, i, w);
+        } else {  // a system that stands still returns the gradient it has
+            for (int k = 0; k < 3; k++) w[k] = s.work[3 * i + k];
+        }
     }
-    if (!og_frozen(s) && og_energy_step(s)) {
+    if (work) {  // whole lines to the host
+        __shared__ double wl[3 * OG_THREADS];
+        for (int k = 0; k < 3; k++) wl[3 * threadIdx.x + k] = w[k];
+        __syncthreads();
+        const int n = 3 * min(OG_THREADS, s.n_atoms - i0);
+        for (int k = threadIdx.x; k < n; k += OG_THREADS) work[3 * (size_t)i0 + k] = wl[k];
+    }
+    if (energy) {
+        __shared__ double sh[2 * (OG_THREADS / 64)];
+        og_add_misc_energies(s, blockIdx.x, e_ex, e_b, sh);
+    }
+    if (!og_last_block(&s.sync->all, gridDim.x)) return;
+    if (energy) {
         __shared__ long long sh[16 * OG_EACC_STRIDE];
         og_take_pair_energies<OG_THREADS>(s, sh);
     }
@@ -954,7 +973,6 @@ void og_launch_energy_reduce(const og_launch &a) {
 void og_launch_point_begin(og_dev_counters *cnt, int rebuild, hipStream_t st) {
     hipLaunchKernelGGL(k_point_begin, dim3(1), dim3(1), 0, st, cnt, rebuild);
 }
-void og_launch_point_end(const og_launch &a, og_point_out *out, double *work, int n_atoms) {
-    const int nb = work ? (3 * n_atoms + 2 * OG_THREADS - 1) / (2 * OG_THREADS) : 0;
-    hipLaunchKernelGGL(k_point_end, dim3(1 + nb), dim3(OG_THREADS), 0, a.stream, a.sys, out, work);
+void og_launch_point_end(const og_launch &a, og_point_out *out, double *work) {
+    hipLaunchKernelGGL(k_point_end, dim3(a.n_blocks), dim3(OG_THREADS), 0, a.stream, a.sys, out, work);
 }
