@@ -1056,13 +1056,26 @@ og_status sys_alloc(og_system *s, const og_system_desc *d, const og_params *p) {
         drop_all(d->impro_ids, 4LL * h.n_impros);
         drop_all(d->nb14_ids, 2LL * h.n_nb14);
         const int nw = (int)std::count(good.begin(), good.end(), 1);
+        std::vector<int> group(n, 0);  // the atom's bias group
+        bool             once = true;
+        for (int k = 0; k < h.vc_na + h.vc_nb; k++) {
+            int &g = group[k < h.vc_na ? d->vc_atoms_a[k] : d->vc_atoms_b[k - h.vc_na]];
+            once &= g == 0;  // the separate kernels take an atom listed twice
+            g = k < h.vc_na ? 1 : 2;
+        }
         std::vector<int> free_ids;
         for (int i = 0; i < n; i++)
             if (water[i] < 0 || !good[water[i]]) free_ids.push_back(i);
-        if (nw > 0 && (nw == nt || !settle) && (int)free_ids.size() <= OG_FREE_MAX) {
+        if (nw > 0 && once && (nw == nt || !settle) && (int)free_ids.size() <= OG_FREE_MAX) {
             if (!A(&h.free_ids, std::max<size_t>(free_ids.size(), 1))) return OG_E_DEVICE;
             if (!free_ids.empty())
                 OG_HIP(hipMemcpy(h.free_ids, free_ids.data(), sizeof(int) * free_ids.size(), hipMemcpyHostToDevice));
+            if (h.vc_na + h.vc_nb > 0) {
+                std::vector<int> fg(std::max<size_t>(free_ids.size(), 1), 0);
+                for (size_t k = 0; k < free_ids.size(); k++) fg[k] = group[free_ids[k]];
+                if (!A(&h.free_group, fg.size())) return OG_E_DEVICE;
+                OG_HIP(hipMemcpy(h.free_group, fg.data(), sizeof(int) * fg.size(), hipMemcpyHostToDevice));
+            }
             h.n_free         = (int)free_ids.size();
             h.n_free_blocks  = std::max(1, cdiv(h.n_free, OG_FREE_PER_BLOCK));
             h.n_waters       = nw;
@@ -1352,7 +1365,7 @@ og_status og_system_footprint(const og_system_desc *d, const og_params *p, uint6
     b += cells * (6 * 4 + 4.0 * OG_ENUM_STAGE + 8) + (cells / 1024 + 1) * 8;
     b += pairs * 12;
     b += 8.0 * OG_EACC_SLOTS * OG_EACC_STRIDE + ke_parts * 8 + OG_E_NTERMS * 8 + log_rows * OG_E_NTERMS * 8;
-    b += std::min(n, (double)OG_FREE_MAX) * 4 + sizeof(og_step_sync) + vc * 28 + vs * 32 + mcs * (4 + 8.0 * OG_MC_NPOLY + 32);
+    b += std::min(n, (double)OG_FREE_MAX) * (vc > 0 ? 8 : 4) + sizeof(og_step_sync) + vc * 28 + vs * 32 + mcs * (4 + 8.0 * OG_MC_NPOLY + 32);
     {
         const double na = d->n_angles, ntr = (double)d->n_torsions + d->n_impros, n14 = d->n_nb14;
         const double nq = p->constraint ? d->n_shake_quads : 0;

@@ -860,7 +860,13 @@ __device__ __forceinline__ void og_free_work(const og_dev_sys &s, const int blk,
 }
 
 __device__ void og_vcmd_lambda(const og_dev_sys &s, double *bias, int &active);  // VcMD section below
-__device__ void og_vcmd_apply(const og_dev_sys &s, const double *bias);
+// what the bias u adds to a component of the gradient of a group atom
+__device__ __forceinline__ double og_vcmd_work(const og_dev_sys &s, const bool group_a, const double u,
+                                               const double mass) {
+    const double minv = group_a ? s.vc_minv_a : s.vc_minv_b;
+    const double dir  = group_a ? 1.0 : -1.0;
+    return dir * (u * minv) * mass;
+}
 
 // Three waves per SIMD (168 registers): left free the kernel takes 203 (two
 // waves), held to 128 it spills (450,000 atoms 430 / 421 / 429 us per step at
@@ -893,17 +899,22 @@ __global__ void __launch_bounds__(OG_WATER_THREADS, 3) k_fused_step(const og_dev
         }
         if (og_last_block(&s.sync->lead, lead)) {
             const int nf = s.n_free;
+            // the bias enters as the atoms are moved: a pass of its own over the groups was 2.4 us
+            double u[3] = {0.0, 0.0, 0.0};
+            bool   on   = false;
             if (biased) {
-                if (tid < 3) bias[tid] = og_take(&s.sync->bias[tid]);
-                const bool on = og_take(&s.sync->active) != 0.0;
-                __syncthreads();
-                if (on) og_vcmd_apply(s, bias);
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                __syncthreads();
+                for (int d = 0; d < 3; d++) u[d] = og_take(&s.sync->bias[d]);
+                on = og_take(&s.sync->active) != 0.0;
             }
             for (int k = tid; k < nf; k += OG_WATER_THREADS) {
-                const int    i     = s.free_ids[k];
-                const double wk[3] = {og_take(&s.work[3 * i]), og_take(&s.work[3 * i + 1]), og_take(&s.work[3 * i + 2])};
+                const int i     = s.free_ids[k];
+                const int group = biased ? s.free_group[k] : 0;
+                double    wk[3] = {og_take(&s.work[3 * i]), og_take(&s.work[3 * i + 1]), og_take(&s.work[3 * i + 2])};
+                if (on && group)
+                    for (int d = 0; d < 3; d++) {
+                        wk[d] += og_vcmd_work(s, group == 1, u[d], (double)s.mass[i]);
+                        og_put(&s.work[3 * i + d], wk[d]);
+                    }
                 if (LEAP) og_leapfrog_atom(s, i, wk);
                 else og_langevin_atom(s, i, step, wk);
             }
@@ -1051,13 +1062,7 @@ __device__ void og_vcmd_apply(const og_dev_sys &s, const double *bias) {
     const int n = s.vc_na + s.vc_nb;
     for (int k = threadIdx.x; k < n; k += blockDim.x) {
         const int    a    = s.vc_atoms[k];
-        const bool   ga   = k < s.vc_na;
-        const double minv = ga ? s.vc_minv_a : s.vc_minv_b;
-        const double dir  = ga ? 1.0 : -1.0;
-        for (int d = 0; d < 3; d++) {
-            double *w = &s.work[3 * a + d];
-            og_put(w, og_take(w) + dir * (bias[d] * minv) * (double)s.mass[a]);
-        }
+        for (int d = 0; d < 3; d++) s.work[3 * a + d] += og_vcmd_work(s, k < s.vc_na, bias[d], (double)s.mass[a]);
     }
 }
 

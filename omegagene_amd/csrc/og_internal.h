@@ -206,6 +206,7 @@ struct og_dev_sys {
     double *pairc_d2;
     int    *settle_ids;     // [n_settle*3]
     int    *free_ids;       // [n_free] atoms outside the waters
+    int    *free_group;     // [n_free] bias group of the atom: 0 none, 1 a, 2 b (with groups)
     int    *water_ids;      // [3*n_waters] settle_ids, or the waters' part of trio_ids
     double *water_d2;       // [3*n_waters] their part of trio_d2 (SHAKE)
     og_step_sync *sync;     // arrivals of a kernel's blocks
