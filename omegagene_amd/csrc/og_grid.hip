@@ -341,7 +341,7 @@ __global__ void __launch_bounds__(OG_THREADS) k_cells_from_grid(const og_dev_sys
 // MiniCell::enumerate_cell_pairs (MiniCell.cpp:938-1149) for one cell1 per
 // wave: lane k takes neighbour column k in the reference loop order
 // (dx outer, dy inner), walks the three z images and the candidate cells in
-// ascending id, so the per-lane prefix sum reproduces the CPU list order.
+// ascending id: the lanes' ranges, one after the other, are the CPU list order.
 __device__ __forceinline__ bool og_valid_pair(int c1, int c2) {
     // MiniCell::check_valid_pair (MiniCell.cpp:1150-1160)
     const bool o1 = (c1 & 1) != 0, o2 = (c2 & 1) != 0;
@@ -368,11 +368,24 @@ __device__ __forceinline__ float og_zgap2(float z2t, float z2b, float z1b, float
 // MODE 1: count the cell's pairs and stage them (cell2 | image << 24, list
 // order) in cp_stage[c1 * OG_ENUM_STAGE ...] as far as they fit;
 // MODE 2: write them at p0 (cells whose pairs did not fit).
-// Bound by its about 900 vector instructions per cell (147 us at 450,000
-// atoms): reading a lane's bins and candidates in batches of eight and four
-// independent loads cost 189 us there.
+// Bound by its instructions and gathered loads: with the candidates of a
+// column walked by its lane (25 of 64 lanes, 13 steps) it took 148 us at
+// 450,000 atoms, 60 for sixteen walkers, 33 at 99,200 atoms; a lane per
+// candidate 105, 53 and 29.  Reading a lane's bins eight at a time is slower
+// (119, 61 and 31): most windows are five bins.
+// LDS written by the wave's lanes is visible to the others after it
+__device__ __forceinline__ void og_wave_lds() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+struct og_enum_lds {  // of one wave
+    int4 at[64];    // by lane (neighbour column): candidates before its own, first cell per z image
+    int3 run[64];   // cells in images 0 and 1, (x, y) distance squared
+    int  mark[65];  // candidate of a chunk -> 1 + the lane whose candidates start there (64: of no chunk)
+};
 template <int MODE>
-__device__ void og_enum_cell(const og_dev_sys &s, int c1, int p0, int *out_count) {
+__device__ void og_enum_cell(const og_dev_sys &s, og_enum_lds &T, int c1, int p0, int *out_count) {
     const int lane  = threadIdx.x & 63;
     const int col1  = s.cell_col[c1];
     const int x1    = col1 % s.nx, y1 = col1 / s.nx;
@@ -401,13 +414,10 @@ __device__ void og_enum_cell(const og_dev_sys &s, int c1, int p0, int *out_count
         fz[2] = lz[2] = -1;
         lz[1]         = tl;
     }
-    int carry = MODE == 2 ? p0 : 0;
-    int total = 0;
+    int pos = MODE == 2 ? p0 : 0;  // of the next pair kept
     for (int r0 = 0; r0 < ncand; r0 += 64) {
         const int k     = r0 + lane;
-        int       mine  = 0;
-        int       c2lo[3], c2hi[3], img2 = 0;
-        uint64_t  kept[3] = {0ull, 0ull, 0ull};
+        int       c2lo[3], c2hi[3];
         float     dd01  = 0.0f;
         int       imgxy = 0;
         for (int ii = 0; ii < 3; ii++) c2lo[ii] = 0, c2hi[ii] = -1;
@@ -468,66 +478,79 @@ __device__ void og_enum_cell(const og_dev_sys &s, int c1, int p0, int *out_count
                 c2lo[ii] = head2 + zc0;
                 c2hi[ii] = head2 + zc1;
             }
-            for (int ii = 0; ii < 3; ii++) {
-                const float sh = (float)(ii - 1) * s.L[2];
-                for (int c2 = c2lo[ii]; c2 <= c2hi[ii]; c2++) {
-                    if (dd01 + og_zgap2(s.cell_zmax[c2] + sh, s.cell_zmin[c2] + sh, z1b, z1t) > s.cutoff_pair2) continue;
-                    if (!og_valid_pair(c1, c2)) continue;
-                    mine++;
-                    // the kept cells of this image as bits from c2lo (the write below
-                    // walks them instead of testing every cell again)
-                    if (c2 - c2lo[ii] < 64) kept[ii] |= 1ull << (c2 - c2lo[ii]);
-                }
-            }
         }
-        // exclusive prefix of per-lane counts in lane order
-        int incl = mine;
+        // The columns' candidates one after the other (column, image, cell: the list's order), a lane per
+        // candidate, two chunks of 64 at a time.
+        const int n0 = c2hi[0] - c2lo[0] + 1, n1 = c2hi[1] - c2lo[1] + 1, mine = n0 + n1 + c2hi[2] - c2lo[2] + 1;
+        int       incl = mine;
         for (int off = 1; off < 64; off <<= 1) {
             const int v = __shfl_up(incl, off, 64);
             if (lane >= off) incl += v;
         }
-        const int round_total = __shfl(incl, 63, 64);
-        if (mine) {
-            int p = carry + incl - mine;
-            for (int ii = 0; ii < 3; ii++) {
-                const float sh = (float)(ii - 1) * s.L[2];
-                img2           = ii == 0 ? 16 : ii == 2 ? 32 : 0;
-                auto emit = [&](int c2) {
-                    const int rec = c2 | ((imgxy | img2) << 24);
+        const int first = incl - mine, total = __builtin_amdgcn_readlane(incl, 63);
+        T.at[lane]  = make_int4(first, c2lo[0] | imgxy << 24, c2lo[1], c2lo[2]);
+        T.run[lane] = make_int3(n0, n1, __float_as_int(dd01));
+        int owner = 0;  // of the last candidate of the chunk before
+        for (int t0 = 0; t0 < total; t0 += 128) {
+            int   c2[2], img[2];
+            float zt[2], zb[2], dxy[2], sh[2];
+            bool  in[2];
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const int t = t0 + 64 * j + lane, d = first - (t - lane);
+                T.mark[lane] = 0;
+                og_wave_lds();
+                T.mark[mine > 0 && d >= 0 && d < 64 ? d : 64] = lane + 1;
+                og_wave_lds();
+                const int      v    = T.mark[lane];
+                const uint64_t m    = __ballot(v != 0) & (~0ull >> (63 - lane));  // starts up to this candidate
+                const int      from = __shfl(v, m ? 63 - __builtin_clzll(m) : lane, 64);
+                const int      own  = m ? from - 1 : owner;
+                owner               = __builtin_amdgcn_readlane(own, 63);
+                const int4 at       = T.at[own];
+                const int3 run      = T.run[own];
+                const int  e = t - at.x, e1 = e - run.x, e2 = e1 - run.y;
+                in[j]  = t < total;
+                c2[j]  = e1 < 0 ? (at.y & 0xffffff) + e : e2 < 0 ? at.z + e1 : at.w + e2;
+                c2[j]  = in[j] ? c2[j] : 0;
+                img[j] = (at.y >> 24) | (e1 < 0 ? 16 : e2 < 0 ? 0 : 32);
+                sh[j]  = (float)(e1 < 0 ? -1 : e2 < 0 ? 0 : 1) * s.L[2];
+                dxy[j] = __int_as_float(run.z);
+                zt[j]  = s.cell_zmax[c2[j]];
+                zb[j]  = s.cell_zmin[c2[j]];
+            }
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const bool keep = in[j] && !(dxy[j] + og_zgap2(zt[j] + sh[j], zb[j] + sh[j], z1b, z1t) > s.cutoff_pair2) &&
+                                  og_valid_pair(c1, c2[j]);
+                const uint64_t m = __ballot(keep);
+                if (keep) {
+                    const int p   = pos + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                                                         __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+                    const int rec = c2[j] | img[j] << 24;
                     if (MODE == 1) {
                         if (p < OG_ENUM_STAGE) s.cp_stage[(size_t)c1 * OG_ENUM_STAGE + p] = rec;
                     } else if (p < s.cap_cell_pairs) {
                         s.cp_c2[p] = rec;
                     }
-                    p++;
-                };
-                if (c2hi[ii] - c2lo[ii] < 64) {
-                    // ascending cell order, as the count
-                    for (uint64_t m = kept[ii]; m; m &= m - 1) emit(c2lo[ii] + __builtin_ctzll(m));
-                } else {
-                    for (int c2 = c2lo[ii]; c2 <= c2hi[ii]; c2++) {
-                        if (dd01 + og_zgap2(s.cell_zmax[c2] + sh, s.cell_zmin[c2] + sh, z1b, z1t) > s.cutoff_pair2)
-                            continue;
-                        if (!og_valid_pair(c1, c2)) continue;
-                        emit(c2);
-                    }
                 }
+                pos += __builtin_popcountll(m);
             }
         }
-        carry += round_total;
-        total += round_total;
+        og_wave_lds();  // the next round overwrites the tables
     }
-    if (MODE == 1 && lane == 0) *out_count = total;
+    if (MODE == 1 && lane == 0) *out_count = pos;
 }
 
 __global__ void __launch_bounds__(OG_THREADS) k_enum_count(const og_dev_sys *__restrict__ S,
                                                            const int2 *__restrict__ map) {
+    __shared__ og_enum_lds lds[OG_THREADS / 64];
     const int2        bm = map[blockIdx.x];
     const og_dev_sys &s  = S[bm.x];
     if (og_rebuild_skip(s)) return;
     const int         c1 = __builtin_amdgcn_readfirstlane(bm.y * (OG_THREADS / 64) + (threadIdx.x >> 6));
     if (c1 >= s.cnt->n_cells) return;
-    og_enum_cell<1>(s, c1, 0, &s.cp_count[c1]);
+    og_enum_cell<1>(s, lds[threadIdx.x >> 6], c1, 0, &s.cp_count[c1]);
 }
 
 // Exclusive scan of the cells' pair counts, blocks of 1024 cells: each cell's
@@ -577,7 +600,10 @@ __global__ void __launch_bounds__(1024) k_enum_scan(const og_dev_sys *__restrict
 // records and masks took three kernels of such chains (450,000 atoms 110 us,
 // now 84; 4,230 atoms 15 us and two launches more, now 9).
 __global__ void __launch_bounds__(OG_THREADS, 8) k_list(const og_dev_sys *__restrict__ S, const int2 *__restrict__ map) {
-    __shared__ int exq[OG_THREADS / 64][OG_NAC * OG_MAX_NB15];  // (cell2 << 6) | bit, per wave
+    __shared__ union {
+        og_enum_lds e;
+        int         ex[OG_NAC * OG_MAX_NB15];  // (cell2 << 6) | bit
+    } lds[OG_THREADS / 64];
     const int2        bm = map[blockIdx.x];
     const og_dev_sys &s  = S[bm.x];
     if (og_rebuild_skip(s)) return;
@@ -585,7 +611,7 @@ __global__ void __launch_bounds__(OG_THREADS, 8) k_list(const og_dev_sys *__rest
     const int c1   = __builtin_amdgcn_readfirstlane(bm.y * (OG_THREADS / 64) + w);
     const int n    = s.cnt->n_cells;
     if (c1 >= n) return;
-    int       *ex  = exq[w];
+    int       *ex  = lds[w].ex;
     const int *src = s.cp_stage + (size_t)c1 * OG_ENUM_STAGE;
     const int  cnt = __builtin_amdgcn_readfirstlane(s.cp_count[c1]);
     int        rec = src[lane];  // the stage of a cell is longer than a wave
@@ -610,7 +636,7 @@ __global__ void __launch_bounds__(OG_THREADS, 8) k_list(const og_dev_sys *__rest
     const int  m1     = __builtin_amdgcn_readfirstlane((int)min(end, cap)) - p0;  // records that fit
     const bool staged = cnt <= OG_ENUM_STAGE;
     if (!staged) {  // did not fit the stage: enumerate again, writing in place
-        og_enum_cell<2>(s, c1, p0, nullptr);
+        og_enum_cell<2>(s, lds[w].e, c1, p0, nullptr);
         __threadfence_block();
         rec = lane < m1 ? s.cp_c2[p0 + lane] : 0;
     }
