@@ -20,7 +20,6 @@
 // (word = x + y * 2^32), so one 64-bit integer atomic adds both and the sums
 // stay exact and order-independent.  Each field holds +-4096 kcal/mol/A; a
 // pair-kernel row beyond +-OG_FXJ_ROW_LIMIT flags the evaluation (an overlap).
-#define OG_FXJ_SCALE 524288.0
 #define OG_FXJ_INV (1.0 / 524288.0)
 #define OG_FXJ_ROW_LIMIT 2048.0f
 // Words of the fixed-point gradient per system, each component padded to whole
