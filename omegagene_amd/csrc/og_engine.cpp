@@ -446,8 +446,8 @@ og_status exec_prepare(og_exec &x) {
 
 og_launch L(const og_exec &x, int kind) { return og_launch{x.d_sys, x.d_map[kind], x.n_blocks[kind], x.stream}; }
 
-void enqueue_rebuild(og_exec &x) {
-    og_launch_grid_bin(L(x, KIND_ATOM));
+void enqueue_rebuild(og_exec &x, bool point = false) {
+    og_launch_grid_bin(L(x, KIND_ATOM), point);
     og_launch_grid_scatter(L(x, KIND_ATOM));
     og_launch_grid_sort(L(x, KIND_COL));
     og_launch_enum_count(L(x, KIND_CELLW));
@@ -1635,8 +1635,8 @@ og_status og_calc_energy_force(og_system *s, int rebuild, double *work_atom, dou
     double       *wpin  = pinned && work_atom ? (double *)(out + 1) : nullptr;
     const bool    fresh = rebuild || !s->grid_valid;
     // a single-point evaluation always carries its energies
-    og_launch_point_begin(s->d_cnt, fresh, x.stream);
-    if (fresh) enqueue_rebuild(x);
+    if (fresh) enqueue_rebuild(x, true);
+    else og_launch_point_begin(s->d_cnt, x.stream);
     enqueue_forces(x, nullptr, nullptr, true);
     og_launch_point_end(L(x, KIND_ATOM), out, wpin);
     OG_HIP(hipGetLastError());

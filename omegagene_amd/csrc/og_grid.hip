@@ -118,11 +118,13 @@ __device__ __forceinline__ void og_scan_columns(const og_dev_sys &s) {
     }
 }
 
+// point: a single-point call's rebuild, whatever the step; the last block
+// leaves the call's requests for the kernels after it.
 __global__ void __launch_bounds__(OG_THREADS) k_grid_bin(const og_dev_sys *__restrict__ S,
-                                                         const int2 *__restrict__ map) {
+                                                         const int2 *__restrict__ map, const int point) {
     const int2        bm = map[blockIdx.x];
     const og_dev_sys &s  = S[bm.x];
-    if (og_rebuild_skip(s)) return;
+    if (point ? og_frozen(s) : og_rebuild_skip(s)) return;
     const int         i  = bm.y * OG_THREADS + threadIdx.x;
     const bool        in = i < s.n_atoms;
     og_clear_bins(s, i, s.n_atom_blocks * OG_THREADS);  // read by the last rebuild only, filled by the sort
@@ -158,7 +160,9 @@ __global__ void __launch_bounds__(OG_THREADS) k_grid_bin(const og_dev_sys *__res
         s.zkey[i]        = og_float_key(bad ? 0.0f : (float)z);
     }
     og_wave_count_add(s.n_atoms_col, c[0] + c[1] * s.nx, in);
-    if (og_last_block(&s.sync->all, s.n_atom_blocks)) og_scan_columns(s);
+    if (!og_last_block(&s.sync->all, s.n_atom_blocks)) return;
+    if (point && threadIdx.x == 0) og_request_point(s.cnt, 1);
+    og_scan_columns(s);
 }
 
 // -------------------------------------------------------------- scatter --
@@ -699,8 +703,8 @@ __global__ void __launch_bounds__(OG_THREADS, 8) k_list(const og_dev_sys *__rest
 void og_launch_grid_clear(const og_launch &cols) {
     hipLaunchKernelGGL(k_grid_clear, dim3(cols.n_blocks), dim3(OG_THREADS), 0, cols.stream, cols.sys, cols.map);
 }
-void og_launch_grid_bin(const og_launch &a) {
-    hipLaunchKernelGGL(k_grid_bin, dim3(a.n_blocks), dim3(OG_THREADS), 0, a.stream, a.sys, a.map);
+void og_launch_grid_bin(const og_launch &a, bool point) {
+    hipLaunchKernelGGL(k_grid_bin, dim3(a.n_blocks), dim3(OG_THREADS), 0, a.stream, a.sys, a.map, (int)point);
 }
 void og_launch_grid_scatter(const og_launch &a) {
     hipLaunchKernelGGL(k_grid_scatter, dim3(a.n_blocks), dim3(OG_THREADS), 0, a.stream, a.sys, a.map);

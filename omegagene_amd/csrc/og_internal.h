@@ -311,6 +311,11 @@ __device__ __forceinline__ long long og_step_mod(long long n, int d) {
 __device__ __forceinline__ long long og_step_div(long long n, int d) {
     return (unsigned long long)n >> 32 ? n / d : (long long)((uint32_t)n / (uint32_t)d);
 }
+// The requests of a single-point call: energies whatever the step, and a grid rebuild.
+__device__ __forceinline__ void og_request_point(og_dev_counters *c, int rebuild) {
+    c->force_energy = 1;
+    if (rebuild) c->rebuild_now = 1;
+}
 // The grid-rebuild kernels run for a system when its own step is a multiple
 // of its rebuild interval (DynamicsMode.cpp:480-486) or a rebuild is forced;
 // systems at other phases in the same launch skip them.
@@ -535,7 +540,7 @@ struct og_launch {
 
 // grid build
 void og_launch_grid_clear(const og_launch &cols);
-void og_launch_grid_bin(const og_launch &atoms);
+void og_launch_grid_bin(const og_launch &atoms, bool point);  // point: for a single-point call
 void og_launch_grid_scatter(const og_launch &atoms);
 void og_launch_grid_sort(const og_launch &cols);
 void og_launch_cells_from_grid(const og_launch &cols);
@@ -561,7 +566,7 @@ struct alignas(16) og_point_out {
     og_dev_counters cnt;
     double          energy[OG_E_NTERMS];
 };
-void og_launch_point_begin(og_dev_counters *cnt, int rebuild, hipStream_t stream);
+void og_launch_point_begin(og_dev_counters *cnt, hipStream_t stream);  // without a rebuild
 void og_launch_point_end(const og_launch &atoms, og_point_out *out, double *work);  // takes the gradient too
 // integration
 void og_launch_leapfrog_vel(const og_launch &atoms);

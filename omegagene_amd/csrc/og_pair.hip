@@ -881,16 +881,14 @@ __global__ void __launch_bounds__(64) k_energy_reduce(const og_dev_sys *__restri
 }
 
 // A single-point evaluation of one system.  Its requests (energies, and a
-// grid rebuild) go into the counters before the first kernel; the last kernel
-// is k_forces_to_work with its outcome sent to pinned host memory: the
-// gradient when work is given, and from the last block the counters and the
-// energies.  One wait for the stream then delivers what took six copies with a
-// wait each (4,230 atoms: 208 us per call, then 116; 5 of them the reduction's
-// own launch, now this last block).
-__global__ void k_point_begin(og_dev_counters *c, int rebuild) {
-    c->force_energy = 1;
-    if (rebuild) c->rebuild_now = 1;
-}
+// grid rebuild) go into the counters in the rebuild's first kernel, or without
+// one in k_point_begin; the last kernel is k_forces_to_work with its outcome
+// sent to pinned host memory: the gradient when work is given, and from the
+// last block the counters and the energies.  One wait for the stream then
+// delivers what took six copies with a wait each (4,230 atoms: 208 us per
+// call, then 116; launches of their own for the requests and the reduction
+// were 7 and 5 us of it).
+__global__ void k_point_begin(og_dev_counters *c) { og_request_point(c, 0); }
 __global__ void __launch_bounds__(OG_THREADS) k_point_end(const og_dev_sys *__restrict__ S,
                                                           og_point_out *__restrict__ out,
                                                           double *__restrict__ work) {
@@ -970,8 +968,8 @@ void og_launch_forces_to_work(const og_launch &a) {
 void og_launch_energy_reduce(const og_launch &a) {
     hipLaunchKernelGGL(k_energy_reduce, dim3(a.n_blocks), dim3(64), 0, a.stream, a.sys, a.map);
 }
-void og_launch_point_begin(og_dev_counters *cnt, int rebuild, hipStream_t st) {
-    hipLaunchKernelGGL(k_point_begin, dim3(1), dim3(1), 0, st, cnt, rebuild);
+void og_launch_point_begin(og_dev_counters *cnt, hipStream_t st) {
+    hipLaunchKernelGGL(k_point_begin, dim3(1), dim3(1), 0, st, cnt);
 }
 void og_launch_point_end(const og_launch &a, og_point_out *out, double *work) {
     hipLaunchKernelGGL(k_point_end, dim3(a.n_blocks), dim3(OG_THREADS), 0, a.stream, a.sys, out, work);
