@@ -273,7 +273,8 @@ int og_alloc_atom_info(int max_n_atoms_exbox, int max_n_cells, int max_n_cell_pa
     CS_TRY(cs_alloc(&h.cp_count, (size_t)h.cap_cells + 1));
     CS_TRY(cs_alloc(&h.cp_stage, (size_t)h.cap_cells * OG_ENUM_STAGE));
     CS_TRY(cs_alloc(&h.cp_head, (size_t)h.cap_cells + 1));
-    CS_TRY(cs_alloc(&h.cp_bsum, (size_t)h.cap_cells / 1024 + 1));
+    CS_TRY(cs_alloc(&h.cp_bsum, 2 * ((size_t)h.cap_cells / 1024 + 1)));
+    h.cp_arrived = (int *)(h.cp_bsum + h.cap_cells / 1024 + 1);  // the second half
     CS_TRY(cs_alloc(&h.cp_c2, max_n_cell_pairs));
     CS_TRY(cs_alloc(&h.cp_mask, max_n_cell_pairs));
     CS_TRY(cs_alloc(&h.fx, OG_FX_WORDS(cap)));
@@ -596,8 +597,8 @@ int og_enumerate_cell_pairs(int **h_atomids, int n_cells, int n_neighbor_col, co
     CS_HIP(hipMemcpy(g_cs.d_cnt, &c, sizeof c, hipMemcpyHostToDevice));
     og_launch_grid_clear(cs_launch(g_cs.map_slot, g_cs.nb_slot));
     og_launch_cells_from_grid(cs_launch(g_cs.map_col, g_cs.nb_col));
-    og_launch_enum_count(cs_launch(g_cs.map_cellw, g_cs.nb_cellw));
-    og_launch_enum_scan(cs_launch(nullptr, g_cs.n_cells / 1024 + 1));
+    og_launch_enum_count(cs_launch(g_cs.map_cellw, g_cs.nb_cellw), cs_launch(nullptr, g_cs.n_cells / 1024 + 1),
+                         g_cs.n_cells);
     og_launch_list(cs_launch(g_cs.map_cellw, g_cs.nb_cellw));
     CS_HIP(hipGetLastError());
     CS_HIP(hipStreamSynchronize(g_cs.stream));

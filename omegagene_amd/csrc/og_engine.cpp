@@ -450,8 +450,7 @@ void enqueue_rebuild(og_exec &x, bool point = false) {
     og_launch_grid_bin(L(x, KIND_ATOM), point);
     og_launch_grid_scatter(L(x, KIND_ATOM));
     og_launch_grid_sort(L(x, KIND_COL));
-    og_launch_enum_count(L(x, KIND_CELLW));
-    og_launch_enum_scan(L(x, KIND_SCANB));
+    og_launch_enum_count(L(x, KIND_CELLW), L(x, KIND_SCANB), x.cells);
     og_launch_list(L(x, KIND_CELLW));
 }
 
@@ -839,9 +838,10 @@ og_status sys_alloc(og_system *s, const og_system_desc *d, const og_params *p) {
               A(&h.cell_zmin, h.cap_cells) && A(&h.cell_zmax, h.cap_cells) && A(&h.cell_u0, h.cap_cells) &&
               A(&h.cell_u1, h.cap_cells) && A(&h.u2c_min, (size_t)(h.n_columns + 2) * h.n_uni_z) &&
               A(&h.u2c_max, (size_t)(h.n_columns + 2) * h.n_uni_z) && A(&h.cp_count, h.cap_cells + 1) && A(&h.cp_stage, (size_t)h.cap_cells * OG_ENUM_STAGE) &&
-              A(&h.cp_head, h.cap_cells + 1) && A(&h.cp_bsum, h.cap_cells / 1024 + 1) && A(&h.cp_c2, h.cap_cell_pairs) && A(&h.cp_mask, h.cap_cell_pairs) &&
+              A(&h.cp_head, h.cap_cells + 1) && A(&h.cp_bsum, 2 * (h.cap_cells / 1024 + 1)) && A(&h.cp_c2, h.cap_cell_pairs) && A(&h.cp_mask, h.cap_cell_pairs) &&
               A(&h.fx, OG_FX_WORDS(cap)) && A(&h.e_acc, (size_t)OG_EACC_SLOTS * OG_EACC_STRIDE) && A(&h.sync, 1);
     if (!ok) return OG_E_DEVICE;
+    h.cp_arrived    = (int *)(h.cp_bsum + h.cap_cells / 1024 + 1);  // the second half
     const int n_tor     = h.n_torsions + h.n_impros;
     const int n_contrib = 3 * h.n_angles + 4 * n_tor + 2 * h.n_nb14;
     if (h.n_bterms) {
@@ -1362,7 +1362,7 @@ og_status og_system_footprint(const og_system_desc *d, const og_params *p, uint6
     b += (ng + 1) * 4 + ng_atoms * 4 + (ng + 1) * 4 + 3 * (ng + 1) * 8;
     b += cols * (4 * 6 + 8) + 2 * (cols + 2) * g.n_uni_z * 4;
     b += cap * (4 + 4 + 24 + 16 + 4 + 4 + 36);                            // tmp_ids, atomids, gcrd, gxyzq, gtype, gcomp, fx
-    b += cells * (6 * 4 + 4.0 * OG_ENUM_STAGE + 8) + (cells / 1024 + 1) * 8;
+    b += cells * (6 * 4 + 4.0 * OG_ENUM_STAGE + 8) + (cells / 1024 + 1) * 16;
     b += pairs * 12;
     b += 8.0 * OG_EACC_SLOTS * OG_EACC_STRIDE + ke_parts * 8 + OG_E_NTERMS * 8 + log_rows * OG_E_NTERMS * 8;
     b += std::min(n, (double)OG_FREE_MAX) * (vc > 0 ? 8 : 4) + sizeof(og_step_sync) + vc * 28 + vs * 32 + mcs * (4 + 8.0 * OG_MC_NPOLY + 32);

@@ -546,15 +546,62 @@ __device__ void og_enum_cell(const og_dev_sys &s, og_enum_lds &T, int c1, int p0
     if (MODE == 1 && lane == 0) *out_count = pos;
 }
 
+// One wave per cell.  SCAN: and the exclusive scan of the cells' pair counts
+// over groups of 1,024 cells, by the last of a group's blocks (k_enum_scan's
+// results).  Small launches save the scan's own launch that way (3 to 5 us and
+// a gap: 4,230 atoms 88 -> 85 us per single-point call, 25,041 143 -> 141);
+// in large ones the blocks' wait for their stores and one counter costs more
+// (99,200 atoms 418 -> 435, 450,000 atoms 70 us per rebuild).
+#define OG_SCAN_CELLS 1024
+template <bool SCAN>
 __global__ void __launch_bounds__(OG_THREADS) k_enum_count(const og_dev_sys *__restrict__ S,
                                                            const int2 *__restrict__ map) {
     __shared__ og_enum_lds lds[OG_THREADS / 64];
     const int2        bm = map[blockIdx.x];
     const og_dev_sys &s  = S[bm.x];
     if (og_rebuild_skip(s)) return;
-    const int         c1 = __builtin_amdgcn_readfirstlane(bm.y * (OG_THREADS / 64) + (threadIdx.x >> 6));
-    if (c1 >= s.cnt->n_cells) return;
-    og_enum_cell<1>(s, lds[threadIdx.x >> 6], c1, 0, &s.cp_count[c1]);
+    constexpr int PER = OG_THREADS / 64;  // cells per block
+    const int     c0  = bm.y * PER, n = s.cnt->n_cells;
+    const int     lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int     c1  = __builtin_amdgcn_readfirstlane(c0 + w);
+    if (c0 >= n) return;
+    if (c1 < n) {
+        int count = 0;
+        og_enum_cell<1>(s, lds[w], c1, 0, &count);
+        if (lane == 0) {
+            if (SCAN) __hip_atomic_store(&s.cp_count[c1], count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            else s.cp_count[c1] = count;
+        }
+    }
+    if (!SCAN) return;
+    static_assert(OG_SCAN_CELLS % PER == 0 && OG_SCAN_CELLS == 4 * OG_THREADS, "whole blocks, four cells per thread");
+    const int g = c0 / OG_SCAN_CELLS, g0 = g * OG_SCAN_CELLS, cells = min(OG_SCAN_CELLS, n - g0);
+    if (!og_last_block(&s.cp_arrived[g], (cells + PER - 1) / PER)) return;
+    int v[4], sum = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int c = 4 * threadIdx.x + j;
+        v[j] = c < cells ? __hip_atomic_load(&s.cp_count[g0 + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) sum += v[j];
+    __shared__ int wsum[PER];
+    int            incl = sum;
+    for (int off = 1; off < 64; off <<= 1) {
+        const int u = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += u;
+    }
+    if (lane == 63) wsum[w] = incl;
+    __syncthreads();
+    int at = incl - sum;
+    for (int q = 0; q < w; q++) at += wsum[q];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int c = 4 * threadIdx.x + j;
+        if (c < cells) s.cp_head[g0 + c] = at;
+        at += v[j];
+    }
+    if (threadIdx.x == OG_THREADS - 1) s.cp_bsum[g] = at;
 }
 
 // Exclusive scan of the cells' pair counts, blocks of 1024 cells: each cell's
@@ -624,7 +671,7 @@ __global__ void __launch_bounds__(OG_THREADS, 8) k_list(const og_dev_sys *__rest
     const int  id1 = s.atomids[c1 * OG_NAC + a1];
     const int  idl = s.atomids[c1 * OG_NAC + (lane & 7)];
     long long  at  = 0;  // the list position of the cell's first record
-    for (int q = lane; q < (c1 >> 10); q += 64) at += s.cp_bsum[q];
+    for (int q = lane; q < c1 / OG_SCAN_CELLS; q += 64) at += s.cp_bsum[q];
     for (int off = 32; off > 0; off >>= 1) at += __shfl_xor(at, off, 64);
     at += s.cp_head[c1];
     const long long end = at + cnt, cap = s.cap_cell_pairs;
@@ -715,11 +762,14 @@ void og_launch_grid_sort(const og_launch &a) {
 void og_launch_cells_from_grid(const og_launch &a) {
     hipLaunchKernelGGL(k_cells_from_grid, dim3(a.n_blocks), dim3(OG_THREADS), 0, a.stream, a.sys, a.map);
 }
-void og_launch_enum_count(const og_launch &a) {
-    hipLaunchKernelGGL(k_enum_count, dim3(a.n_blocks), dim3(OG_THREADS), 0, a.stream, a.sys, a.map);
-}
-void og_launch_enum_scan(const og_launch &a) {
-    hipLaunchKernelGGL(k_enum_scan, dim3(a.n_blocks), dim3(1024), 0, a.stream, a.sys, a.map);
+void og_launch_enum_count(const og_launch &cellw, const og_launch &blocks, long long cells) {
+    const dim3 nb(cellw.n_blocks), nt(OG_THREADS);
+    if (cells <= OG_SCAN_FUSED_CELLS) {
+        hipLaunchKernelGGL(k_enum_count<true>, nb, nt, 0, cellw.stream, cellw.sys, cellw.map);
+        return;
+    }
+    hipLaunchKernelGGL(k_enum_count<false>, nb, nt, 0, cellw.stream, cellw.sys, cellw.map);
+    hipLaunchKernelGGL(k_enum_scan, dim3(blocks.n_blocks), dim3(1024), 0, blocks.stream, blocks.sys, blocks.map);
 }
 void og_launch_list(const og_launch &a) {
     hipLaunchKernelGGL(k_list, dim3(a.n_blocks), dim3(OG_THREADS), 0, a.stream, a.sys, a.map);

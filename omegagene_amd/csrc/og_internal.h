@@ -235,7 +235,8 @@ struct og_dev_sys {
     int      *cp_count;     // [cap_cells]
     int      *cp_stage;     // [cap_cells * OG_ENUM_STAGE] pairs of each cell from the counting pass
     int      *cp_head;      // [cap_cells+1]
-    long long *cp_bsum;     // [cap_cells / 1024 + 1] block totals of the multi-block offset scan
+    long long *cp_bsum;     // [cap_cells / 1024 + 1] pair totals of the groups of 1,024 cells
+    int       *cp_arrived;  // [cap_cells / 1024 + 1] blocks of a group that have counted (zero between launches)
     int      *cp_c2;        // [cap_cell_pairs] cell2 | image << 24
     uint64_t *cp_mask;      // [cap_cell_pairs] bit a2*8+a1 set = skip
     // ---- forces / energies ----
@@ -544,8 +545,10 @@ void og_launch_grid_bin(const og_launch &atoms, bool point);  // point: for a si
 void og_launch_grid_scatter(const og_launch &atoms);
 void og_launch_grid_sort(const og_launch &cols);
 void og_launch_cells_from_grid(const og_launch &cols);
-void og_launch_enum_count(const og_launch &cellw);
-void og_launch_enum_scan(const og_launch &blocks);  // blocks of 1024 cells (cap_cells + 1); null map: one system
+// blocks: of 1,024 cells (cap_cells + 1; null map: one system); cells of the launch's systems: up to
+// OG_SCAN_FUSED_CELLS the counting scans as well (figures at k_enum_count)
+constexpr long long OG_SCAN_FUSED_CELLS = 4096;
+void og_launch_enum_count(const og_launch &cellw, const og_launch &blocks, long long cells);
 void og_launch_list(const og_launch &cellw);
 // forces
 // pair forms of og_launch_pair
