@@ -383,7 +383,9 @@ struct og_unit {
 };
 // Work unit u of a system with n cells: cells 0 .. n-m-1 whole, then the last
 // m cells as two units each (first and second half of their records).  run is
-// false past the last unit, for a frozen system and after a list overflow.
+// false past the last unit, for a frozen system and after a list overflow.  It
+// is the one field that two waves of a launch may read differently, as units
+// that run flag an overlap (OG_F_NAN) meanwhile.
 // The list head, the cell's atoms and the counters are read together (a unit
 // is a chain of memory round trips of about a microsecond each: block map,
 // system record, these, the records, their atoms); only a unit of the split
@@ -403,7 +405,7 @@ __device__ __forceinline__ og_unit og_unit_start(const og_dev_sys &s, const int 
     asm volatile("" ::"v"(t.p.x), "v"(t.ty), "s"(a), "s"(b));
     t.run    = !og_frozen_c(c) && !(c.flags & OG_F_CP_OVERFLOW) && u < n + m;
     t.energy = og_energy_step_c(s, c);
-    if (u >= n - m && t.run) {
+    if (u >= n - m && u < n + m) {  // whatever run is: which cell a unit is must not hang on the flags
         const int half = (u - (n - m)) & 1;
         t.c1 = n - m + ((u - (n - m)) >> 1);
         a    = s.cp_head[t.c1], b = s.cp_head[t.c1 + 1];
@@ -645,6 +647,7 @@ struct og_team {
     float coef[OG_TEAM][OG_NAC][64];               // by pass: gradient coefficients of the row's pairs
     float en[OG_TEAM][3][64];                      // by pass: the rows' LJ and electrostatic energy and virial
     int   cnt[2][OG_TEAM_G];                       // rows kept by each group of a batch, by batch parity
+    int   run;                                     // the block's unit runs
     og_f4 shift[64];
 };
 
@@ -843,8 +846,11 @@ __global__ void __launch_bounds__(64 * OG_TEAM) k_pair_team(const og_dev_sys *__
     const og_dev_sys &s  = S[bm.x];
     const og_unit     un = og_unit_start(s, bm.y);
     const int rows = og_pair_tables<FORM, 64 * OG_TEAM>(s, T.shift, ljl);
+    // One wave decides for the block: if another block flags an overlap between two waves' reads of the
+    // flags, waves that left would leave queue entries unwritten that the others go on to read.
+    if (threadIdx.x == 0) T.run = un.run;
     og_lds_barrier();
-    if (!un.run) return;  // block-uniform
+    if (!T.run) return;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (un.energy) {
         if (__all(un.ty < rows)) og_team_cell<FORM, true, true>(s, un, w, T, ljl);

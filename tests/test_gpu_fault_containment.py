@@ -1,0 +1,119 @@
+"""Overlapping atoms under the pair kernel of four waves per cell (launches of
+at most 900 cells): the blocks that meet the overlap flag the system while
+others of the launch still start, and a block's waves must go on or leave
+together.  The flagged system reports OG_E_NAN and stands still, its partner
+in the launch gives the bits it gives alone, and the system itself gives the
+bits of a new one once its coordinates are good again."""
+import numpy as np
+import pytest
+import torch
+
+from omegagene_amd import gen
+from omegagene_amd.celeste import ZeroDipole, pairwise_ljzd_noalloc
+from omegagene_amd.engine import OG_E_NAN, Batch, EngineError, System
+
+pytestmark = pytest.mark.gpu
+
+CFG = {"cutoff": 12.0, "nsgrid-cutoff": 13.0, "nsgrid-update-intvl": 5, "time-step": 1.0, "gap-bug": 0,
+       "integrator": "langevin", "constraint": "shake", "const-tolerance": 1e-10, "temperature": 300.0,
+       "langevin-gamma": 20.0, "random-seed": 5, "log-cap": 32}
+STEPS = 15
+
+
+def _overlapped(ls):
+    """Every 50th water's neighbour in the list moved onto it, 0.05 A apart."""
+    crd = ls.crd.copy()
+    for w in range(0, len(crd) // 3 - 1, 50):
+        crd[3 * w + 3] = crd[3 * w] + np.array([0.05, 0.0, 0.0])
+    return crd
+
+
+def _alone(ls):
+    s = System(ls, CFG)
+    w, e = s.energy_force(rebuild=True)
+    s.run(STEPS)
+    out = (w, s.state(), s.energy_log())
+    s.close()
+    return out
+
+
+def _equal(a, b):
+    return np.array_equal(a[0], b[0]) and all(np.array_equal(x, y) for x, y in zip(a[1], b[1])) and \
+        np.array_equal(a[2], b[2])
+
+
+def test_overlap_in_a_small_launch_is_contained():
+    good, bad = gen.build_system(700, seed=41), gen.build_system(500, seed=42)
+    assert good.n_atoms + bad.n_atoms <= 7200
+    print("[gpu-test] overlap in a batch of", good.n_atoms, bad.n_atoms, flush=True)
+    ref_good, ref_bad = _alone(good), _alone(bad)
+    sg, sb = System(good, CFG), System(bad, CFG)
+    wg = sg.energy_force(rebuild=True)[0]
+    sb.set_state(_overlapped(bad), bad.vel)
+    with pytest.raises(EngineError) as e:   # the single-point call
+        sb.energy_force(rebuild=True)
+    assert e.value.code == OG_E_NAN
+    b = Batch()
+    b.add(sg)
+    b.add(sb)
+    with pytest.raises(EngineError) as e:
+        b.run(STEPS)
+    assert e.value.code == OG_E_NAN
+    assert sg.status() == 0 and sb.status() == OG_E_NAN and sb.step() == 0 and sg.step() == STEPS
+    b.close()
+    assert _equal((wg, sg.state(), sg.energy_log()), ref_good)
+    sb.set_state(bad.crd, bad.vel)
+    wb = sb.energy_force(rebuild=True)[0]
+    sb.run(STEPS)
+    assert _equal((wb, sb.state(), sb.energy_log()), ref_bad)
+    sg.close()
+    sb.close()
+
+
+def test_overlap_in_the_allocation_free_call_is_flagged():
+    ls = gen.build_system(600, seed=43)
+    s = System(ls, CFG)
+    s.nsgrid_update()
+    ids, gcrd, _ = s.grid()
+    cps, head = s.cell_pairs()
+    s.close()
+    lj6, lj12 = ls.lj_tables_f32()
+    real = ids >= 0
+    xyzq, types = np.zeros((len(ids), 4), np.float32), np.zeros(len(ids), np.int32)
+    xyzq[:, :3] = gcrd
+    xyzq[real, 3] = ls.charge.astype(np.float32)[ids[real]]
+    types[real] = ls.atom_type[ids[real]]
+    mask = cps[:, 3].astype(np.uint32).astype(np.uint64) | (cps[:, 4].astype(np.uint32).astype(np.uint64) << 32)
+    dev = torch.device("cuda:0")
+    put = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)  # noqa: E731
+    d_types, d_lj = put(types), put(np.stack([lj6, lj12], -1).astype(np.float32))
+    d_head, d_mask = put(head.astype(np.int32)), put(mask.view(np.int64))
+    d_c2 = put((cps[:, 1].astype(np.int64) | (cps[:, 2].astype(np.int64) << 24)).astype(np.int32))
+    L = np.array([ls.box[0], ls.box[4], ls.box[8]], np.float32)
+    n_cells = len(ids) // 8
+    assert n_cells <= 900
+    print("[gpu-test] overlap in the allocation-free call,", n_cells, "cells", flush=True)
+    other = xyzq.copy()
+    o = np.nonzero(real)[0]
+    for k in range(0, len(o) - 8, 90):   # an atom and the next of another water in slot order
+        a = o[k]
+        b = next(j for j in o[k + 1:] if ids[j] // 3 != ids[a] // 3)
+        other[b, :3] = other[a, :3] + np.array([0.05, 0.0, 0.0], np.float32)
+
+    def call(x):
+        d_x = put(x)
+        work = torch.zeros((8 * n_cells, 3), dtype=torch.float64, device=dev)
+        energy = torch.zeros(2, dtype=torch.float64, device=dev)
+        flags = torch.zeros(1, dtype=torch.int32, device=dev)
+        pairwise_ljzd_noalloc(d_x.data_ptr(), d_types.data_ptr(), d_lj.data_ptr(), lj6.shape[0], d_head.data_ptr(),
+                              d_c2.data_ptr(), d_mask.data_ptr(), n_cells, L, 12.0, ZeroDipole(12.0),
+                              work.data_ptr(), energy.data_ptr(), flags.data_ptr(),
+                              torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        return work.cpu().numpy(), energy.cpu().numpy(), int(flags.cpu()[0])
+
+    w0, e0, f0 = call(xyzq)
+    assert f0 == 0 and np.isfinite(w0).all()
+    assert call(other)[2] != 0
+    w1, e1, f1 = call(xyzq)
+    assert f1 == 0 and np.array_equal(w0, w1) and np.array_equal(e0, e1)
