@@ -124,7 +124,8 @@ __global__ void __launch_bounds__(OG_THREADS) k_grid_bin(const og_dev_sys *__res
                                                          const int2 *__restrict__ map, const int point) {
     const int2        bm = map[blockIdx.x];
     const og_dev_sys &s  = S[bm.x];
-    if (point ? og_frozen(s) : og_rebuild_skip(s)) return;
+    // this kernel flags non-finite atoms; blocks that leave for it do not arrive (the host clears the count)
+    if (og_block_decides(point ? og_frozen(s) : og_rebuild_skip(s))) return;
     const int         i  = bm.y * OG_THREADS + threadIdx.x;
     const bool        in = i < s.n_atoms;
     og_clear_bins(s, i, s.n_atom_blocks * OG_THREADS);  // read by the last rebuild only, filled by the sort

@@ -312,6 +312,15 @@ __device__ __forceinline__ long long og_step_mod(long long n, int d) {
 __device__ __forceinline__ long long og_step_div(long long n, int d) {
     return (unsigned long long)n >> 32 ? n / d : (long long)((uint32_t)n / (uint32_t)d);
 }
+// The first wave's answer for the whole block.  Waves that read a system's
+// flags for themselves can read them differently where the launch itself
+// raises some, and a block with a barrier must not go on with a part of its waves.
+__device__ __forceinline__ bool og_block_decides(const bool mine) {
+    __shared__ int answer;
+    if (threadIdx.x == 0) answer = mine;
+    __syncthreads();
+    return answer != 0;
+}
 // The requests of a single-point call: energies whatever the step, and a grid rebuild.
 __device__ __forceinline__ void og_request_point(og_dev_counters *c, int rebuild) {
     c->force_energy = 1;

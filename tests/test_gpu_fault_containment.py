@@ -3,7 +3,10 @@ at most 900 cells): the blocks that meet the overlap flag the system while
 others of the launch still start, and a block's waves must go on or leave
 together.  The flagged system reports OG_E_NAN and stands still, its partner
 in the launch gives the bits it gives alone, and the system itself gives the
-bits of a new one once its coordinates are good again."""
+bits of a new one once its coordinates are good again.  The same for atoms
+that the binning of a grid rebuild finds out of any box: its blocks count
+their arrivals, and what a fault leaves of the counts must not reach the next
+rebuild."""
 import numpy as np
 import pytest
 import torch
@@ -117,3 +120,42 @@ def test_overlap_in_the_allocation_free_call_is_flagged():
     assert call(other)[2] != 0
     w1, e1, f1 = call(xyzq)
     assert f1 == 0 and np.array_equal(w0, w1) and np.array_equal(e0, e1)
+
+
+def test_fault_in_the_binning_leaves_nothing_behind():
+    """Atoms of several blocks thrown to 1e31 A by their velocity: the next
+    step's binning flags them, a single-point call meets them again, and with
+    good coordinates the system gives a new one's bits; its partner never
+    notices."""
+    cfg = dict(CFG, **{"integrator": "leapfrog-presto", "constraint": "none", "nsgrid-update-intvl": 1,
+                       "time-step": 0.5})
+    good, bad = gen.build_system(700, seed=44), gen.build_system(900, seed=45, n_beads=10)
+    refs = []
+    for ls in (good, bad):
+        s = System(ls, cfg)
+        w, _ = s.energy_force(rebuild=True)
+        s.run(STEPS)
+        refs.append((w, s.state()))
+        s.close()
+    sg, sb = System(good, cfg), System(bad, cfg)
+    vel = bad.vel.copy()
+    vel[7::300, 0] = 1e31
+    sb.set_state(bad.crd, vel)
+    print("[gpu-test] fault in the binning,", good.n_atoms, bad.n_atoms, "atoms", flush=True)
+    b = Batch()
+    b.add(sg)
+    b.add(sb)
+    with pytest.raises(EngineError) as e:
+        b.run(STEPS)
+    assert e.value.code == OG_E_NAN and sg.status() == 0 and sb.status() == OG_E_NAN and sb.step() == 1
+    b.close()
+    assert all(np.array_equal(x, y) for x, y in zip(sg.state(), refs[0][1]))
+    with pytest.raises(EngineError) as e:
+        sb.energy_force(rebuild=True)
+    assert e.value.code == OG_E_NAN
+    sb.set_state(bad.crd, bad.vel)
+    w, _ = sb.energy_force(rebuild=True)
+    sb.run(STEPS)
+    assert np.array_equal(w, refs[1][0]) and all(np.array_equal(x, y) for x, y in zip(sb.state(), refs[1][1]))
+    sg.close()
+    sb.close()
