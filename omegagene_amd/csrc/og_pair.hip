@@ -332,7 +332,8 @@ __device__ __forceinline__ og_jatom og_load_atom(const og_list &L, const unsigne
 }
 // Filter of one group: shifts the lanes' atoms to their pairs' periodic images
 // and returns the mask of the lanes to keep (within the cutoff of the cell1
-// box and not masked against all its atoms).
+// box and not masked against all its atoms).  A row without a number for its
+// distance is kept, so its pairs flag the evaluation.
 __device__ __forceinline__ uint64_t og_keep(const float (&lo)[3], const float (&hi)[3], const float rcb2,
                                             const og_f4 *__restrict__ shift, const unsigned cp, const unsigned m8,
                                             og_f4 &p) {
@@ -345,7 +346,7 @@ __device__ __forceinline__ uint64_t og_keep(const float (&lo)[3], const float (&
     const float gx = p.x - __builtin_amdgcn_fmed3f(p.x, lo[0], hi[0]);
     const float gy = p.y - __builtin_amdgcn_fmed3f(p.y, lo[1], hi[1]);
     const float gz = p.z - __builtin_amdgcn_fmed3f(p.z, lo[2], hi[2]);
-    return __builtin_amdgcn_ballot_w64(fmaf(gz, gz, fmaf(gx, gx, gy * gy)) < rcb2) &
+    return __builtin_amdgcn_ballot_w64(!(fmaf(gz, gz, fmaf(gx, gx, gy * gy)) >= rcb2)) &
            __builtin_amdgcn_ballot_w64(m8 != 0xffu);
 }
 // The cell1's atoms and box from the lanes' atoms p and types ty (lane & 7).
