@@ -194,8 +194,8 @@ typedef struct {
     double   capacity_factor;      /* cell-pair list capacity multiplier (1.0 default) */
     double   enhance_sigma;        /* --enhance-sigma (VcMD, A) */
     double   enhance_recov_coef;   /* --enhance-recovery-coef (VcMD) */
-    int      split_step;           /* 1: run a Langevin step as separate kernels even where the fused
-                                      one-kernel step applies (same trajectory; for comparison) */
+    int      split_step;           /* 1: run a step as separate kernels even where the fused one-kernel
+                                      step applies (same trajectory; for comparison) */
     int      thermostat;           /* --thermostat: OG_THERMOSTAT_NONE or OG_THERMOSTAT_SCALING (leapfrog-presto,
                                       no constraints: ThermostatScaling::apply_thermostat, Thermostat.cpp:57-84) */
     double   berendsen_tau;        /* --berendsen-tau already in fs (Config.cpp:162-164); the step replaces it
@@ -391,8 +391,10 @@ og_status   og_set_pair_shape_order(og_system *sys, int waves, int order);
 og_status   og_autotune_cell_edge(const og_system_desc *desc, const og_params *params, int trials,
                                   double *best_scale, double *pair_ms);
 og_status   og_batch_set_pair_shape(og_batch *b, int waves, int order);
-/* 1 when an MD step of this system runs as the fused one-kernel Langevin step
- * (Langevin, SETTLE waters bound to nothing outside the water, at most 4096 other atoms) */
+/* 1 when an MD step of this system by itself runs as the fused one-kernel step: Langevin, or leapfrog
+ * without thermostat and COM removal; waters (SETTLE, or without any the SHAKE trios that qualify) bound to
+ * nothing outside the water; no four-atom SHAKE group and no V-McMD; at most 4096 other atoms.  A batch takes
+ * it when every member does in the same form. */
 og_status   og_step_fused(og_system *sys, int *fused);
 /* device memory a created system holds (bytes) */
 og_status   og_system_device_bytes(og_system *sys, uint64_t *bytes);

@@ -301,13 +301,18 @@ og_status exec_release(og_exec &x) {
     return OG_OK;
 }
 
-// (re)build the descriptor array and block maps of an execution context
+// Whether a system by itself takes the fused step, and its form (a context does when all members do in one form).
+bool fused_step(const og_dev_sys &h) {
+    // V-McMD scales the whole gradient by the step's potential energy
+    return h.n_water_blocks > 0 && h.mc_mode != OG_MC_VMCMD;
+}
 int fused_form(const og_dev_sys &h) {
     const bool shake = h.n_settle == 0;  // the waters are SHAKE trios
     return h.integrator == 1 ? (shake ? OG_FUSED_LANGEVIN_SHAKE : OG_FUSED_LANGEVIN_SETTLE)
                              : (shake ? OG_FUSED_LEAPFROG_SHAKE : OG_FUSED_LEAPFROG_SETTLE);
 }
 
+// (re)build the descriptor array and block maps of an execution context
 og_status exec_prepare(og_exec &x) {
     if (!x.dirty) return OG_OK;
     free_graphs(x);
@@ -345,13 +350,12 @@ og_status exec_prepare(og_exec &x) {
         x.any_constraint |= d.constraint != 0;
         x.any_vcmd |= d.vc_n_states > 0 || d.mc_mode == OG_MC_VAUS;
         x.any_vmcmd |= d.mc_mode == OG_MC_VMCMD;
-        x.fused &= d.mc_mode != OG_MC_VMCMD;  // V-McMD scales the whole gradient by the step's potential energy
         x.any_thermo |= d.thermostat == OG_THERMOSTAT_SCALING;
         x.any_bonded |= d.n_bterms > 0;
         x.any_quad |= d.constraint != 0 && d.n_quads > 0;
         const int form = fused_form(d);
         if (si == 0) x.fused_form = form;
-        x.fused &= d.n_water_blocks > 0 && form == x.fused_form;
+        x.fused &= fused_step(d) && form == x.fused_form;
         x.cells += cdiv(d.n_atoms, OG_NAC);
         int       cnt[KIND_N];
         cnt[KIND_ATOM]  = cdiv(d.n_atoms, OG_THREADS);
@@ -1877,7 +1881,7 @@ og_status og_system_device_bytes(og_system *s, uint64_t *bytes) {
 
 og_status og_step_fused(og_system *s, int *fused) {
     if (!s || !fused) return OG_E_ARG;
-    *fused = s->h.n_water_blocks > 0 && fused_form(s->h) == OG_FUSED_LANGEVIN_SETTLE;
+    *fused = fused_step(s->h);
     return OG_OK;
 }
 

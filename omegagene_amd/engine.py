@@ -470,7 +470,7 @@ class System:
         return b.value
 
     def step_fused(self):
-        """True when an MD step runs as the fused one-kernel Langevin step."""
+        """True when an MD step of this system by itself runs as the fused one-kernel step, in any of its forms."""
         f = C.c_int()
         _check(lib().og_step_fused(self.h, C.byref(f)))
         return bool(f.value)
