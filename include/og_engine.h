@@ -393,8 +393,9 @@ og_status   og_autotune_cell_edge(const og_system_desc *desc, const og_params *p
 og_status   og_batch_set_pair_shape(og_batch *b, int waves, int order);
 /* 1 when an MD step of this system by itself runs as the fused one-kernel step: Langevin, or leapfrog
  * without thermostat and COM removal; waters (SETTLE, or without any the SHAKE trios that qualify) bound to
- * nothing outside the water; no four-atom SHAKE group and no V-McMD; at most 4096 other atoms.  A batch takes
- * it when every member does in the same form. */
+ * nothing outside the water; no four-atom SHAKE group and no V-McMD; at most 512 + waters / 100 other atoms,
+ * and at most 4096.  A batch takes it when every member qualifies in the same form, with the waters of all
+ * members in that bound. */
 og_status   og_step_fused(og_system *sys, int *fused);
 /* device memory a created system holds (bytes) */
 og_status   og_system_device_bytes(og_system *sys, uint64_t *bytes);

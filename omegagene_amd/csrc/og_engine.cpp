@@ -301,7 +301,8 @@ og_status exec_release(og_exec &x) {
     return OG_OK;
 }
 
-// Whether a system by itself takes the fused step, and its form (a context does when all members do in one form).
+// Whether a system can take the fused step, and its form.  A context takes it when all members can in one
+// form and none has more free atoms than og_free_limit allows.
 bool fused_step(const og_dev_sys &h) {
     // V-McMD scales the whole gradient by the step's potential energy
     return h.n_water_blocks > 0 && h.mc_mode != OG_MC_VMCMD;
@@ -331,6 +332,8 @@ og_status exec_prepare(og_exec &x) {
     x.any_bonded = x.any_quad = x.any_vmcmd = false;
     x.fused        = true;
     x.cells        = 0;
+    int       free_most = 0;  // the members' largest
+    long long waters    = 0;
     x.intvl        = x.members[0]->prm.nsgrid_update_intvl;
     for (int si = 0; si < ns; si++) {
         og_system *s = x.members[si];
@@ -357,6 +360,8 @@ og_status exec_prepare(og_exec &x) {
         if (si == 0) x.fused_form = form;
         x.fused &= fused_step(d) && form == x.fused_form;
         x.cells += cdiv(d.n_atoms, OG_NAC);
+        free_most = std::max(free_most, d.n_free);
+        waters += d.n_waters;
         int       cnt[KIND_N];
         cnt[KIND_ATOM]  = cdiv(d.n_atoms, OG_THREADS);
         cnt[KIND_CELLW] = cdiv(d.cap_cells, OG_THREADS / 64);
@@ -376,6 +381,7 @@ og_status exec_prepare(og_exec &x) {
             for (int b = 0; b < nb; b++) maps[KIND_PAIR + lw].push_back(make_int2(si, b));
         }
     }
+    x.fused &= free_most <= og_free_limit(waters);
     // pair kernel, blocks round-robin across the systems of a batch
     for (int lw = 0; lw < 4; lw++) {
         int most = 0;
@@ -1020,7 +1026,7 @@ og_status sys_alloc(og_system *s, const og_system_desc *d, const og_params *p) {
     // The fused step (one kernel per MD step after the pair kernel) takes
     // waters three lanes each, so each water must interact with no other atom
     // through exclusions and carry no bond, VcMD group or other constraint;
-    // the other atoms (at most OG_FREE_MAX) go through one block.  Its waters
+    // the other atoms (at most OG_FREE_MAX, and see og_free_limit) are moved by one block.  Its waters
     // are the SETTLE waters (all of them, or the step is not fused) or, with
     // none, the SHAKE trios that qualify, which are moved to the end of the
     // trio list (the trios are independent of each other).
@@ -1881,7 +1887,7 @@ og_status og_system_device_bytes(og_system *s, uint64_t *bytes) {
 
 og_status og_step_fused(og_system *s, int *fused) {
     if (!s || !fused) return OG_E_ARG;
-    *fused = fused_step(s->h);
+    *fused = fused_step(s->h) && s->h.n_free <= og_free_limit(s->h.n_waters);
     return OG_OK;
 }
 

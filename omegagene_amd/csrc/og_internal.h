@@ -290,7 +290,30 @@ __host__ __device__ __forceinline__ int og_pair_split_cells(int split, int n_cel
 #define OG_WATERS_PER_WAVE 21  // fused step: three lanes per water
 #define OG_WATERS_PER_BLOCK (OG_WATERS_PER_WAVE * (OG_WATER_THREADS / 64))
 #define OG_FREE_PER_BLOCK (OG_WATER_THREADS / 8)  // fused step: eight lanes per free atom
-#define OG_FREE_MAX 4096      // fused step: most atoms outside SETTLE waters (one block takes them)
+#define OG_FREE_MAX 4096      // fused step: most atoms outside the waters of a system that qualifies
+// Of the contexts whose systems all qualify, those take the fused step in
+// which no system has more free atoms than og_free_limit (waters: of all its
+// systems).  One block moves a system's free atoms, 256 at a time, and each
+// round adds 4 to 6 us to the launch; the separate kernels cost 10 us of
+// launches and another pass over the waters.  us per step, fused / separate
+// (pair kernel and rebuilds included):
+//   leapfrog, SHAKE waters; free atoms with bonds | with bonds and SHAKE trios
+//     free atoms      768                1,050              2,040              4,095
+//      13,000 atoms   51/55   54/55      57/57   63/56      67/56   78/56      92/57  114/56
+//      50,000        105/113 110/112    110/113 118/112    120/113 133/113    147/113 172/112
+//     150,000        223/236 225/230    224/233 233/231    234/232 248/230    259/232 285/235
+//     450,000        580/601 579/600    575/598 575/598    581/602 596/600    610/598 633/599
+//   Langevin, SETTLE waters
+//      13,000         54/55   58/58      62/54   69/58      75/55   86/58     108/55  131/58
+//      50,000        108/111 112/114    116/111 123/113    127/110 140/114    161/110 185/114
+//     450,000        569/587 567/590    568/588 572/593    575/590 586/593    605/593 627/590
+//     16 x 6,000     182/190 183/189    193/182 197/183    219/187 232/200    290/194 333/191
+// At 6,000 atoms the lines cross between 600 and 900 free atoms, at 450 and
+// fewer the fused step is ahead everywhere (42/46 to 46/46).
+__host__ __forceinline__ int og_free_limit(const long long waters) {
+    const long long most = 512 + waters / 100;
+    return (int)(most < OG_FREE_MAX ? most : OG_FREE_MAX);
+}
 #define OG_CP_BLOCKS_PER_SYS_MIN 64
 
 // ---- small device helpers ----
