@@ -1066,17 +1066,13 @@ og_status sys_alloc(og_system *s, const og_system_desc *d, const og_params *p) {
         drop_all(d->impro_ids, 4LL * h.n_impros);
         drop_all(d->nb14_ids, 2LL * h.n_nb14);
         const int nw = (int)std::count(good.begin(), good.end(), 1);
-        std::vector<int> group(n, 0);  // the atom's bias group
-        bool             once = true;
-        for (int k = 0; k < h.vc_na + h.vc_nb; k++) {
-            int &g = group[k < h.vc_na ? d->vc_atoms_a[k] : d->vc_atoms_b[k - h.vc_na]];
-            once &= g == 0;  // the separate kernels take an atom listed twice
-            g = k < h.vc_na ? 1 : 2;
-        }
+        std::vector<int> group(n, 0);  // the atom's bias group (creation refuses groups that share an atom)
+        for (int k = 0; k < h.vc_na; k++) group[d->vc_atoms_a[k]] = 1;
+        for (int k = 0; k < h.vc_nb; k++) group[d->vc_atoms_b[k]] = 2;
         std::vector<int> free_ids;
         for (int i = 0; i < n; i++)
             if (water[i] < 0 || !good[water[i]]) free_ids.push_back(i);
-        if (nw > 0 && once && (nw == nt || !settle) && (int)free_ids.size() <= OG_FREE_MAX) {
+        if (nw > 0 && (nw == nt || !settle) && (int)free_ids.size() <= OG_FREE_MAX) {
             if (!A(&h.free_ids, std::max<size_t>(free_ids.size(), 1))) return OG_E_DEVICE;
             if (!free_ids.empty())
                 OG_HIP(hipMemcpy(h.free_ids, free_ids.data(), sizeof(int) * free_ids.size(), hipMemcpyHostToDevice));
