@@ -598,7 +598,7 @@ int og_enumerate_cell_pairs(int **h_atomids, int n_cells, int n_neighbor_col, co
     og_launch_grid_clear(cs_launch(g_cs.map_slot, g_cs.nb_slot));
     og_launch_cells_from_grid(cs_launch(g_cs.map_col, g_cs.nb_col));
     og_launch_enum_count(cs_launch(g_cs.map_cellw, g_cs.nb_cellw), cs_launch(nullptr, g_cs.n_cells / 1024 + 1),
-                         g_cs.n_cells);
+                         og_scan_with_count(true, g_cs.n_cells, g_cs.n_cells));
     og_launch_list(cs_launch(g_cs.map_cellw, g_cs.nb_cellw));
     CS_HIP(hipGetLastError());
     CS_HIP(hipStreamSynchronize(g_cs.stream));

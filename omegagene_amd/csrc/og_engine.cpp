@@ -275,7 +275,7 @@ struct og_exec {
     bool                     fused = false;       // every member takes the fused step, in one form
     int                      fused_form = 0;
     int                      pair_shape = OG_PAIR_DEFAULT;  // pair-kernel launch shape (KIND_PAIR + pair_shape)
-    long long                cells = 0;           // cells of all members, at most a few per cent short
+    long long                cells = 0, cells_most = 0;  // cells of all members and of the largest, at most a few per cent short
     int                      intvl = 1;
     int                      graph_steps = 0;     // steps per captured graph (0: automatic)
 };
@@ -331,7 +331,7 @@ og_status exec_prepare(og_exec &x) {
     x.any_langevin = x.any_leapfrog = x.any_com = x.any_constraint = x.any_vcmd = x.any_thermo = false;
     x.any_bonded = x.any_quad = x.any_vmcmd = false;
     x.fused        = true;
-    x.cells        = 0;
+    x.cells = x.cells_most = 0;
     int       free_most = 0;  // the members' largest
     long long waters    = 0;
     x.intvl        = x.members[0]->prm.nsgrid_update_intvl;
@@ -360,6 +360,7 @@ og_status exec_prepare(og_exec &x) {
         if (si == 0) x.fused_form = form;
         x.fused &= fused_step(d) && form == x.fused_form;
         x.cells += cdiv(d.n_atoms, OG_NAC);
+        x.cells_most = std::max<long long>(x.cells_most, cdiv(d.n_atoms, OG_NAC));
         free_most = std::max(free_most, d.n_free);
         waters += d.n_waters;
         int       cnt[KIND_N];
@@ -460,7 +461,7 @@ void enqueue_rebuild(og_exec &x, bool point = false) {
     og_launch_grid_bin(L(x, KIND_ATOM), point);
     og_launch_grid_scatter(L(x, KIND_ATOM));
     og_launch_grid_sort(L(x, KIND_COL));
-    og_launch_enum_count(L(x, KIND_CELLW), L(x, KIND_SCANB), x.cells);
+    og_launch_enum_count(L(x, KIND_CELLW), L(x, KIND_SCANB), og_scan_with_count(point, x.cells, x.cells_most));
     og_launch_list(L(x, KIND_CELLW));
 }
 

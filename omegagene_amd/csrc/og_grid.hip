@@ -549,10 +549,9 @@ __device__ void og_enum_cell(const og_dev_sys &s, og_enum_lds &T, int c1, int p0
 
 // One wave per cell.  SCAN: and the exclusive scan of the cells' pair counts
 // over groups of 1,024 cells, by the last of a group's blocks (k_enum_scan's
-// results).  Small launches save the scan's own launch that way (3 to 5 us and
-// a gap: 4,230 atoms 88 -> 85 us per single-point call, 25,041 143 -> 141);
-// in large ones the blocks' wait for their stores and one counter costs more
-// (99,200 atoms 418 -> 435, 450,000 atoms 70 us per rebuild).
+// results).  That saves the scan's own launch; against it stand the blocks'
+// wait for their stores and one counter per group (og_scan_with_count has both
+// sides; 450,000 atoms 70 us per rebuild).
 #define OG_SCAN_CELLS 1024
 template <bool SCAN>
 __global__ void __launch_bounds__(OG_THREADS) k_enum_count(const og_dev_sys *__restrict__ S,
@@ -763,9 +762,9 @@ void og_launch_grid_sort(const og_launch &a) {
 void og_launch_cells_from_grid(const og_launch &a) {
     hipLaunchKernelGGL(k_cells_from_grid, dim3(a.n_blocks), dim3(OG_THREADS), 0, a.stream, a.sys, a.map);
 }
-void og_launch_enum_count(const og_launch &cellw, const og_launch &blocks, long long cells) {
+void og_launch_enum_count(const og_launch &cellw, const og_launch &blocks, bool scan) {
     const dim3 nb(cellw.n_blocks), nt(OG_THREADS);
-    if (cells <= OG_SCAN_FUSED_CELLS) {
+    if (scan) {
         hipLaunchKernelGGL(k_enum_count<true>, nb, nt, 0, cellw.stream, cellw.sys, cellw.map);
         return;
     }
