@@ -61,6 +61,17 @@ class GroupCoordDef:
     crd: List[np.ndarray]                    # per group float64[n_atoms_in_group, 3]
 
 
+def box12(box) -> np.ndarray:
+    """The 12 box values that the engine reads (3 x 3 matrix, centre); of a matrix alone, the centre is at half
+    the edges."""
+    b = np.ascontiguousarray(box, np.float64).ravel()
+    if len(b) == 9:
+        b = np.concatenate([b, 0.5 * b[[0, 4, 8]]])
+    if len(b) < 12:
+        raise ValueError("a box has 12 values (3 x 3 matrix, centre) or 9, not %d" % len(b))
+    return b
+
+
 @dataclass
 class LaunchSet:
     box: np.ndarray                      # float64[12] = {Lx,0,0, 0,Ly,0, 0,0,Lz, cx,cy,cz}

@@ -12,7 +12,7 @@ from typing import Optional
 
 import numpy as np
 
-from .cls import LaunchSet
+from .cls import LaunchSet, box12
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libog_engine.so")
@@ -197,7 +197,7 @@ def desc_from_launchset(ls: LaunchSet, constraint: int = 1, com_groups=None, vcm
     n = ls.n_atoms
     x = Desc()
     x.n_atoms = n
-    x.box = d(ls.box)
+    x.box = d(box12(ls.box))  # the engine reads 12 values
     x.crd = d(ls.crd)
     x.vel = d(ls.vel)
     x.charge = d(ls.charge)

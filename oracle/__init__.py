@@ -123,9 +123,19 @@ def _p(a, ct):
     return a.ctypes.data_as(C.POINTER(ct))
 
 
+def _box12(box):
+    """The 12 values that the C side reads: of a 3 x 3 matrix alone, the centre is at half the edges."""
+    b = np.ascontiguousarray(box, np.float64).ravel()
+    if len(b) == 9:
+        b = np.concatenate([b, 0.5 * b[[0, 4, 8]]])
+    if len(b) < 12:
+        raise ValueError("a box has 12 values (3 x 3 matrix, centre) or 9, not %d" % len(b))
+    return b
+
+
 def grid_setup(n_atoms, box, nscut) -> Grid:
     g = Grid()
-    rc = lib().orc_grid_setup(C.byref(g), C.c_int(n_atoms), _p(np.ascontiguousarray(box, np.float64), C.c_double),
+    rc = lib().orc_grid_setup(C.byref(g), C.c_int(n_atoms), _p(_box12(box), C.c_double),
                               C.c_double(nscut))
     if rc != 0:
         raise ValueError("orc_grid_setup failed (%d): box too small for the list radius" % rc)
@@ -289,7 +299,7 @@ def pbc_from_box(box):
     L = (C.c_float * 3)()
     lb = (C.c_float * 3)()
     ub = (C.c_float * 3)()
-    lib().orc_pbc_from_box(_p(np.ascontiguousarray(box, np.float64), C.c_double), L, lb, ub)
+    lib().orc_pbc_from_box(_p(_box12(box), C.c_double), L, lb, ub)
     return np.array(L[:], np.float32), np.array(lb[:], np.float32), np.array(ub[:], np.float32)
 
 
