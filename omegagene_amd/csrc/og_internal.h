@@ -578,16 +578,17 @@ void og_launch_grid_scatter(const og_launch &atoms);
 void og_launch_grid_sort(const og_launch &cols);
 void og_launch_cells_from_grid(const og_launch &cols);
 // Whether the counting kernel scans as well (k_enum_count<true>) instead of a launch after it: in a call that the
-// host waits for (one system), where a launch more costs 2 to 3 us, up to 2,048 cells; in an MD step, where it costs
-// 1 us, as long as no system has more cells than one group of the scan.  cells, most: of the launch's systems
+// host waits for (one system), where a launch more costs 2 to 6 us by host, up to 4,096 cells; in an MD step, where it
+// costs 1 us, as long as no system has more cells than one group of the scan.  cells, most: of the launch's systems
 // together and of the largest.  us with a launch of its own / scanned by the counting kernel (steps rebuild each time):
-//   atoms                    2,400      4,200      8,000      12,000      16,000       20,000       25,000       99,000
-//   single-point call      79.2/75.0  80.8/78.1  93.9/91.1  101.0/98.6  109.2/109.9  121.4/120.5  147.4/147.1  427/437
-//   step with a rebuild    67.5/66.4  67.6/67.1  77.3/77.4   80.7/81.9   85.1/87.9    92.0/95.7   101.9/106.5  250/263
+//   atoms                    4,200      8,000      12,000     16,000       20,000       25,000     32,000   50,000   99,000
+//   single-point call      80.8/78.1  93.9/91.1  101.0/98.6  109.2/109.9  121.4/120.5  147.4/147.1  172/171  254/259  427/437
+//     on a slower host     84.6/77.9  97.9/91.1  103.0/98.7  115.8/110.4  128.6/121.5  154.0/147.8
+//   step with a rebuild    67.6/67.1  77.3/77.4   80.7/81.9   85.1/87.9    92.0/95.7   101.9/106.5  115/122  152/160  250/263
 //   batch (step)  8 x 3,000 111.8/110.6   48 x 3,000 348.4/349.1   8 x 6,000 153.2/152.2   4 x 8,000 116.6/116.3
 //                 8 x 8,000 176.7/177.7   16 x 8,000 280.5/282.4   4 x 12,000 151.1/151.8  8 x 12,000 224.5/228.0
 __host__ __forceinline__ bool og_scan_with_count(const bool call, const long long cells, const long long most) {
-    return call ? cells <= 2048 : most <= 1024 && cells <= 8192;
+    return call ? cells <= 4096 : most <= 1024 && cells <= 8192;
 }
 // blocks: of 1,024 cells (cap_cells + 1; null map: one system)
 void og_launch_enum_count(const og_launch &cellw, const og_launch &blocks, bool scan);

@@ -1,5 +1,5 @@
 """The offset scan of the cell-pair list by the counting kernel (single-point
-calls up to 2,048 cells, MD steps and grid updates while no system has more
+calls up to 4,096 cells, MD steps and grid updates while no system has more
 than 1,024) against the scan launched after it: around both lines the list
 that a single-point call leaves equals the one of a grid update, entry for
 entry, and a batch's list is that of its members alone."""
@@ -22,7 +22,7 @@ def _list(s):
     return ids, gcrd, cp, head
 
 
-@pytest.mark.parametrize("waters", [2720, 2731, 2780, 5450, 5462, 5500])   # 1,020 to 2,063 cells before padding
+@pytest.mark.parametrize("waters", [2720, 2731, 2780, 5462, 10922, 10930])   # 1,020 to 4,099 cells before padding
 def test_list_of_a_call_equals_the_list_of_an_update(waters):
     s = System(gen.build_system(waters, seed=waters), CFG)
     lists = []
