@@ -75,6 +75,8 @@ __device__ __forceinline__ void og_scan_columns(const og_dev_sys &s) {
     auto count = [&](int k) {
         return __hip_atomic_load(&s.n_atoms_col[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     };
+    // read with the counts; flagged by the binning (or before it): there is no grid to lay out
+    const int flags = __hip_atomic_load(&s.cnt->flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     int local = 0, mx = 0;
 #pragma unroll 4
     for (int k = k0; k < k1; k++) {
@@ -82,6 +84,7 @@ __device__ __forceinline__ void og_scan_columns(const og_dev_sys &s) {
         local += (n + OG_NAC - 1) / OG_NAC;
         mx = max(mx, n);
     }
+    if (flags & OG_F_FATAL) return;
     int incl = local;
     for (int off = 1; off < 64; off <<= 1) {
         const int v = __shfl_up(incl, off, 64);
@@ -124,11 +127,13 @@ __global__ void __launch_bounds__(OG_THREADS) k_grid_bin(const og_dev_sys *__res
                                                          const int2 *__restrict__ map, const int point) {
     const int2        bm = map[blockIdx.x];
     const og_dev_sys &s  = S[bm.x];
-    // this kernel flags non-finite atoms; blocks that leave for it do not arrive (the host clears the count)
-    if (og_block_decides(point ? og_frozen(s) : og_rebuild_skip(s))) return;
+    // A launch raises flags itself (non-finite atoms), which the waves of a block may read differently: a wave that
+    // finds one does no work, but every block arrives, and the scan reads the flags when all are raised.
+    if (s.cnt->step >= s.cnt->step_end || !(point || og_rebuild_due(s))) return;
+    const bool        run = (s.cnt->flags & OG_F_FATAL) == 0;
     const int         i  = bm.y * OG_THREADS + threadIdx.x;
-    const bool        in = i < s.n_atoms;
-    og_clear_bins(s, i, s.n_atom_blocks * OG_THREADS);  // read by the last rebuild only, filled by the sort
+    const bool        in = run && i < s.n_atoms;
+    if (run) og_clear_bins(s, i, s.n_atom_blocks * OG_THREADS);  // read by the last rebuild only, filled by the sort
     int  c[2] = {0, 0};
     bool bad = false;
     if (in) {

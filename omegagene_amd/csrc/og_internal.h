@@ -335,15 +335,6 @@ __device__ __forceinline__ long long og_step_mod(long long n, int d) {
 __device__ __forceinline__ long long og_step_div(long long n, int d) {
     return (unsigned long long)n >> 32 ? n / d : (long long)((uint32_t)n / (uint32_t)d);
 }
-// The first wave's answer for the whole block.  Waves that read a system's
-// flags for themselves can read them differently where the launch itself
-// raises some, and a block with a barrier must not go on with a part of its waves.
-__device__ __forceinline__ bool og_block_decides(const bool mine) {
-    __shared__ int answer;
-    if (threadIdx.x == 0) answer = mine;
-    __syncthreads();
-    return answer != 0;
-}
 // The requests of a single-point call: energies whatever the step, and a grid rebuild.
 __device__ __forceinline__ void og_request_point(og_dev_counters *c, int rebuild) {
     c->force_energy = 1;
@@ -352,9 +343,10 @@ __device__ __forceinline__ void og_request_point(og_dev_counters *c, int rebuild
 // The grid-rebuild kernels run for a system when its own step is a multiple
 // of its rebuild interval (DynamicsMode.cpp:480-486) or a rebuild is forced;
 // systems at other phases in the same launch skip them.
-__device__ __forceinline__ bool og_rebuild_skip(const og_dev_sys &s) {
-    return og_frozen(s) || (s.rebuild_intvl > 0 && og_step_mod(s.cnt->step, s.rebuild_intvl) != 0 && !s.cnt->rebuild_now);
+__device__ __forceinline__ bool og_rebuild_due(const og_dev_sys &s) {
+    return s.rebuild_intvl <= 0 || og_step_mod(s.cnt->step, s.rebuild_intvl) == 0 || s.cnt->rebuild_now;
 }
+__device__ __forceinline__ bool og_rebuild_skip(const og_dev_sys &s) { return og_frozen(s) || !og_rebuild_due(s); }
 // Energies (pair, virial) are evaluated on logged steps and on request; the
 // forces and the pair count on every step.
 __device__ __forceinline__ bool og_energy_step_c(const og_dev_sys &s, const og_dev_counters &c) {

@@ -851,7 +851,7 @@ __global__ void __launch_bounds__(64 * OG_TEAM) k_pair_team(const og_dev_sys *__
     // flags, waves that left would leave queue entries unwritten that the others go on to read.
     if (threadIdx.x == 0) T.run = un.run;
     og_lds_barrier();
-    if (!T.run) return;
+    if (!__builtin_amdgcn_readfirstlane(T.run)) return;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (un.energy) {
         if (__all(un.ty < rows)) og_team_cell<FORM, true, true>(s, un, w, T, ljl);
