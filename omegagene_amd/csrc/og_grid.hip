@@ -166,7 +166,7 @@ __global__ void __launch_bounds__(OG_THREADS) k_grid_bin(const og_dev_sys *__res
         s.zkey[i]        = og_float_key(bad ? 0.0f : (float)z);
     }
     og_wave_count_add(s.n_atoms_col, c[0] + c[1] * s.nx, in);
-    if (!og_last_block(&s.sync->all, s.n_atom_blocks)) return;
+    if (!og_last_block_of(s.sync, bm.y, s.n_atom_blocks)) return;
     if (point && threadIdx.x == 0) og_request_point(s.cnt, 1);
     og_scan_columns(s);
 }
